@@ -13,9 +13,10 @@
 //     works through hundreds of substeps.
 //
 // Layout: rho is species-major [ns][n] (coalesced per species), E and dt [n].
-// The mechanism lives in constant memory.  Arithmetic keeps the reference's
-// operation order (-ffp-contract=off); exp/log/log10/pow are the device
-// library's, so results agree with the CPU restatement to a few ulps per call.
+// The mechanism lives in constant memory, the arithmetic in ocfd_chem_core.h.
+// Sums keep the reference's order; the exponentials are the core's own and the
+// logarithms the device library's, so results agree with the CPU restatement
+// to a few ulps per call.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -29,36 +30,11 @@
 #include "ocfd_mlp.h"
 #include "ocfd_mlp_tile.h"
 
-#define CH_NS 9
-#define CH_NR_MAX 32
-#define CH_NT_MAX 4
-#define CH_R0 8.314
-#define CH_ATM 1.013e5
+#include "ocfd_chem_core.h"
 
-struct ChemMech {
-  int ns, nr, n_tct;
-  int rereac;                      // 0 Gibbs Kc, 1 Arrhenius reverse rates, 2 Park fit of Kc
-  double rev[CH_NR_MAX][5];        // ReReac 1: A_r, b_r, E_r; ReReac 2: A1r..A5r
-  int af_type[CH_NR_MAX], tb[CH_NR_MAX], sgm[CH_NR_MAX];
-  double fc[CH_NR_MAX], arr[CH_NR_MAX][2][3], eff[CH_NR_MAX][CH_NS];
-  int vf[CH_NR_MAX][CH_NS], vr[CH_NR_MAX][CH_NS];
-  double tct[CH_NT_MAX], tct_max;
-  double mi[CH_NS], ri[CH_NS], coef[CH_NS][CH_NT_MAX][7], ect[CH_NS][CH_NT_MAX];
-};
-
-__constant__ ChemMech cm;
-
-// The mechanism as seen by the device functions: a pointer into the constant
-// bank (address space 4, so loads through it are scalar loads).  The kernels
-// pass it through an empty asm statement at the top of every substep; the
-// compiler then cannot hoist the hundreds of constant loads of the rate and
-// thermo code out of the substep loop into registers, which otherwise
-// exhausts the register file and spills.
-typedef const __attribute__((address_space(4))) ChemMech* Mech;
-__device__ __forceinline__ Mech mech_opaque(Mech m) {
-  asm volatile("" : "+s"(m));
-  return m;
-}
+// threads per workgroup of the one-cell-per-lane kernels: one wavefront, so
+// that no wavefront waits for another's LDS to be freed
+constexpr int CH_BLOCK = 64;
 
 // Integration state of a cell handed from the per-lane queue to the
 // cooperative kernel (struct of arrays, capacity cap records).
@@ -72,6 +48,7 @@ struct HeavyBuf {
 namespace {
 struct ChemCtx {
   bool ready = false;
+  bool h2 = false;         // the mechanism has the structure of ChemH2
   bool rev_ready = false;  // reverse-rate data present (always for ReReac = 0)
   ChemMech h{};
   hipStream_t stream = nullptr, own = nullptr;
@@ -109,376 +86,12 @@ int cfail(const std::string& m) {
 }
 }  // namespace
 
-__device__ __forceinline__ double q2(double x) { return x * x; }
-__device__ __forceinline__ double q3(double x) { double x2 = x * x; return x2 * x; }
-__device__ __forceinline__ double q4(double x) { double x2 = x * x; return x2 * x2; }
-__device__ __forceinline__ double q5(double x) { double x2 = x * x; return (x2 * x2) * x; }
-// Fortran x**n for an integer n (repeated squaring; negative n -> 1/x**|n|)
-__device__ __forceinline__ double ipow(double x, int n) {
-  if (n == 0) return 1.0;
-  int m = n < 0 ? -n : n;
-  double r = 1.0, b = x;
-  bool first = true;
-  while (m) {
-    if (m & 1) { r = first ? b : r * b; first = false; }
-    m >>= 1;
-    if (m) b = b * b;
-  }
-  return n < 0 ? 1.0 / r : r;
-}
-
-__device__ __forceinline__ int trange(Mech m, double T) {
-  int jc = 0;
-  for (int j = 0; j < m->n_tct - 1; j++)
-    if (T > m->tct[j]) jc = j + 1;
-  return jc;
-}
-
-// comput_T_rgas, CHEM_thermdyn.f90:326-382 (Newton, 1e-3 K, <= 31 iterations)
-__device__ double chem_T(Mech m, const double* di, double E) {
-  double A1[CH_NT_MAX], B1[CH_NT_MAX], C1[CH_NT_MAX], D1[CH_NT_MAX], E1[CH_NT_MAX], Ect[CH_NT_MAX];
-#pragma unroll
-  for (int j = 0; j < CH_NT_MAX; j++) {
-    A1[j] = B1[j] = C1[j] = D1[j] = E1[j] = Ect[j] = 0.0;
-    if (j < m->n_tct) {
-#pragma unroll
-      for (int k = 0; k < CH_NS; k++) {
-        const double R1 = m->ri[k];
-        A1[j] = A1[j] + (m->coef[k][j][0] - 1.0) * R1 * di[k];
-        B1[j] = B1[j] + m->coef[k][j][1] * R1 * di[k];
-        C1[j] = C1[j] + m->coef[k][j][2] * R1 * di[k];
-        D1[j] = D1[j] + m->coef[k][j][3] * R1 * di[k];
-        E1[j] = E1[j] + m->coef[k][j][4] * R1 * di[k];
-        Ect[j] = Ect[j] + m->ect[k][j] * R1 * di[k];
-      }
-    }
-  }
-  double T1 = E / A1[0], T2 = T1;
-  for (int ks = 0; ks <= 30; ks++) {
-    const int jc = trange(m, T1);
-    double a = A1[0], b = B1[0], c = C1[0], d = D1[0], e = E1[0], ect = Ect[0];
-#pragma unroll
-    for (int j = 1; j < CH_NT_MAX; j++)
-      if (jc == j) { a = A1[j]; b = B1[j]; c = C1[j]; d = D1[j]; e = E1[j]; ect = Ect[j]; }
-    double Et1, Ex;
-    if (T1 <= m->tct_max) {
-      Et1 = a * T1 + b * q2(T1) / 2.0 + c * q3(T1) / 3.0 + d * q4(T1) / 4.0 + e * q5(T1) / 5.0 + ect;
-      Ex = a + b * T1 + c * q2(T1) + d * q3(T1) + e * q4(T1);
-    } else {
-      const double tm = m->tct_max;
-      Ex = a + b * tm + c * q2(tm) + d * q3(tm) + e * q4(tm);
-      Et1 = a * tm + b * q2(tm) / 2.0 + c * q3(tm) / 3.0 + d * q4(tm) / 4.0 + e * q5(tm) / 5.0 + ect + Ex * (T1 - tm);
-    }
-    T2 = T1 - (Et1 - E) / Ex;
-    const double error = fabs(T2 - T1);
-    T1 = T2;
-    if (error < 1.0e-3) break;
-  }
-  return T2;
-}
-
-// comput_gibbs, CHEM_thermdyn.f90:296-319
-__device__ __forceinline__ double chem_gibbs(Mech m, int k, double T, double logT) {
-  const int jc = trange(m, T);
-  const auto c = m->coef[k][jc];  // pointer into the constant bank
-  if (T <= m->tct_max)
-    return c[0] * (1.0 - logT) * T - c[1] * q2(T) / 2.0 - c[2] * q3(T) / 6.0 - c[3] * q4(T) / 12.0 - c[4] * q5(T) / 20.0 +
-           c[5] - c[6] * T;
-  const double tm = m->tct_max;
-  const double Cp_max = c[0] + c[1] * tm + c[2] * q2(tm) + c[3] * q3(tm) + c[4] * q4(tm);
-  const double h_max = c[0] * tm + c[1] * q2(tm) / 2.0 + c[2] * q3(tm) / 3.0 + c[3] * q4(tm) / 4.0 + c[4] * q5(tm) / 5.0 + c[5];
-  const double S_max = c[0] * log(tm) + c[1] * tm + c[2] * q2(tm) / 2.0 + c[3] * q3(tm) / 3.0 + c[4] * q4(tm) / 4.0 + c[6];
-  return h_max + Cp_max * (T - tm) - T * (S_max + Cp_max * log(T / tm));
-}
-
-// Reaction_rate_coef (CHEM_reactions.f90:130-197) + Reaction_rate_and_Matrix
-// (:230-272).  ri in mol/cm3/s; A[i][j] = d ri / d cj if JAC.
-// Constants of one reaction (read_Reac, CHEM_reactions.f90:15-71).
-struct RxnConst {
-  int af_type, tb, sgm, rereac;
-  double fc, a0, b0, e0, a1, b1, e1;
-  double r[5];                     // reverse-rate data (ReReac 1 or 2)
-  double eff[CH_NS];
-  int vf[CH_NS], vr[CH_NS];
-};
-
-__device__ __forceinline__ RxnConst load_rxn(Mech m, int k) {
-  RxnConst R;
-  R.af_type = m->af_type[k];
-  R.tb = m->tb[k];
-  R.sgm = m->sgm[k];
-  R.fc = m->fc[k];
-  R.a0 = m->arr[k][0][0];
-  R.b0 = m->arr[k][0][1];
-  R.e0 = m->arr[k][0][2];
-  R.a1 = m->arr[k][1][0];
-  R.b1 = m->arr[k][1][1];
-  R.e1 = m->arr[k][1][2];
-  R.rereac = m->rereac;
-#pragma unroll
-  for (int a = 0; a < 5; a++) R.r[a] = m->rev[k][a];
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    R.eff[i] = m->eff[k][i];
-    R.vf[i] = m->vf[k][i];
-    R.vr[i] = m->vr[k][i];
-  }
-  return R;
-}
-
-// Rate of one reaction with concentrations: Reaction_rate_coef
-// (CHEM_reactions.f90:130-197) and the mass-action products of
-// Reaction_rate_and_Matrix (:246-250).  gi = G_i/R_i of every species.
-__device__ __forceinline__ void chem_reaction_c(const RxnConst& R, double T, const double* gi, const double* ci,
-                                                double& wf1, double& wr1) {
-  const double Rs = CH_R0 / CH_ATM * 1.0e6;
-  // comput_KjX (CHEM_reactions.f90:76-103), used by ReReac = 0 only
-  double kjx = 0.0;
-  if (R.rereac == 0) {
-    double dgi = 0.0;
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) dgi = dgi + gi[i] * (R.vr[i] - R.vf[i]);
-    kjx = exp(-dgi / T) * ipow(Rs * T, -R.sgm);
-  }
-  double Ctrb = 0.0;
-  if (R.tb == 1) {
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) Ctrb = Ctrb + ci[i] * R.eff[i];
-  }
-  const double wf1a = R.a0 * pow(T, R.b0) * exp(-R.e0 / T);
-  double wf, wr;
-  if (R.af_type == 0) {
-    wf = wf1a;
-  } else if (R.af_type == 2) {
-    const double wf2 = R.a1 * pow(T, R.b1) * exp(-R.e1 / T);
-    wf = wf1a + wf2;
-  } else {
-    const double wf2 = R.a1 * pow(T, R.b1) * exp(-R.e1 / T);
-    const double Prs = wf1a / wf2 * Ctrb;
-    const double Fc = R.fc;
-    const double lfc = log10(Fc);
-    const double ac = -0.4 - (double)0.67f * lfc;   // REAL(4) literals of the reference
-    const double an = 0.75 - (double)1.27f * lfc;
-    const double lp = log10(Prs);
-    const double F = pow(10.0, lfc / (1.0 + q2((lp + ac) / (an - 0.14 * (lp + ac)))));
-    wf = wf2 * Prs / (1.0 + Prs) * F;
-  }
-  if (R.rereac == 0) {
-    wr = wf / kjx;
-  } else if (R.rereac == 1) {
-    wr = R.r[0] * pow(T, R.r[1]) * exp(-R.r[2] / T);      // Arrhenius reverse rate (:180-181)
-  } else {
-    // ParkCurveFit (:113-118) with the 1e-30 floor (:182-186)
-    const double z = 10000.0 / T;
-    double kp = exp(R.r[0] + R.r[1] * z + R.r[2] * q2(z) + R.r[3] * q3(z) + R.r[4] * q4(z));
-    if (kp < 1.0e-30) kp = 1.0e-30;
-    wr = wf / kp;
-  }
-  if (R.tb == 1 && R.af_type != 1) {
-    wf = wf * Ctrb;
-    wr = wr * Ctrb;
-  }
-  wf1 = wf;
-  wr1 = wr;
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    if (R.vf[i] != 0) wf1 = wf1 * ipow(ci[i], R.vf[i]);
-    if (R.vr[i] != 0) wr1 = wr1 * ipow(ci[i], R.vr[i]);
-  }
-}
-
-__device__ __forceinline__ void chem_reaction(Mech m, int k, double T, const double* gi, const double* ci, double& wf1,
-                                              double& wr1) {
-  chem_reaction_c(load_rxn(m, k), T, gi, ci, wf1, wr1);
-}
-
-// d(ri)/d(cj) contribution of reaction k (CHEM_reactions.f90:262-268)
-__device__ __forceinline__ double chem_dA(Mech m, int k, int j, double wf1, double wr1, const double* ci) {
-  const double Awf = m->vf[k][j] * wf1 / (ci[j] + 1.0e-20);
-  const double Awr = m->vr[k][j] * wr1 / (ci[j] + 1.0e-20);
-  return Awf - Awr;
-}
-
-// Reaction_rate_coef (CHEM_reactions.f90:130-197) + Reaction_rate_and_Matrix
-// (:230-272).  ri in mol/cm3/s; A[i][j] = d ri / d cj if JAC.  k is uniform
-// across the wavefront, so the stoichiometry tests are scalar branches and
-// the fully unrolled i/j loops keep ri and A in registers.
-template <bool JAC>
-__device__ void chem_rates(Mech m, const double* ci, double T, double* ri, double (*A)[CH_NS]) {
-  double gi[CH_NS];
-  if (m->rereac == 0) {
-    const double logT = log(T);
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) gi[i] = chem_gibbs(m, i, T, logT);
-  }
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    ri[i] = 0.0;
-    if (JAC) {
-#pragma unroll
-      for (int j = 0; j < CH_NS; j++) A[i][j] = 0.0;
-    }
-  }
-  for (int k = 0; k < m->nr; k++) {
-    double wf1, wr1;
-    chem_reaction(m, k, T, gi, ci, wf1, wr1);
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) {
-      const int nu = m->vr[k][i] - m->vf[k][i];
-      if (nu != 0) ri[i] = ri[i] + (wf1 - wr1) * nu;
-    }
-    if (JAC) {
-#pragma unroll
-      for (int j = 0; j < CH_NS; j++) {
-        if (m->vf[k][j] == 0 && m->vr[k][j] == 0) continue;
-        const double dA = chem_dA(m, k, j, wf1, wr1, ci);
-#pragma unroll
-        for (int i = 0; i < CH_NS; i++) {
-          const int nu = m->vr[k][i] - m->vf[k][i];
-          if (nu != 0) A[i][j] = A[i][j] + dA * nu;
-        }
-      }
-    }
-  }
-}
-
-// Gauss elimination with partial pivoting (CHEM_reactions.f90:523-567),
-// fully unrolled so the 9x9 system stays in registers; row swaps are selects.
-__device__ void chem_gauss(double (*a)[CH_NS], double* b, double* x) {
-#pragma unroll
-  for (int k = 0; k < CH_NS - 1; k++) {
-    double fmax = fabs(a[k][k]);
-    int kk = k;
-#pragma unroll
-    for (int i = k + 1; i < CH_NS; i++)
-      if (fabs(a[i][k]) > fmax) { fmax = fabs(a[i][k]); kk = i; }
-#pragma unroll
-    for (int i = k + 1; i < CH_NS; i++) {
-      const bool sw = (i == kk);
-#pragma unroll
-      for (int j = k; j < CH_NS; j++) {
-        const double t = a[k][j];
-        a[k][j] = sw ? a[i][j] : a[k][j];
-        a[i][j] = sw ? t : a[i][j];
-      }
-      const double t = b[k];
-      b[k] = sw ? b[i] : b[k];
-      b[i] = sw ? t : b[i];
-    }
-#pragma unroll
-    for (int i = k + 1; i < CH_NS; i++) {
-      const double f = -a[i][k] / a[k][k];
-#pragma unroll
-      for (int j = 0; j < CH_NS; j++) a[i][j] = a[i][j] + f * a[k][j];
-      b[i] = b[i] + f * b[k];
-    }
-  }
-  x[CH_NS - 1] = b[CH_NS - 1] / a[CH_NS - 1][CH_NS - 1];
-#pragma unroll
-  for (int i = CH_NS - 2; i >= 0; i--) {
-    double xi = b[i];
-#pragma unroll
-    for (int j = i + 1; j < CH_NS; j++) xi = xi - a[i][j] * x[j];
-    x[i] = xi / a[i][i];
-  }
-}
-
-// update_Et, CHEM_thermdyn.f90:184-196
-__device__ __forceinline__ void chem_update_et(Mech m, const double* di, const double* dinew, double& E) {
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) E = E - (dinew[i] - di[i]) * m->ri[i] * m->coef[i][0][5];
-}
-
-// The linear system of chemical_Euler_implicit (CHEM_reactions.f90:491-505)
-// with step h, solved in place: Ar becomes I - Ar (M_i/M_j) h and is
-// eliminated; dd = the increment of the partial densities.
-__device__ __forceinline__ void chem_implicit_solve(Mech m, const double* ri, double (*Ar)[CH_NS], double h, double* dd) {
-  double rhs[CH_NS];
-#pragma unroll
-  for (int j = 0; j < CH_NS; j++)
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) Ar[i][j] = (i == j ? 1.0 : 0.0) - Ar[i][j] * m->mi[i] / m->mi[j] * h;
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) rhs[i] = ri[i] * m->mi[i] * 1.0e6 * h;
-  chem_gauss(Ar, rhs, dd);
-}
-
-__device__ __forceinline__ void chem_apply(Mech m, double* di, double& E, const double* dd) {
-  double dinew[CH_NS];
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) dinew[i] = di[i] + dd[i];
-  chem_update_et(m, di, dinew, E);
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) di[i] = dinew[i];
-}
-
-// chemical_Euler_implicit, CHEM_reactions.f90:473-516
-__device__ void chem_step_implicit(Mech m, double* di, double& E, double dt) {
-  double ci[CH_NS], ri[CH_NS], Ar[CH_NS][CH_NS];
-  const double T = chem_T(m, di, E);
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) ci[i] = di[i] / m->mi[i] * 1.0e-6;
-  chem_rates<true>(m, ci, T, ri, Ar);
-  double dd[CH_NS];
-  chem_implicit_solve(m, ri, Ar, dt, dd);
-  chem_apply(m, di, E, dd);
-}
-
-__device__ void chem_explicit_rates(Mech m, const double* di_c, double T, double* ri) {
-  double ci[CH_NS];
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) ci[i] = di_c[i] / m->mi[i] * 1.0e-6;
-  chem_rates<false>(m, ci, T, ri, nullptr);
-}
-
-// chemical_Euler (:395-425), chemical_RK2 (:429-469), chemical_RK3 (:572-602)
-template <int MODE>
-__device__ void chem_step(Mech m, double* di, double& E, double dt) {
-  if (MODE == -1) {
-    chem_step_implicit(m, di, E, dt);
-  } else if (MODE == 1) {
-    double ri[CH_NS], dinew[CH_NS];
-    const double T = chem_T(m, di, E);
-    chem_explicit_rates(m, di, T, ri);
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) dinew[i] = di[i] + ri[i] * m->mi[i] * 1.0e6 * dt;
-    chem_update_et(m, di, dinew, E);
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) di[i] = dinew[i];
-  } else if (MODE == 2) {
-    double ri[CH_NS], di1[CH_NS], dinew[CH_NS];
-    double T = chem_T(m, di, E);
-    chem_explicit_rates(m, di, T, ri);
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) di1[i] = di[i] + ri[i] * m->mi[i] * 1.0e6 * dt;
-    chem_update_et(m, di, di1, E);
-    T = chem_T(m, di, E);  // the reference evaluates T from the old di here
-    chem_explicit_rates(m, di1, T, ri);
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) dinew[i] = 0.5 * di[i] + 0.5 * di1[i] + 0.5 * ri[i] * m->mi[i] * 1.0e6 * dt;
-    chem_update_et(m, di1, dinew, E);
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) di[i] = dinew[i];
-  } else {
-    const double Ra[3] = {0.0, 3.0 / 4.0, 1.0 / 3.0}, Rb[3] = {1.0, 1.0 / 4.0, 2.0 / 3.0};
-    double din[CH_NS], ri[CH_NS], dinew[CH_NS];
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) din[i] = di[i];
-    for (int krk = 0; krk < 3; krk++) {
-      const double T = chem_T(m, di, E);
-      chem_explicit_rates(m, di, T, ri);
-#pragma unroll
-      for (int i = 0; i < CH_NS; i++) dinew[i] = Ra[krk] * din[i] + Rb[krk] * (di[i] + ri[i] * m->mi[i] * 1.0e6 * dt);
-      chem_update_et(m, di, dinew, E);
-#pragma unroll
-      for (int i = 0; i < CH_NS; i++) di[i] = dinew[i];
-    }
-  }
-}
-
-template <int MODE>
-__global__ __launch_bounds__(128) void k_chem_fixed(long n, double* rho, double* Ecell, const double* dtcell, int nsub) {
+template <int MODE, class ST>
+__global__ __launch_bounds__(CH_BLOCK, MODE == 1 ? 3 : 2) void k_chem_fixed(long n, double* rho, double* Ecell,
+                                                                         const double* dtcell, int nsub) {
+  __shared__ LaneLds<CH_BLOCK, MODE == -1> L;
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  lane_lds_init(L);
   if (c >= n) return;
   double di[CH_NS];
 #pragma unroll
@@ -488,72 +101,11 @@ __global__ __launch_bounds__(128) void k_chem_fixed(long n, double* rho, double*
   Mech m = (Mech)&cm;
   for (int s = 0; s < nsub; s++) {
     m = mech_opaque(m);
-    chem_step<MODE>(m, di, E, h);
+    chem_step<MODE, ST>(m, L, di, E, h);
   }
 #pragma unroll
   for (int i = 0; i < CH_NS; i++) rho[(long)i * n + c] = di[i];
   Ecell[c] = E;
-}
-
-// Adaptive point-implicit substepping (no reference counterpart).  One
-// attempt: T, rates and Jacobian at the current state (negative partial
-// densities enter the rates as zero: the reference's regularised Jacobian
-// d(ri)/d(cj) ~ 1/(cj + 1e-20) makes cj = -1e-20 mol/cm3 a fixed point of the
-// point-implicit update of a consumed species, where it divides by zero);
-// proposed step
-//   h = min(dt - t, h_cap, min_k s_k/|w_k|, s_T/|q|)
-// with s_k = rtol_y (max(rho_k,0) + y_floor rho), s_T = rtol_t T rcv,
-// rcv = sum_k 2.5 R_k rho_k, w_k = ri_k M_k 1e6 and q = sum_k w_k R_k F_k;
-// the linear solve gives dd, accepted when |dd_k| <= 2 s_k for all k and
-// |sum_k dd_k R_k F_k| <= 2 s_T.  Accepted: the update is applied and
-// h_cap = 2h.  Rejected: the state is unchanged and h_cap = h/2.  Returns
-// whether the attempt was accepted; h_taken is the step on acceptance.
-struct ChemCtl {
-  double rtol_y, y_floor, rtol_t;
-  int max_sub;
-};
-
-__device__ __forceinline__ bool chem_adaptive_attempt(Mech m, double* di, double& E, double dt, double t, double& h_cap,
-                                                      const ChemCtl& ctl, double& h_taken) {
-  double ci[CH_NS], ri[CH_NS], Ar[CH_NS][CH_NS], sk[CH_NS], dd[CH_NS];
-  const double T = chem_T(m, di, E);
-  double rho = 0.0;
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    ci[i] = (di[i] > 0.0 ? di[i] : 0.0) / m->mi[i] * 1.0e-6;
-    rho = rho + di[i];
-  }
-  chem_rates<true>(m, ci, T, ri, Ar);
-  double h = dt - t;
-  if (h_cap < h) h = h_cap;
-  double q = 0.0, rcv = 0.0;
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    const double w = ri[i] * m->mi[i] * 1.0e6;
-    sk[i] = ctl.rtol_y * ((di[i] > 0.0 ? di[i] : 0.0) + ctl.y_floor * rho);
-    if (fabs(w) * h > sk[i]) h = sk[i] / fabs(w);
-    q = q + w * m->ri[i] * m->coef[i][0][5];
-    rcv = rcv + 2.5 * m->ri[i] * di[i];
-  }
-  const double sT = ctl.rtol_t * T * rcv;
-  if (fabs(q) * h > sT) h = sT / fabs(q);
-  chem_implicit_solve(m, ri, Ar, h, dd);
-  bool ok = true;
-  double de = 0.0;
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    ok = ok && fabs(dd[i]) <= 2.0 * sk[i];
-    de = de + dd[i] * m->ri[i] * m->coef[i][0][5];
-  }
-  ok = ok && fabs(de) <= 2.0 * sT;
-  if (!ok) {
-    h_cap = 0.5 * h;
-    return false;
-  }
-  chem_apply(m, di, E, dd);
-  h_cap = 2.0 * h;
-  h_taken = h;
-  return true;
 }
 
 // queue[0]: next cell of the work queue; queue[1]: cells left unfinished
@@ -567,9 +119,12 @@ __device__ __forceinline__ void chem_finish(long c, long n, double* rho, double*
   if (!finished) atomicAdd(queue + 1, 1ull);
 }
 
-__global__ __launch_bounds__(128) void k_chem_adaptive(long n, double* rho, double* Ecell, const double* dtcell,
+template <class ST>
+__global__ __launch_bounds__(CH_BLOCK, 2) void k_chem_adaptive(long n, double* rho, double* Ecell, const double* dtcell,
                                                         ChemCtl ctl, int* nsub_out, unsigned long long* queue) {
+  __shared__ LaneLds<CH_BLOCK, true> L;
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  lane_lds_init(L);
   if (c >= n) return;
   double di[CH_NS];
 #pragma unroll
@@ -581,7 +136,7 @@ __global__ __launch_bounds__(128) void k_chem_adaptive(long n, double* rho, doub
   Mech m = (Mech)&cm;
   while (t < dt && nsub < ctl.max_sub && nrej < ctl.max_sub) {
     m = mech_opaque(m);
-    if (!chem_adaptive_attempt(m, di, E, dt, t, h_cap, ctl, h)) {
+    if (!chem_adaptive_attempt<ST>(m, L, di, E, dt, t, h_cap, ctl, h)) {
       nrej++;
       continue;
     }
@@ -592,45 +147,99 @@ __global__ __launch_bounds__(128) void k_chem_adaptive(long n, double* rho, doub
   chem_finish(c, n, rho, Ecell, di, E, nsub, t >= dt || dt - t <= 1e-12 * dt, nsub_out, queue);
 }
 
-// Persistent kernel with a lane-level work queue.  A lane whose cell is done
-// takes the next one; the wavefront asks the queue once for all its idle
-// lanes (one atomic per refill).  Each pass runs one attempt per busy lane,
-// with the same per-cell loop as k_chem_adaptive.  A cell ends after at most
-// 2 max_sub attempts, and a lane leaves once the queue is empty and its cell
-// is done, so every wave reaches the exit.
-// With a list, the queue runs over the cells list[0 .. *list_count) instead
+// The rest of one cell's integration on a whole wavefront; every lane holds
+// the state.  Ends after at most 2 max_sub attempts.
+template <class ST>
+__device__ __forceinline__ void coop_cell(Mech m, CoopLds& L, const double2* tab, int lane, long c, long n, double* rho,
+                                          double* Ecell, double* di, double E, double dt, double t, double h_cap,
+                                          int nsub, int nrej, const ChemCtl& ctl, int* nsub_out,
+                                          unsigned long long* queue) {
+  // readfirstlane states that the loop decisions are uniform, which keeps
+  // the control flow scalar
+  while (__builtin_amdgcn_readfirstlane((t < dt && nsub < ctl.max_sub && nrej < ctl.max_sub) ? 1 : 0)) {
+    m = mech_opaque(m);
+    double h = 0.0;
+    if (!coop_attempt<ST>(m, L, tab, lane, di, E, dt, t, h_cap, ctl, h)) {
+      nrej++;
+      continue;
+    }
+    t = t + h;
+    nsub++;
+    if (__builtin_amdgcn_readfirstlane((dt - t <= 1e-12 * dt) ? 1 : 0)) break;
+  }
+  if (lane == 0) chem_finish(c, n, rho, Ecell, di, E, nsub, t >= dt || dt - t <= 1e-12 * dt, nsub_out, queue);
+  __builtin_amdgcn_wave_barrier();  // the wavefront goes on together
+}
+
+// Persistent kernel with a lane-level work queue, one wavefront a workgroup.
+// Each pass runs one attempt per busy lane, with the same per-cell loop as
+// k_chem_adaptive.  With a list, the cells are list[0 .. *list_count) instead
 // of 0 .. n (n stays the array stride).
-// With budget > 0, a cell still running after `budget` attempts is handed
-// to the cooperative kernel (k_chem_coop) with its full controller state, so
-// the few cells that need hundreds of substeps do not hold a lane for the
-// whole kernel.  A list of at most direct_max cells (the surrogate's
-// rejects: few, and mostly stiff) hands every cell over after its first
-// attempt: each then has a wavefront to itself.
-__global__ __launch_bounds__(128) void k_chem_queue(long n, double* rho, double* Ecell, const double* dtcell,
+//   - First cells: all resident wavefronts are launched and share the
+//     cells, so that a batch of fewer cells than lanes spreads over them.
+//     With a list (longest first), lane l of wavefront w takes entry w + l W:
+//     every wavefront gets one cell of each stratum instead of 64 of the
+//     longest; without one, consecutive cells (their loads coalesce).
+//   - Refill: a lane whose cell is done takes the next one; the wavefront
+//     asks the queue once for all its idle lanes.
+//   - Tail: once the queue is empty and at most COOP_TAIL lanes of the
+//     wavefront still run, their cells go on one after the other with the
+//     whole wavefront each (coop_attempt: 7 us an attempt against 14 us for
+//     any number of lanes, so two cells break even).
+//   - budget > 0: a cell still running after `budget` attempts is handed to
+//     k_chem_coop with its full controller state.  A list of at most
+//     direct_max cells (the surrogate's rejects: few, and mostly stiff) hands
+//     every cell over after its first attempt.
+// A cell ends after at most 2 max_sub attempts, and a lane leaves once the
+// queue is empty and its cell is done, so every wave reaches the exit.
+constexpr int COOP_TAIL = 2;
+template <class ST>
+__global__ __launch_bounds__(CH_BLOCK, 2) void k_chem_queue(long n, double* rho, double* Ecell, const double* dtcell,
                                                      ChemCtl ctl, int* nsub_out, unsigned long long* queue,
                                                      const int* list, const unsigned long long* list_count, int budget,
                                                      int direct_max, HeavyBuf hb) {
+  // the lanes' columns, and in the tail the one-cell tables, whose space
+  // they share
+  __shared__ union Lds {
+    LaneLds<CH_BLOCK, true> lane;
+    struct {
+      CoopLds L;
+      double2 tab[CH_EXPN];
+    } coop;
+    __device__ Lds() {}
+  } U;
+  LaneLds<CH_BLOCK, true>& L = U.lane;
+  lane_lds_init(L);
   const unsigned long long count =
       list ? (*list_count < (unsigned long long)n ? *list_count : (unsigned long long)n) : (unsigned long long)n;
   if (list && budget > 0 && count <= (unsigned long long)direct_max) budget = 1;
   const int lane = threadIdx.x & 63;
   const unsigned long long lt = (1ull << lane) - 1ull;
+  const unsigned long long W = gridDim.x, per = (count + W - 1) / W;
+  const unsigned long long quota = per < 64ull ? per : 64ull;  // first cells of a wavefront
   long cell = -1;  // -1: needs work, -2: queue exhausted
   double di[CH_NS];
   double E = 0.0, dt = 0.0, t = 0.0, h_cap = 0.0;
   int nsub = 0, nrej = 0;
+  bool first = true;
   Mech m = (Mech)&cm;
   while (true) {
     m = mech_opaque(m);
     const bool need = (cell == -1);
     const unsigned long long mask = __ballot(need);
     if (mask) {
-      const int leader = __ffsll((long long)mask) - 1;
-      unsigned long long base = 0;
-      if (lane == leader) base = atomicAdd(queue, (unsigned long long)__popcll(mask));
-      base = __shfl(base, leader);
+      unsigned long long my;
+      if (first) {
+        my = list ? blockIdx.x + (unsigned long long)lane * W : blockIdx.x * quota + lane;
+        if ((unsigned long long)lane >= quota) my = count;
+        first = false;
+      } else {
+        const int leader = __ffsll((long long)mask) - 1;
+        unsigned long long base = 0;
+        if (lane == leader) base = atomicAdd(queue, (unsigned long long)__popcll(mask));
+        my = W * quota + __shfl(base, leader) + (unsigned long long)__popcll(mask & lt);
+      }
       if (need) {
-        const unsigned long long my = base + (unsigned long long)__popcll(mask & lt);
         if (my < count) {
           cell = list ? (long)list[my] : (long)my;
           if (cell < 0 || cell >= n) cell = -1;  // a list entry outside the batch is skipped
@@ -649,12 +258,14 @@ __global__ __launch_bounds__(128) void k_chem_queue(long n, double* rho, double*
         }
       }
     }
-    if (__ballot(cell != -2) == 0) break;  // every lane has found the queue empty
+    const unsigned long long busy = __ballot(cell != -2);
+    if (busy == 0) break;  // every lane has found the queue empty
+    if (budget == 0 && __popcll(busy) <= COOP_TAIL && __ballot(cell == -1) == 0) break;  // the tail
     if (cell >= 0) {
       bool done = !(t < dt && nsub < ctl.max_sub && nrej < ctl.max_sub);
       double h = 0.0;
       if (!done) {
-        if (chem_adaptive_attempt(m, di, E, dt, t, h_cap, ctl, h)) {
+        if (chem_adaptive_attempt<ST>(m, L, di, E, dt, t, h_cap, ctl, h)) {
           t = t + h;
           nsub++;
           done = dt - t <= 1e-12 * dt;
@@ -680,216 +291,49 @@ __global__ __launch_bounds__(128) void k_chem_queue(long n, double* rho, double*
       }
     }
   }
-}
-
-// Cooperative integration of one cell per wavefront (64-thread workgroup).
-// Every lane holds the same copy of the cell state; the parallel parts (the
-// species' Gibbs functions, the reactions, ri, the Jacobian entries and the
-// Gauss elimination) exchange values through LDS, and every value is computed
-// with the same operations in the same order as chem_adaptive_attempt, so
-// the results are bit-identical to the per-lane integrator.
-struct CoopLds {
-  double gi[CH_NS];
-  double wf1[CH_NR_MAX], wr1[CH_NR_MAX];
-  double ri[CH_NS];
-  double A[CH_NS][CH_NS + 1];  // Jacobian, then the system; column CH_NS = right-hand side
-  double f[CH_NS];
-  double dA[CH_NR_MAX][CH_NS];  // d(rate of reaction k)/d(c_j), shared by every row i
-  // mechanism tables read with lane-dependent indices (staged once)
-  double coef[CH_NS][CH_NT_MAX][7];
-  double mi[CH_NS];
-  signed char vf[CH_NR_MAX][CH_NS], vr[CH_NR_MAX][CH_NS];
-};
-
-// comput_gibbs (CHEM_thermdyn.f90:296-319) with the coefficients from LDS
-__device__ __forceinline__ double coop_gibbs(Mech m, const double (*coefk)[7], double T, double logT) {
-  const int jc = trange(m, T);
-  const double* c = coefk[jc];
-  if (T <= m->tct_max)
-    return c[0] * (1.0 - logT) * T - c[1] * q2(T) / 2.0 - c[2] * q3(T) / 6.0 - c[3] * q4(T) / 12.0 - c[4] * q5(T) / 20.0 +
-           c[5] - c[6] * T;
-  const double tm = m->tct_max;
-  const double Cp_max = c[0] + c[1] * tm + c[2] * q2(tm) + c[3] * q3(tm) + c[4] * q4(tm);
-  const double h_max = c[0] * tm + c[1] * q2(tm) / 2.0 + c[2] * q3(tm) / 3.0 + c[3] * q4(tm) / 4.0 + c[4] * q5(tm) / 5.0 + c[5];
-  const double S_max = c[0] * log(tm) + c[1] * tm + c[2] * q2(tm) / 2.0 + c[3] * q3(tm) / 3.0 + c[4] * q4(tm) / 4.0 + c[6];
-  return h_max + Cp_max * (T - tm) - T * (S_max + Cp_max * log(T / tm));
-}
-
-__device__ bool coop_attempt(Mech m, CoopLds& L, const RxnConst& R, int lane, double* di, double& E, double dt,
-                             double t, double& h_cap, const ChemCtl& ctl, double& h_taken) {
-  double ci[CH_NS], sk[CH_NS], dd[CH_NS];
+  unsigned long long left = __ballot(cell >= 0);
+  if (left == 0) return;
   __syncthreads();
-  const double T = chem_T(m, di, E);
-  double rho = 0.0;
+  U.coop.tab[lane] = make_double2(cm.exp2t[lane][0], cm.exp2t[lane][1]);
+  coop_lds_init(m, U.coop.L, lane);
+  while (left) {
+    const int src = __ffsll((long long)left) - 1;
+    left &= left - 1;
+    double d1[CH_NS];
 #pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    ci[i] = (di[i] > 0.0 ? di[i] : 0.0) / m->mi[i] * 1.0e-6;
-    rho = rho + di[i];
+    for (int i = 0; i < CH_NS; i++) d1[i] = bcast(di[i], src);
+    const long c = __double_as_longlong(bcast(__longlong_as_double(cell), src));
+    coop_cell<ST>(m, U.coop.L, U.coop.tab, lane, c, n, rho, Ecell, d1, bcast(E, src), bcast(dt, src), bcast(t, src),
+                  bcast(h_cap, src), __builtin_amdgcn_readlane(nsub, src), __builtin_amdgcn_readlane(nrej, src), ctl,
+                  nsub_out, queue);
   }
-  if (lane < CH_NS) L.gi[lane] = coop_gibbs(m, L.coef[lane], T, log(T));
-  __syncthreads();
-  const int nr = m->nr;
-  if (lane < nr) {
-    double gi[CH_NS];
-#pragma unroll
-    for (int i = 0; i < CH_NS; i++) gi[i] = L.gi[i];
-    double wf1, wr1;
-    chem_reaction_c(R, T, gi, ci, wf1, wr1);
-    L.wf1[lane] = wf1;
-    L.wr1[lane] = wr1;
-  }
-  __syncthreads();
-  if (lane < CH_NS) {
-    double r = 0.0;
-    for (int k = 0; k < nr; k++) {
-      const int nu = L.vr[k][lane] - L.vf[k][lane];
-      if (nu != 0) r = r + (L.wf1[k] - L.wr1[k]) * nu;
-    }
-    L.ri[lane] = r;
-  }
-  // the factor (Awf - Awr) of chem_dA once per (reaction, species) ...
-  for (int e = lane; e < nr * CH_NS; e += 64) {
-    const int k = e / CH_NS, j = e % CH_NS;
-    const int vfj = L.vf[k][j], vrj = L.vr[k][j];
-    double cjv = ci[0];  // ci[j] for the lane-dependent j, without dynamic register indexing
-#pragma unroll
-    for (int q = 1; q < CH_NS; q++)
-      if (j == q) cjv = ci[q];
-    const double Awf = vfj * L.wf1[k] / (cjv + 1.0e-20);
-    const double Awr = vrj * L.wr1[k] / (cjv + 1.0e-20);
-    L.dA[k][j] = Awf - Awr;
-  }
-  __syncthreads();
-  // ... then every Jacobian entry sums its reactions in order
-  for (int e = lane; e < CH_NS * CH_NS; e += 64) {
-    const int i = e / CH_NS, j = e % CH_NS;
-    double a = 0.0;
-    for (int k = 0; k < nr; k++) {
-      if (L.vf[k][j] == 0 && L.vr[k][j] == 0) continue;
-      const int nu = L.vr[k][i] - L.vf[k][i];
-      if (nu != 0) a = a + L.dA[k][j] * nu;
-    }
-    L.A[i][j] = a;
-  }
-  __syncthreads();
-  double h = dt - t;
-  if (h_cap < h) h = h_cap;
-  double q = 0.0, rcv = 0.0;
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    const double w = L.ri[i] * m->mi[i] * 1.0e6;
-    sk[i] = ctl.rtol_y * ((di[i] > 0.0 ? di[i] : 0.0) + ctl.y_floor * rho);
-    if (fabs(w) * h > sk[i]) h = sk[i] / fabs(w);
-    q = q + w * m->ri[i] * m->coef[i][0][5];
-    rcv = rcv + 2.5 * m->ri[i] * di[i];
-  }
-  const double sT = ctl.rtol_t * T * rcv;
-  if (fabs(q) * h > sT) h = sT / fabs(q);
-  for (int e = lane; e < CH_NS * CH_NS; e += 64) {
-    const int i = e / CH_NS, j = e % CH_NS;
-    L.A[i][j] = (i == j ? 1.0 : 0.0) - L.A[i][j] * L.mi[i] / L.mi[j] * h;
-  }
-  if (lane < CH_NS) L.A[lane][CH_NS] = L.ri[lane] * L.mi[lane] * 1.0e6 * h;
-  __syncthreads();
-  // Gauss elimination with partial pivoting (CHEM_reactions.f90:523-567)
-  for (int k = 0; k < CH_NS - 1; k++) {
-    double fmax = fabs(L.A[k][k]);
-    int kk = k;
-    for (int i = k + 1; i < CH_NS; i++)
-      if (fabs(L.A[i][k]) > fmax) {
-        fmax = fabs(L.A[i][k]);
-        kk = i;
-      }
-    if (kk != k && lane >= k && lane <= CH_NS) {
-      const double tmp = L.A[k][lane];
-      L.A[k][lane] = L.A[kk][lane];
-      L.A[kk][lane] = tmp;
-    }
-    __syncthreads();
-    if (lane > k && lane < CH_NS) L.f[lane] = -L.A[lane][k] / L.A[k][k];
-    __syncthreads();
-    const int w = CH_NS + 1 - k;  // columns k .. CH_NS (right-hand side included)
-    for (int e = lane; e < (CH_NS - 1 - k) * w; e += 64) {
-      const int i = k + 1 + e / w, j = k + e % w;
-      L.A[i][j] = L.A[i][j] + L.f[i] * L.A[k][j];
-    }
-    __syncthreads();
-  }
-  dd[CH_NS - 1] = L.A[CH_NS - 1][CH_NS] / L.A[CH_NS - 1][CH_NS - 1];
-#pragma unroll
-  for (int i = CH_NS - 2; i >= 0; i--) {
-    double xi = L.A[i][CH_NS];
-#pragma unroll
-    for (int j = i + 1; j < CH_NS; j++) xi = xi - L.A[i][j] * dd[j];
-    dd[i] = xi / L.A[i][i];
-  }
-  bool ok = true;
-  double de = 0.0;
-#pragma unroll
-  for (int i = 0; i < CH_NS; i++) {
-    ok = ok && fabs(dd[i]) <= 2.0 * sk[i];
-    de = de + dd[i] * m->ri[i] * m->coef[i][0][5];
-  }
-  ok = ok && fabs(de) <= 2.0 * sT;
-  if (!ok) {
-    h_cap = 0.5 * h;
-    return false;
-  }
-  chem_apply(m, di, E, dd);
-  h_cap = 2.0 * h;
-  h_taken = h;
-  return true;
 }
 
 // One wavefront per handed-off cell, taken from a queue over the records.
-__global__ __launch_bounds__(64) void k_chem_coop(long n, double* rho, double* Ecell, const double* dtcell, ChemCtl ctl,
+template <class ST>
+__global__ __launch_bounds__(64, 2) void k_chem_coop(long n, double* rho, double* Ecell, const double* dtcell, ChemCtl ctl,
                                                   int* nsub_out, unsigned long long* queue, HeavyBuf hb) {
   __shared__ CoopLds L;
+  __shared__ double2 tab[CH_EXPN];
   const int lane = threadIdx.x;
   Mech m = (Mech)&cm;
   const unsigned long long count = queue[3];
-  // stage the lane-indexed mechanism data: this lane's reaction in
-  // registers, the stoichiometry, NASA coefficients and molar masses in LDS
-  const int nr = m->nr;
-  RxnConst R = load_rxn(m, lane < nr ? lane : 0);
-  for (int e = lane; e < CH_NR_MAX * CH_NS; e += 64) {
-    const int k = e / CH_NS, i = e % CH_NS;
-    L.vf[k][i] = (signed char)(k < nr ? m->vf[k][i] : 0);
-    L.vr[k][i] = (signed char)(k < nr ? m->vr[k][i] : 0);
-  }
-  for (int e = lane; e < CH_NS * CH_NT_MAX * 7; e += 64) {
-    const int i = e / (CH_NT_MAX * 7), j = (e / 7) % CH_NT_MAX, c = e % 7;
-    L.coef[i][j][c] = m->coef[i][j][c];
-  }
-  if (lane < CH_NS) L.mi[lane] = m->mi[lane];
-  __syncthreads();
+  tab[lane] = make_double2(cm.exp2t[lane][0], cm.exp2t[lane][1]);
+  coop_lds_init(m, L, lane);
   while (true) {
-    unsigned long long r = 0;
-    if (lane == 0) r = atomicAdd(queue + 4, 1ull);
-    r = __shfl(r, 0);
+    // No branch on the lane here: with `if (lane == 0)` at the end of one
+    // pass (chem_finish) and at the start of the next, the compiler may join
+    // the two and let the other lanes run ahead of lane 0, into a shuffle
+    // that reads a lane which is not there.
+    const unsigned long long rl = atomicAdd(queue + 4, lane == 0 ? 1ull : 0ull);
+    const unsigned long long r = (unsigned long long)__double_as_longlong(bcast(__longlong_as_double((long long)rl), 0));
     if (r >= count) break;
     const long c = hb.cell[r];
     double di[CH_NS];
 #pragma unroll
     for (int i = 0; i < CH_NS; i++) di[i] = hb.di[(long)i * hb.cap + r];
-    double E = hb.E[r], t = hb.t[r], h_cap = hb.h_cap[r];
-    int nsub = hb.nsub[r], nrej = hb.nrej[r];
-    const double dt = dtcell[c];
-    // every lane holds the same state: readfirstlane states that the loop
-    // decisions are uniform, which keeps the control flow scalar
-    while (__builtin_amdgcn_readfirstlane((t < dt && nsub < ctl.max_sub && nrej < ctl.max_sub) ? 1 : 0)) {
-      m = mech_opaque(m);
-      double h = 0.0;
-      const bool acc = coop_attempt(m, L, R, lane, di, E, dt, t, h_cap, ctl, h);
-      if (!__builtin_amdgcn_readfirstlane(acc ? 1 : 0)) {
-        nrej++;
-        continue;
-      }
-      t = t + h;
-      nsub++;
-      if (__builtin_amdgcn_readfirstlane((dt - t <= 1e-12 * dt) ? 1 : 0)) break;
-    }
-    if (lane == 0) chem_finish(c, n, rho, Ecell, di, E, nsub, t >= dt || dt - t <= 1e-12 * dt, nsub_out, queue);
+    coop_cell<ST>(m, L, tab, lane, c, n, rho, Ecell, di, hb.E[r], dtcell[c], hb.t[r], hb.h_cap[r], hb.nsub[r],
+                  hb.nrej[r], ctl, nsub_out, queue);
   }
 }
 
@@ -1361,31 +805,32 @@ int launch_adaptive(long n, double* rho, double* E, const double* dt, const Chem
                     unsigned long long* counter = nullptr) {
   if (!counter) counter = CX.counter;
   if (scheduler == 0 && !list) {
-    hipLaunchKernelGGL(k_chem_adaptive, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, CX.stream, n, rho, E, dt, ctl,
+    hipLaunchKernelGGL(CX.h2 ? k_chem_adaptive<ChemH2> : k_chem_adaptive<ChemAny>, dim3((unsigned)((n + CH_BLOCK - 1) / CH_BLOCK)), dim3(CH_BLOCK), 0, CX.stream, n, rho, E, dt, ctl,
                        nsub_out, counter);
     return hipGetLastError() == hipSuccess ? 0 : cfail("chemistry: launch failed");
   }
+  const auto queue = CX.h2 ? k_chem_queue<ChemH2> : k_chem_queue<ChemAny>;
   int dev = 0, ncu = 0, per = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_chem_queue, 128, 0) != hipSuccess)
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, queue, CH_BLOCK, 0) != hipSuccess)
     return cfail("chemistry: device query failed");
   if (per < 1) per = 1;
   long blocks = (long)ncu * per;
-  const long need = (n + 127) / 128;
-  if (blocks > need) blocks = need;
+  if (blocks > n) blocks = n;
   const bool coop = scheduler == 2;
   if (coop && ensure_heavy(n)) return 1;
-  hipLaunchKernelGGL(k_chem_queue, dim3((unsigned)blocks), dim3(128), 0, CX.stream, n, rho, E, dt, ctl, nsub_out,
+  hipLaunchKernelGGL(queue, dim3((unsigned)blocks), dim3(CH_BLOCK), 0, CX.stream, n, rho, E, dt, ctl, nsub_out,
                      counter, list, list_count, coop ? CX.coop_budget : 0, direct ? CX.coop_direct_max : 0,
                      coop ? CX.heavy : HeavyBuf{});
   if (coop) {
+    const auto coopk = CX.h2 ? k_chem_coop<ChemH2> : k_chem_coop<ChemAny>;
     int per2 = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per2, k_chem_coop, 64, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per2, coopk, 64, 0) != hipSuccess)
       return cfail("chemistry: device query failed");
     long b2 = (long)ncu * (per2 < 1 ? 1 : per2);
     if (b2 > n) b2 = n;
-    hipLaunchKernelGGL(k_chem_coop, dim3((unsigned)b2), dim3(64), 0, CX.stream, n, rho, E, dt, ctl, nsub_out,
+    hipLaunchKernelGGL(coopk, dim3((unsigned)b2), dim3(64), 0, CX.stream, n, rho, E, dt, ctl, nsub_out,
                        counter, CX.heavy);
   }
   return hipGetLastError() == hipSuccess ? 0 : cfail("chemistry: launch failed");
@@ -1501,18 +946,39 @@ int32_t ocfd_chem_set_mechanism(int32_t ns, int32_t nr, int32_t rereac, const in
   h.nr = nr;
   h.n_tct = n_tct;
   for (int j = 0; j < nr; j++) {
-    h.af_type[j] = af_type[j];
-    h.tb[j] = third_body[j];
-    h.fc[j] = fc_troe[j];
-    for (int a = 0; a < 2; a++)
-      for (int b = 0; b < 3; b++) h.arr[j][a][b] = arrhenius[(j * 2 + a) * 3 + b];
-    h.sgm[j] = 0;
-    for (int i = 0; i < ns; i++) {
-      h.vf[j][i] = vf[j * ns + i];
-      h.vr[j][i] = vr[j * ns + i];
-      h.eff[j][i] = eff[j * ns + i];
-      h.sgm[j] = h.sgm[j] + h.vr[j][i] - h.vf[j][i];
+    ChemRx& R = h.rx[j];
+    R.af_type = af_type[j];
+    R.tb = third_body[j];
+    const double* a = arrhenius + j * 6;
+    R.a0 = a[0]; R.b0 = a[1]; R.e0 = a[2];
+    R.a1 = a[3]; R.b1 = a[4]; R.e1 = a[5];
+    if (af_type[j] != 0 && af_type[j] != 2) {
+      R.lfc = std::log10(fc_troe[j]);
+      R.ac = -0.4 - (double)0.67f * R.lfc;  // REAL(4) literals of the reference
+      R.an = 0.75 - (double)1.27f * R.lfc;
     }
+    for (int i = 0; i < ns; i++) {
+      const int f = vf[j * ns + i], r = vr[j * ns + i];
+      R.vf[i] = f;
+      R.vr[i] = r;
+      R.nu[i] = r - f;
+      R.eff[i] = eff[j * ns + i];
+      R.sgm += r - f;
+      if (f != 0 || r != 0) R.part |= 1 << i;
+    }
+    // the mass-action products as species slots, where they fit (else ipow)
+    auto slots = [&](const int32_t* v, unsigned long long& s) {
+      s = 0;
+      int c = 0;
+      for (int i = 0; i < ns; i++) {
+        if (v[i] < 0 || c + v[i] > 8) return -1;
+        for (int q = 0; q < v[i]; q++) s |= (unsigned long long)i << (8 * c++);
+      }
+      for (int q = c; q < CH_SLOTS; q++) s |= (unsigned long long)CH_NS << (8 * q);
+      return c;
+    };
+    R.nsf = slots(vf + j * ns, R.sf);
+    R.nsr = slots(vr + j * ns, R.sr);
   }
   for (int j = 0; j < n_tct - 1; j++) h.tct[j] = tct[j];
   h.tct_max = tct_max;
@@ -1523,17 +989,39 @@ int32_t ocfd_chem_set_mechanism(int32_t ns, int32_t nr, int32_t rereac, const in
   for (int k = 0; k < ns; k++) {
     h.mi[k] = mi[k];
     h.ri[k] = CH_R0 / mi[k];
+    h.ci6[k] = 1.0e-6 / mi[k];
+    h.rcv[k] = 2.5 * h.ri[k];
     for (int j = 0; j < n_tct; j++)
       for (int c = 0; c < 7; c++) h.coef[k][j][c] = coef[(k * n_tct + j) * 7 + c];
-    h.ect[k][0] = 0.0;  // read_Spec, CHEM_thermdyn.f90:43-47
-    for (int j = 0; j < n_tct - 1; j++) {
-      const double t = h.tct[j];
-      h.ect[k][j + 1] = -((h.coef[k][j + 1][0] - h.coef[k][j][0]) * t + (h.coef[k][j + 1][1] - h.coef[k][j][1]) * P2(t) / 2.0 +
-                          (h.coef[k][j + 1][2] - h.coef[k][j][2]) * P3(t) / 3.0 +
-                          (h.coef[k][j + 1][3] - h.coef[k][j][3]) * P4(t) / 4.0 +
-                          (h.coef[k][j + 1][4] - h.coef[k][j][4]) * P5(t) / 5.0) +
-                        h.ect[k][j];
+    h.rf[k] = h.ri[k] * h.coef[k][0][5];
+    double ect = 0.0;  // read_Spec, CHEM_thermdyn.f90:43-47
+    for (int j = 0; j < n_tct; j++) {
+      const double* c = h.coef[k][j];
+      if (j > 0) {
+        const double t = h.tct[j - 1];
+        const double* p = h.coef[k][j - 1];
+        ect = -((c[0] - p[0]) * t + (c[1] - p[1]) * P2(t) / 2.0 + (c[2] - p[2]) * P3(t) / 3.0 +
+                (c[3] - p[3]) * P4(t) / 4.0 + (c[4] - p[4]) * P5(t) / 5.0) +
+              ect;
+      }
+      h.ev[j][0][k] = (c[0] - 1.0) * h.ri[k];
+      for (int a = 1; a < 5; a++) h.ev[j][a][k] = c[a] * h.ri[k];
+      h.ev[j][5][k] = ect * h.ri[k];
+      const double gb[7] = {c[0], c[1] / 2.0, c[2] / 6.0, c[3] / 12.0, c[4] / 20.0, c[5], c[6]};
+      for (int a = 0; a < 7; a++) h.gb[k][j][a] = gb[a];
     }
+  }
+  for (int j = 0; j < 64; j++) {
+    const long double v = std::exp2((long double)j / 64.0L);
+    h.exp2t[j][0] = (double)v;
+    h.exp2t[j][1] = (double)(v - (long double)h.exp2t[j][0]);
+  }
+  CX.h2 = rereac == 0 && nr == ChemH2::NR && n_tct == ChemH2::NT;
+  for (int j = 0; CX.h2 && j < nr; j++) {
+    const ChemRx& R = h.rx[j];
+    const int ar = (R.b0 != 0.0) | (R.e0 != 0.0) << 1 | (R.b1 != 0.0) << 2 | (R.e1 != 0.0) << 3;
+    CX.h2 = R.af_type == ChemH2::af[j] && (R.tb == 1) == (ChemH2::tb[j] == 1) && ar == ChemH2::ar[j];
+    for (int i = 0; i < ns; i++) CX.h2 = CX.h2 && R.vf[i] == ChemH2::vf[j][i] && R.vr[i] == ChemH2::vr[j][i];
   }
   if (!CX.own) {
     if (hipStreamCreateWithFlags(&CX.own, hipStreamNonBlocking) != hipSuccess) return cfail("no HIP device/stream");
@@ -1554,7 +1042,7 @@ int32_t ocfd_chem_set_reverse_rates(const double* rev) {
   if (!rev) return cfail("ocfd_chem_set_reverse_rates: null data");
   ChemMech& h = CX.h;
   for (int j = 0; j < h.nr; j++)
-    for (int a = 0; a < 5; a++) h.rev[j][a] = rev[j * 5 + a];
+    for (int a = 0; a < 5; a++) h.rx[j].r[a] = rev[j * 5 + a];
   if (hipDeviceSynchronize() != hipSuccess) return cfail("ocfd_chem_set_reverse_rates: device error");
   if (hipMemcpyToSymbol(HIP_SYMBOL(cm), &h, sizeof(ChemMech)) != hipSuccess) return cfail("hipMemcpyToSymbol failed");
   CX.rev_ready = true;
@@ -1568,12 +1056,12 @@ int32_t ocfd_chem_timeadv_batch(int64_t n, double* rho, double* E, const double*
   if (!CX.rev_ready) return cfail("ocfd_chem_timeadv_batch: ReReac 1/2 needs ocfd_chem_set_reverse_rates");
   if (n <= 0) return 0;
   if (nsub < 1) return cfail("ocfd_chem_timeadv_batch: nsub must be >= 1");
-  dim3 g((unsigned)((n + 127) / 128)), b(128);
+  dim3 g((unsigned)((n + CH_BLOCK - 1) / CH_BLOCK)), b(CH_BLOCK);
   switch (mode) {
-    case 1: hipLaunchKernelGGL(k_chem_fixed<1>, g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
-    case 2: hipLaunchKernelGGL(k_chem_fixed<2>, g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
-    case 3: hipLaunchKernelGGL(k_chem_fixed<3>, g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
-    case -1: hipLaunchKernelGGL(k_chem_fixed<-1>, g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
+    case 1: hipLaunchKernelGGL((CX.h2 ? k_chem_fixed<1, ChemH2> : k_chem_fixed<1, ChemAny>), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
+    case 2: hipLaunchKernelGGL((CX.h2 ? k_chem_fixed<2, ChemH2> : k_chem_fixed<2, ChemAny>), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
+    case 3: hipLaunchKernelGGL((CX.h2 ? k_chem_fixed<3, ChemH2> : k_chem_fixed<3, ChemAny>), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
+    case -1: hipLaunchKernelGGL((CX.h2 ? k_chem_fixed<-1, ChemH2> : k_chem_fixed<-1, ChemAny>), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
     default: return cfail("ocfd_chem_timeadv_batch: CHEM_TimeAdv must be 1, 2, 3 or -1");
   }
   if (hipGetLastError() != hipSuccess) return cfail("ocfd_chem_timeadv_batch: launch failed");
