@@ -61,6 +61,7 @@ struct DevState {
   const double* bl_pertb;
   // flow arrays
   double *f, *fn, *du, *di, *din;
+  double *duy, *duz;   // eta and zeta parts of du as the sweeps leave them (du: xi)
   double *d, *u, *v, *w, *T, *p, *Et, *Et_prev;
   double *Amu, *Amk;
   double *Axx, *Ayy, *Azz;

@@ -219,28 +219,43 @@ __device__ __forceinline__ void split_point(int kind, double Et1, double p1, dou
 // classifying and sorting again.  A list entry is (kind << 12) | entry.
 enum { KC_NONE = 0, KC_WRITE = 1, KC_READ = 2 };
 
+// LDS of a sweep tile: split fluxes (phase 1-2), interface values (phase
+// 2-3), the sorted list, per-pencil indices.
 template <int DIR, int V>
-__global__ __launch_bounds__((SweepTile<DIR, V>::NT)) void k_sweep(DevState S, int kmode, unsigned short* kc,
-                                                                   int* kct) {
+struct SweepLds {
+  using T = SweepTile<DIR, V>;
+  static constexpr int NPT = T::TS + 8, NIF = T::TS + 1, NE = 2 * T::NP * NIF;
+  double F[10 * T::NP * NPT];
+  double H[10 * T::NP * NIF];
+  PencilBase<DIR, T::NP> pb;
+  int cnt[T::NT / 64][10];
+  int total;
+  unsigned short list[NE];
+  unsigned char kind[NE];
+};
+
+// One tile lb of direction DIR, the tiles ordered along the pencil first (gx
+// tiles a pencil).  ACC: du is accumulated as the reference does, x into du, y
+// added to it, z added and multiplied by -Ajac; otherwise the direction's own
+// differences go to out and the update adds the three (RK_DU3).
+template <int DIR, int V, bool ACC>
+__device__ __forceinline__ void sweep_tile(const DevState& S, SweepLds<DIR, V>& L, long lb, int gx, int kmode,
+                                           unsigned short* kc, int* kct, double* __restrict__ out) {
   constexpr int NP = SweepTile<DIR, V>::NP, TS = SweepTile<DIR, V>::TS, NT = SweepTile<DIR, V>::NT;
   constexpr int NW = NT / 64;
   constexpr int NPT = TS + 8, NIF = TS + 1, NE = 2 * NP * NIF;
   static_assert(NT % 64 == 0, "whole wavefronts");
   static_assert(NE < 0x1000, "entry index must fit in 12 bits");
-  // split fluxes (phase 1-2) and interface values (phase 2-3)
-  __shared__ double sF[10 * NP * NPT];
-  __shared__ double sH[10 * NP * NIF];
-  __shared__ unsigned short sList[NE];
-  __shared__ unsigned char sKind[NE];
-  __shared__ int sCnt[NW][10];
-  __shared__ int sTotal;
-  __shared__ PencilBase<DIR, NP> PB;
+  double* const sF = L.F;
+  double* const sH = L.H;
+  unsigned short* const sList = L.list;
+  unsigned char* const sKind = L.kind;
+  int(*const sCnt)[10] = L.cnt;
+  int& sTotal = L.total;
+  PencilBase<DIR, NP>& PB = L.pb;
   const int n = S.n[DIR];
-  // XCD-aware tile order over the flattened 2-D grid
-  const long nb = (long)gridDim.x * gridDim.y;
-  const long lb = xcd_block((long)blockIdx.y * gridDim.x + blockIdx.x, nb);
-  const int bx = (int)(lb % gridDim.x);
-  const long by = lb / gridDim.x;
+  const int bx = (int)(lb % gx);
+  const long by = lb / gx;
   const int c0 = bx * TS + 1;
   const int ncell = min(TS, n - c0 + 1);
   const long npen = DIR == 0 ? (long)S.ny * S.nz : DIR == 1 ? (long)S.nx * S.nz : (long)S.nx * S.ny;
@@ -412,8 +427,8 @@ __global__ __launch_bounds__((SweepTile<DIR, V>::NT)) void k_sweep(DevState S, i
   }
   __syncthreads();
 
-  // phase 3: du from interface differences, one thread per cell for the
-  // five components (the cell's index work done once)
+  // phase 3: differences of the interface values, one thread per cell for
+  // the five components (the cell's index work done once)
   const double h1 = S.h_1[DIR];
   for (int r = tid; r < NP * TS; r += NT) {
     const int pl = DIR == 0 ? r / TS : r % NP;
@@ -428,20 +443,29 @@ __global__ __launch_bounds__((SweepTile<DIR, V>::NT)) void k_sweep(DevState S, i
       const double hp1 = Hc[m * NP * NIF + LIS], hp0 = Hc[m * NP * NIF];
       const double hm1 = Hc[(5 + m) * NP * NIF + LIS], hm0 = Hc[(5 + m) * NP * NIF];
       val[m] = (hp1 - hp0 + hm1 - hm0) * h1;
-      if (DIR != 0) old[m] = S.du[ci + (long)m * S.ni];
+      if (ACC && DIR != 0) old[m] = out[ci + (long)m * S.ni];
     }
-    if (DIR == 0) {
+    if (!ACC || DIR == 0) {
 #pragma unroll
-      for (int m = 0; m < 5; m++) S.du[ci + (long)m * S.ni] = val[m];
+      for (int m = 0; m < 5; m++) out[ci + (long)m * S.ni] = val[m];
     } else if (DIR == 1) {
 #pragma unroll
-      for (int m = 0; m < 5; m++) S.du[ci + (long)m * S.ni] = old[m] + val[m];
+      for (int m = 0; m < 5; m++) out[ci + (long)m * S.ni] = old[m] + val[m];
     } else {
       const double aj = S.Ajac[PB.hq1[pl] + (long)(c0 + c - 1) * S.sh[DIR]];
 #pragma unroll
-      for (int m = 0; m < 5; m++) S.du[ci + (long)m * S.ni] = -(old[m] + val[m]) * aj;
+      for (int m = 0; m < 5; m++) out[ci + (long)m * S.ni] = -(old[m] + val[m]) * aj;
     }
   }
+}
+
+template <int DIR, int V>
+__global__ __launch_bounds__((SweepTile<DIR, V>::NT)) void k_sweep(DevState S, int kmode, unsigned short* kc,
+                                                                   int* kct) {
+  __shared__ SweepLds<DIR, V> L;
+  // XCD-aware tile order over the flattened 2-D grid
+  const long lb = xcd_block((long)blockIdx.y * gridDim.x + blockIdx.x, (long)gridDim.x * gridDim.y);
+  sweep_tile<DIR, V, true>(S, L, lb, (int)gridDim.x, kmode, kc, kct, S.du);
 }
 
 // OCFD2d_flux1 / OCFD2d_flux2 over a batch of pencils (the 1-D scheme entry
@@ -645,6 +669,22 @@ __global__ __launch_bounds__(256) void k_sweep_char(DevState S) {
   }
 }
 
+// S.du = -((x + y) + z) Ajac: the inviscid right-hand side as one field, from
+// the parts that the sweeps left (the update adds them itself)
+__global__ __launch_bounds__(256) void k_du_sum(DevState S) {
+  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= S.ni) return;
+  const int i = (int)(c % S.nx) + 1;
+  const int j = (int)((c / S.nx) % S.ny) + 1;
+  const int k = (int)(c / ((long)S.nx * S.ny)) + 1;
+  const double aj = S.Ajac[hq(S, i, j, k)];
+#pragma unroll
+  for (int m = 0; m < 5; m++) {
+    const long e = c + m * S.ni;
+    S.du[e] = -((S.du[e] + S.duy[e]) + S.duz[e]) * aj;
+  }
+}
+
 #include "ocfd_species.h"
 #include "ocfd_diag.h"
 #include "ocfd_io.h"
@@ -808,9 +848,8 @@ __device__ __forceinline__ void visc_prep_cell(const DevState& S, long c, long q
 
 // one thread per cell
 template <int CD, bool MS, bool MT>
-__global__ __launch_bounds__(256) void k_visc_prep(DevState S) {
+__device__ __forceinline__ void visc_prep_at(const DevState& S, long c) {
   constexpr int R = CD == 1 ? 4 : 3;
-  const long c = cell_index();
   if (c >= S.ni) return;
   const int i = (int)(c % S.nx) + 1;
   const int j = (int)((c / S.nx) % S.ny) + 1;
@@ -837,6 +876,50 @@ __global__ __launch_bounds__(256) void k_visc_prep(DevState S) {
   if (ix && iy) visc_prep_cell<CD, MS, true, true, MT>(S, c, q, i, j, k, zd[0], zd[1], zd[2], zd[3]);
   else if (iy) visc_prep_cell<CD, MS, false, true, MT>(S, c, q, i, j, k, zd[0], zd[1], zd[2], zd[3]);
   else visc_prep_cell<CD, MS, false, false, MT>(S, c, q, i, j, k, zd[0], zd[1], zd[2], zd[3]);
+}
+template <int CD, bool MS, bool MT>
+__global__ __launch_bounds__(256) void k_visc_prep(DevState S) {
+  visc_prep_at<CD, MS, MT>(S, cell_index());
+}
+
+// A stage of a small grid in one launch: the three sweeps, each leaving its
+// own part of du, and the viscous preparation, on separate ranges of blocks.
+// None reads what another writes.  On a grid whose sweeps are a few rounds of
+// blocks each, every launch of its own costs its ramp, its last half-empty
+// round and 2 to 4 us between launches (with the preparation on a second
+// stream 10 us a stage for the fork and join): 32^3 box, us per RK3 step, 264
+// with one launch each, 192 without the second stream, 151 in this form (27
+// us of each stage's 50 are this launch).  A large grid keeps its launches:
+// its update is bound by memory and would read 80 B a cell more (640x120x64:
+// 5.95 against 5.51 ms per step).
+struct StageArgs {
+  long nb[3];  // sweep blocks of each direction (padded to multiples of 8 in the grid, one per XCD)
+  int gx[3], mode[3];
+  unsigned short* kc[3];
+  int* kct[3];
+};
+template <int CD, bool MT>
+__global__ __launch_bounds__(256) void k_stage(DevState S, StageArgs A) {
+  __shared__ union Lds {
+    SweepLds<0, 0> x;
+    SweepLds<1, 0> y;
+    SweepLds<2, 0> z;
+    __device__ Lds() {}
+  } U;
+  const long p0 = (A.nb[0] + 7) & ~7L, p1 = p0 + ((A.nb[1] + 7) & ~7L), p2 = p1 + ((A.nb[2] + 7) & ~7L);
+  const long b = (long)blockIdx.x;
+  if (b < p0) {
+    if (b < A.nb[0])
+      sweep_tile<0, 0, false>(S, U.x, xcd_block(b, A.nb[0]), A.gx[0], A.mode[0], A.kc[0], A.kct[0], S.du);
+  } else if (b < p1) {
+    if (b - p0 < A.nb[1])
+      sweep_tile<1, 0, false>(S, U.y, xcd_block(b - p0, A.nb[1]), A.gx[1], A.mode[1], A.kc[1], A.kct[1], S.duy);
+  } else if (b < p2) {
+    if (b - p1 < A.nb[2])
+      sweep_tile<2, 0, false>(S, U.z, xcd_block(b - p1, A.nb[2]), A.gx[2], A.mode[2], A.kc[2], A.kct[2], S.duz);
+  } else {
+    visc_prep_at<CD, false, MT>(S, xcd_block(b - p2, (long)gridDim.x - p2) * blockDim.x + threadIdx.x);
+  }
 }
 
 // marching over k planes with the z windows of u, v, w, T in registers.
@@ -994,7 +1077,13 @@ __global__ __launch_bounds__(256) void k_transport(DevState S) {
 // The flags select the pieces so the per-stage entry points share this code.
 // A cell with Et <= 0 is recorded for handle_NegativeEt (k_negt_repair).
 // ===========================================================================
-enum { RK_MASS = 1, RK_VISC = 2, RK_WRITE_DU = 4, RK_UPDATE_F = 8, RK_PRIMS = 16, RK_DI_FROM_D = 32, RK_MS = 64 };
+// RK_DU3: the inviscid right-hand side comes as the sweeps' three parts
+// (S.du, S.duy, S.duz), added here in their order.  So no sweep waits for
+// another's result or reads it back; each kernel moves the same bytes.
+// RK_SAVE0 (krk = 1): the stage starts from fn = f, kept here from the f that
+// the update reads, instead of by a copy kernel ahead of the step.
+enum { RK_MASS = 1, RK_VISC = 2, RK_WRITE_DU = 4, RK_UPDATE_F = 8, RK_PRIMS = 16, RK_DI_FROM_D = 32, RK_MS = 64,
+       RK_DU3 = 128, RK_SAVE0 = 256 };
 
 // The stepping path's flag sets are compile-time (F >= 0), so the kernel is
 // straight-line code and its loads can be in flight together; F = -1 reads
@@ -1008,16 +1097,25 @@ __device__ __forceinline__ void rk_cell(const DevState& S, long c, long q, int i
   const long ni = S.ni;
   const double d_old = S.d[q];
   double du[5];
-  if (flags & (RK_MASS | RK_VISC | RK_UPDATE_F)) {
+  const double ajac = (flags & (RK_VISC | RK_DU3)) ? jac_at<MT>(S, q, i, j, k) : 0.0;
+  if (flags & RK_DU3) {
+#pragma unroll
+    for (int m = 0; m < 5; m++) {
+      const long e = c + m * ni;
+      du[m] = -((S.du[e] + S.duy[e]) + S.duz[e]) * ajac;
+    }
+  } else if (flags & (RK_MASS | RK_VISC | RK_UPDATE_F)) {
 #pragma unroll
     for (int m = 0; m < 5; m++) du[m] = S.du[c + m * ni];
   }
   // the stage's old solution, read before the flux divergence so that its
   // loads overlap the stencil loads
   double fnv[5], fov[5];
+  const bool save0 = (flags & RK_SAVE0) && krk == 1;
   if (flags & RK_UPDATE_F) {
+    const double* f0 = save0 ? S.f : S.fn;
 #pragma unroll
-    for (int m = 0; m < 5; m++) fnv[m] = S.fn[c + m * ni];
+    for (int m = 0; m < 5; m++) fnv[m] = f0[c + m * ni];
     if (krk != 1) {
 #pragma unroll
       for (int m = 0; m < 5; m++) fov[m] = S.f[c + m * ni];
@@ -1030,7 +1128,6 @@ __device__ __forceinline__ void rk_cell(const DevState& S, long c, long q, int i
     du[4] = du[4] + d_old * (S.u[q] * S.mf[0] + S.v[q] * S.mf[1] + S.w[q] * S.mf[2]);
   }
   if (flags & RK_VISC) {
-    const double ajac = jac_at<MT>(S, q, i, j, k);
     double uk[4], ui[4];
     constexpr int R = CD == 1 ? 4 : 3;
     // generic taps (closures, periodic wrap) of component m of direction g
@@ -1096,6 +1193,11 @@ __device__ __forceinline__ void rk_cell(const DevState& S, long c, long q, int i
     if (krk == 1) {
 #pragma unroll
       for (int m = 0; m < 5; m++) f[m] = fnv[m] + dt * du[m];
+      if (save0) {
+#pragma unroll
+        for (int m = 0; m < 5; m++) S.fn[c + m * ni] = fnv[m];
+        S.din[c] = S.di[q];
+      }
     } else {
       const double ra = krk == 2 ? 3.0 / 4.0 : 1.0 / 3.0;
       const double rb = krk == 2 ? 1.0 / 4.0 : 2.0 / 3.0;
@@ -2157,6 +2259,7 @@ struct Ctx {
   hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_qp = nullptr;
   int concurrent = 1;
   int use_graph = 0;
+  bool du_parts = false;     // S.du, duy, duz hold the sweeps' parts, not their sum
   int metric_tables = 0;     // OCFD_OPT_METRIC_TABLES (off: the divisions cost more than the loads)
   double* filt_tmp = nullptr;  // ocfd_filtering's copy of f
   long bl_nin = 0, bl_nup = 0;  // lengths of the boundary-layer inlet and upper data
@@ -2285,8 +2388,16 @@ void launch_rk_f(int krk, double dt, int flags) {
 
 template <int CD>
 void launch_rk_cd(int krk, double dt, int flags) {
-  constexpr int STEP1 = RK_VISC | RK_UPDATE_F | RK_PRIMS | RK_DI_FROM_D;
+  constexpr int STEP1 = RK_SAVE0 | RK_VISC | RK_UPDATE_F | RK_PRIMS | RK_DI_FROM_D;
   constexpr int STEPMS = RK_VISC | RK_UPDATE_F | RK_PRIMS | RK_MS;
+  if (flags & RK_DU3) {  // small grids: one thread per cell
+    constexpr int STEPS = STEP1 | RK_DU3;
+    const DevState& S = G.S;
+    const auto kern = flags == STEPS ? (S.mt_on ? k_rk<CD, STEPS, true> : k_rk<CD, STEPS, false>)
+                                     : (S.mt_on ? k_rk<CD, -1, true> : k_rk<CD, -1, false>);
+    launch("k_rk", kern, grid1(S.ni), dim3(256), S, krk, dt, flags);
+    return;
+  }
   switch (flags) {
     case STEP1: launch_rk_f<CD, STEP1>(krk, dt, flags); break;
     case STEP1 & ~RK_VISC: launch_rk_f<CD, (STEP1 & ~RK_VISC)>(krk, dt, flags); break;
@@ -2396,6 +2507,49 @@ void launch_sweep() {
   launch_sweep_variant<DIR>(G.sweep_variant[DIR]);
 }
 
+void enq_sweeps() {
+  launch_sweep<0>();
+  launch_sweep<1>();
+  launch_sweep<2>();
+  G.du_parts = false;
+}
+
+// Grids up to this many cells take the small grid's stage (k_stage).  us per
+// RK3 step, k_stage / separate launches, on periodic boxes: 48^3 253 / 348,
+// 64^3 504 / 535, 80^3 946 / 976, 88^3 1201 / 1184, 96^3 1473 / 1412; on
+// plates: 161x61x33 605 / 678, 200x61x40 844 / 900, 240x81x33 (642,000
+// cells) 1163 / 1165, 320x80x33 1443 / 1365.  Above the line the update's
+// 80 B a cell more outweigh the ramps and gaps saved.  Only the default tiles
+// have a form in k_stage, and a timed run shows the kernels one by one.
+constexpr long SMALL_CELLS = 1L << 19;
+bool small_stage() {
+  return G.S.ns == 1 && G.S.viscous && G.S.ni <= SMALL_CELLS && !G.cfg.if_scheme_character && !G.timing &&
+         G.col_planes < 0 && G.sweep_variant[0] == 0 && G.sweep_variant[1] == 0 && G.sweep_variant[2] == 0;
+}
+
+void enq_small_sweeps() {
+  const DevState& S = G.S;
+  StageArgs A{};
+  long grid = 0;
+  auto dir = [&](int d, int np, int ts, long npen) {
+    A.gx[d] = (S.n[d] + ts - 1) / ts;
+    A.nb[d] = A.gx[d] * ((npen + np - 1) / np);
+    A.mode[d] = G.kc_var[d] == 0 ? KC_READ : KC_WRITE;
+    G.kc_var[d] = 0;
+    A.kc[d] = G.kc[d];
+    A.kct[d] = G.kct[d];
+    grid += (A.nb[d] + 7) / 8 * 8;
+  };
+  dir(0, SweepTile<0, 0>::NP, SweepTile<0, 0>::TS, (long)S.ny * S.nz);
+  dir(1, SweepTile<1, 0>::NP, SweepTile<1, 0>::TS, (long)S.nx * S.nz);
+  dir(2, SweepTile<2, 0>::NP, SweepTile<2, 0>::TS, (long)S.nx * S.ny);
+  grid += (S.ni + 255) / 256;
+  const auto kern = S.mt_on ? (S.cd8 ? k_stage<1, true> : k_stage<0, true>)
+                            : (S.cd8 ? k_stage<1, false> : k_stage<0, false>);
+  launch("k_stage", kern, dim3((unsigned)grid), dim3(256), S, A);
+  G.du_parts = true;
+}
+
 template <int SCALE, bool REDO = false>
 void launch_masks() {
   const DevState& S = G.S;
@@ -2452,20 +2606,19 @@ void enq_bc() {
 
 void enq_stage(int krk, double dt1) {
   const DevState& S = G.S;
+  const bool small = small_stage();
+  const int flags = (S.mass_force ? RK_MASS : 0) | (S.viscous ? RK_VISC : 0) | (small ? RK_DU3 : 0) | RK_SAVE0 |
+                    RK_UPDATE_F | RK_PRIMS | RK_DI_FROM_D;
   // the viscous preparation does not read the hybrid masks: fork before the sensor
-  const hipStream_t vs = fork_side();
-  if (S.viscous) launch_visc_prep(false, vs);
-  else launch_s(vs, "k_transport", k_transport, grid1(S.ni), dim3(256), S);
-  // the step's saved solution (fn, din) is first read by this stage's
-  // k_rk, after the join: its copy runs beside the sweeps (k_save0 is
-  // launched inside stage 1 on either path)
-  if (krk == 1) launch_s(vs, "k_save0", k_save0, grid1(S.ni), dim3(256), S);
+  const hipStream_t vs = small ? G.stream : fork_side();
+  if (!small) {
+    if (S.viscous) launch_visc_prep(false, vs);
+    else launch_s(vs, "k_transport", k_transport, grid1(S.ni), dim3(256), S);
+  }
   if (krk == 1 && G.cfg.scheme_invis == OCFD_SCHEME_HYBRID) enq_rhybrid();
-  launch_sweep<0>();
-  launch_sweep<1>();
-  launch_sweep<2>();
+  if (small) enq_small_sweeps();
+  else enq_sweeps();
   join_side(vs);
-  const int flags = (S.mass_force ? RK_MASS : 0) | (S.viscous ? RK_VISC : 0) | RK_UPDATE_F | RK_PRIMS | RK_DI_FROM_D;
   launch("k_negt_reset", k_negt_reset, dim3(1), dim3(64), S, 0);
   launch_rk(krk, dt1, flags);
   launch("k_negt_repair", k_negt_repair, dim3(1), dim3(64), S);
@@ -2542,9 +2695,7 @@ void enq_stage_ms(int krk, double dt1) {
   // the second stream, fn by k_rk after the join
   if (krk == 1) launch_s(sp, "k_save0", k_save0, grid1(S.ni), dim3(256), S);
   enq_species(krk, dt1, sp, sp != G.stream ? G.ev_qp : nullptr);
-  launch_sweep<0>();
-  launch_sweep<1>();
-  launch_sweep<2>();
+  enq_sweeps();
   if (S.viscous) {
     if (sp != G.stream) hipStreamWaitEvent(G.stream, G.ev_qp, 0);
     launch_visc_prep(true);
@@ -2565,6 +2716,13 @@ void enq_step(double dt1) {
     else enq_stage(krk, dt1);
   }
   hipMemcpyAsync(G.h_negt, S.negt + 17, sizeof(int), hipMemcpyDeviceToHost, G.stream);
+}
+
+// S.du as one field, for whoever reads it apart from the update
+void du_whole() {
+  if (!G.du_parts) return;
+  launch("k_du_sum", k_du_sum, grid1(G.S.ni), dim3(256), G.S);
+  G.du_parts = false;
 }
 
 void drop_graph() {
@@ -2679,6 +2837,7 @@ int32_t ocfd_init(const ocfd_cfg* cfg) {
   G.col_planes = -1;
   G.concurrent = 1;
   G.use_graph = 0;
+  G.du_parts = false;
   G.timing = 0;
   if (!cfg) return fail("ocfd_init: null config");
   const ocfd_cfg& c = *cfg;
@@ -2776,8 +2935,10 @@ int32_t ocfd_init(const ocfd_cfg* cfg) {
       hipEventCreateWithFlags(&G.ev_qp, hipEventDisableTiming) != hipSuccess)
     return fail("ocfd_init: stream or event creation failed");
   const long nh = S.nh, ni = S.ni, ns = S.ns, nms = S.ns > 1 ? S.ns : 0;
+  const long nsm = S.ns == 1 && ni <= SMALL_CELLS ? 5 * ni : 0;  // the small grid's stage alone uses them
   struct { double** p; long n; double v; } arrs[] = {
-      {&S.f, 5 * ni, 0.0}, {&S.fn, 5 * ni, 0.0}, {&S.du, 5 * ni, 0.0}, {&S.di, nh * ns, 1.0}, {&S.din, ni * ns, 1.0},
+      {&S.f, 5 * ni, 0.0}, {&S.fn, 5 * ni, 0.0}, {&S.du, 5 * ni, 0.0}, {&S.duy, nsm, 0.0}, {&S.duz, nsm, 0.0},
+      {&S.di, nh * ns, 1.0}, {&S.din, ni * ns, 1.0},
       {&S.AmD, ni * nms, 0.0}, {&S.dus, ni * nms, 0.0}, {&S.Evs, 3 * ni * nms, 0.0}, {&S.Qp, 3 * ni, 0.0}, {&S.cs, ni * nms, 0.0},
       {(double**)&S.jet_in, (long)S.ny * S.nz * (5 + ns), 1.0},
       {&S.d, nh, 1.0}, {&S.u, nh, 1.0}, {&S.v, nh, 1.0}, {&S.w, nh, 1.0}, {&S.T, nh, 300.0}, {&S.p, nh, 1.0},
@@ -3006,6 +3167,7 @@ int32_t ocfd_set_bc_jet(const double* inlet2d) {
 // A*1 = A*/Ajac arrays.
 static int mesh_setup(const double* axx, const double* ayy, const double* azz, const double* span,
                       const double* metrics) {
+  du_whole();  // with the Jacobian that the step had
   DevState& S = G.S;
   const size_t bytes = sizeof(double) * (size_t)S.nh;
   // staging buffer, freed on every return path (hipFree waits for the device)
@@ -3272,6 +3434,8 @@ int32_t ocfd_upload_field(int32_t field, const double* host) {
   long n;
   double* p = field_ptr(field, &n);
   if (!p || !host) return fail("ocfd_upload_field: bad field id or null pointer");
+  if (field == OCFD_FIELD_DU) G.du_parts = false;
+  else if (field == OCFD_FIELD_AJAC) du_whole();  // with the Jacobian that the step had
   HIPCHK(hipMemcpyAsync(p, host, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, G.stream));
   HIPCHK(hipStreamSynchronize(G.stream));
   return 0;
@@ -3281,6 +3445,7 @@ int32_t ocfd_download_field(int32_t field, double* host) {
   if (check_ready()) return 1;
   long n;
   double* p = field_ptr(field, &n);
+  if (p && field == OCFD_FIELD_DU) du_whole();
   if (!p || !host) return fail("ocfd_download_field: bad field id or null pointer");
   HIPCHK(hipMemcpyAsync(host, p, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, G.stream));
   HIPCHK(hipStreamSynchronize(G.stream));
@@ -3342,6 +3507,7 @@ int32_t ocfd_flow_time_advance(double dt1) {
   } else {
     enq_step(dt1);
   }
+  G.du_parts = G.S.ns == 1 && small_stage();  // also after a replay
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -3380,9 +3546,7 @@ int32_t ocfd_comput_rhybrid(void) {
 }
 int32_t ocfd_du_inviscous(void) {
   if (check_ready()) return 1;
-  launch_sweep<0>();
-  launch_sweep<1>();
-  launch_sweep<2>();
+  enq_sweeps();
   if (G.S.mass_force) launch_rk(1, 0.0, (int)(RK_MASS | RK_WRITE_DU));
   HIPCHK(hipGetLastError());
   return 0;
@@ -3413,6 +3577,7 @@ int32_t ocfd_flux1d_batch(int32_t side, int32_t scheme, int64_t npen, int32_t n,
 int32_t ocfd_du_viscous(void) {
   if (check_ready()) return 1;
   launch_visc_prep(G.S.ns > 1);
+  du_whole();
   launch_rk(1, 0.0, (int)(RK_VISC | RK_WRITE_DU));
   HIPCHK(hipGetLastError());
   return 0;
@@ -3420,6 +3585,7 @@ int32_t ocfd_du_viscous(void) {
 int32_t ocfd_time_adv_rk3(int32_t krk, double dt) {
   if (check_ready()) return 1;
   if (krk < 1 || krk > 3) return fail("ocfd_time_adv_rk3: KRK must be 1, 2 or 3");
+  du_whole();
   launch_rk((int)krk, dt, (int)RK_UPDATE_F);
   HIPCHK(hipGetLastError());
   return 0;
@@ -3679,6 +3845,7 @@ int32_t ocfd_autotune(int32_t reps) {
   }
   hipEventDestroy(a);
   hipEventDestroy(b);
+  G.du_parts = false;
   G.timing = saved_timing;
   HIPCHK(hipGetLastError());
   return 0;
