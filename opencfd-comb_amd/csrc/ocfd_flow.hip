@@ -685,6 +685,16 @@ __global__ __launch_bounds__(256) void k_du_sum(DevState S) {
   }
 }
 
+// Negative-Et bookkeeping (Num_NegT=0, Comput_flow_variables.f90:8): negt[18 +
+// krk] counts the bad cells of stage krk, negt[1..16] lists the first of them,
+// negt[17] is the step's largest count.  Every stage has its own counter, so
+// one reset serves a step: the counter of a stage is read by every block of
+// its boundary kernel, which could not clear it.
+__device__ __forceinline__ void negt_reset(const DevState& S, int step) {
+  for (int krk = 1; krk <= 3; krk++) S.negt[18 + krk] = 0;
+  if (step) S.negt[17] = 0;
+}
+
 #include "ocfd_species.h"
 #include "ocfd_diag.h"
 #include "ocfd_io.h"
@@ -895,6 +905,7 @@ __global__ __launch_bounds__(256) void k_visc_prep(DevState S) {
 struct StageArgs {
   long nb[3];  // sweep blocks of each direction (padded to multiples of 8 in the grid, one per XCD)
   int gx[3], mode[3];
+  int first;   // the step's first stage: it resets the negative-Et counters
   unsigned short* kc[3];
   int* kct[3];
 };
@@ -908,6 +919,7 @@ __global__ __launch_bounds__(256) void k_stage(DevState S, StageArgs A) {
   } U;
   const long p0 = (A.nb[0] + 7) & ~7L, p1 = p0 + ((A.nb[1] + 7) & ~7L), p2 = p1 + ((A.nb[2] + 7) & ~7L);
   const long b = (long)blockIdx.x;
+  if (A.first && b == 0 && threadIdx.x == 0) negt_reset(S, 1);
   if (b < p0) {
     if (b < A.nb[0])
       sweep_tile<0, 0, false>(S, U.x, xcd_block(b, A.nb[0]), A.gx[0], A.mode[0], A.kc[0], A.kct[0], S.du);
@@ -1075,7 +1087,7 @@ __global__ __launch_bounds__(256) void k_transport(DevState S) {
 //   f = alpha*fn + beta*(f + dt*du)                      (OCFD_Time_Adv.f90:98-130)
 //   d,u,v,w,Et from f; Rescaling_di; T(E); p             (Comput_flow_variables.f90:3-46,101-121)
 // The flags select the pieces so the per-stage entry points share this code.
-// A cell with Et <= 0 is recorded for handle_NegativeEt (k_negt_repair).
+// A cell with Et <= 0 is recorded for handle_NegativeEt (negt_repair).
 // ===========================================================================
 // RK_DU3: the inviscid right-hand side comes as the sweeps' three parts
 // (S.du, S.duy, S.duz), added here in their order.  So no sweep waits for
@@ -1216,7 +1228,7 @@ __device__ __forceinline__ void rk_cell(const DevState& S, long c, long q, int i
   const double Et = f[4] - (f[1] * uu + f[2] * vv + f[3] * ww) * 0.5;
   S.Et_prev[c] = S.Et[q];
   if (Et <= 0.0) {
-    const int slot = atomicAdd(&S.negt[0], 1);
+    const int slot = atomicAdd(&S.negt[18 + krk], 1);
     if (slot < 16) S.negt[1 + slot] = (int)c;
   }
   if (flags & RK_MS) {
@@ -1361,24 +1373,20 @@ __global__ __launch_bounds__(256) void k_di_from_d(DevState S) {
   if (q < S.nh) S.di[q] = S.d[q];
 }
 
-// start of a stage's negative-Et bookkeeping (Num_NegT=0, Comput_flow_variables.f90:8)
-__global__ void k_negt_reset(DevState S, int all) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    S.negt[0] = 0;
-    if (all) S.negt[17] = 0;
-  }
+// the reset where no other kernel of the step's start does it
+__global__ void k_negt_reset(DevState S, int step) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) negt_reset(S, step);
 }
 
 // handle_NegativeEt (OCFD_handle_NegativeT.f90:1-20), replayed in the
 // reference's (k,j,i) order by one thread: a neighbour already visited by
 // the reference loop holds its new Et, a later one (and every ghost) its old.
-__global__ void k_negt_repair(DevState S) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const int cnt = S.negt[0];
+// idx: 16 entries of LDS
+__device__ __forceinline__ void negt_repair(const DevState& S, int krk, int* idx) {
+  const int cnt = S.negt[18 + krk];
   if (cnt > S.negt[17]) S.negt[17] = cnt;
   if (cnt == 0) return;
   int n = cnt < 16 ? cnt : 16;
-  int idx[16];
   for (int a = 0; a < n; a++) idx[a] = S.negt[1 + a];
   for (int a = 1; a < n; a++) {
     int x = idx[a], b = a - 1;
@@ -1420,6 +1428,10 @@ __global__ void k_negt_repair(DevState S) {
     S.p[q] = 0.0 + S.Ri0 * di * T;
   }
 }
+__global__ void k_negt_repair(DevState S) {  // after comput_flow_variables
+  __shared__ int idx[16];
+  if (threadIdx.x == 0 && blockIdx.x == 0) negt_repair(S, 1, idx);
+}
 
 // ===========================================================================
 // Boundary conditions (OCFD_bc, OCFD_BC.f90:2-188; boundary layer case
@@ -1434,10 +1446,7 @@ __device__ __forceinline__ double bl_data(const double* r, int kind, int a, int 
   return r[(a - 1) + (long)na * ((b - 1) + (long)nb * m)];
 }
 
-__global__ void k_bl_inlet(DevState S) {  // :50-97 (BcData_inlet = 0, 1, 2)
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)S.ny * S.nz) return;
-  const int j = (int)(t % S.ny) + 1, k = (int)(t / S.ny) + 1;
+__device__ __forceinline__ void bl_inlet(const DevState& S, int j, int k) {  // :50-97 (BcData_inlet = 0, 1, 2)
   const long q = hq(S, 1, j, k);
   const double* r = S.bl_in;
   const int kind = S.bl_inlet;
@@ -1449,11 +1458,9 @@ __global__ void k_bl_inlet(DevState S) {  // :50-97 (BcData_inlet = 0, 1, 2)
   S.di[q] = bl_data(r, kind, j, k, S.ny, S.nz, 5);
 }
 
-__global__ void k_bl_upper(DevState S) {  // :100-140 (BcData_upper = 0, 1, 2; Dirichlet where not non-reflecting)
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)S.nx * S.nz) return;
-  if (S.bl_nonref[t] != 0) return;
-  const int i = (int)(t % S.nx) + 1, k = (int)(t / S.nx) + 1;
+// :100-140 (BcData_upper = 0, 1, 2; Dirichlet where not non-reflecting)
+__device__ __forceinline__ void bl_upper(const DevState& S, int i, int k) {
+  if (S.bl_nonref[(i - 1) + (long)S.nx * (k - 1)] != 0) return;
   const long q = hq(S, i, S.ny, k);
   const double* r = S.bl_up;
   const int kind = S.bl_upper;
@@ -1465,10 +1472,9 @@ __global__ void k_bl_upper(DevState S) {  // :100-140 (BcData_upper = 0, 1, 2; D
   S.di[q] = bl_data(r, kind, i, k, S.nx, S.nz, 5);
 }
 
-__global__ void k_bl_wall(DevState S) {  // :143-201 (isothermal, non-catalytic, blow/suction)
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)S.nx * S.nz) return;
-  const int i = (int)(t % S.nx) + 1, k = (int)(t / S.nx) + 1;
+// :143-201 (isothermal, non-catalytic, blow/suction)
+__device__ __forceinline__ void bl_wall(const DevState& S, int i, int k) {
+  const long t = (i - 1) + (long)S.nx * (k - 1);
   const long q1 = hq(S, i, 1, k), q2 = hq(S, i, 2, k), q3 = hq(S, i, 3, k);
   if (S.Axx[q1] < S.bl_xinit) {
     S.d[q1] = S.d[q2];
@@ -1499,10 +1505,7 @@ __global__ void k_bl_wall(DevState S) {  // :143-201 (isothermal, non-catalytic,
   S.di[q1] = di1 * d1;
 }
 
-__global__ void k_bl_outlet(DevState S) {  // :203-232 (types 1 and 2)
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)S.ny * S.nz) return;
-  const int j = (int)(t % S.ny) + 1, k = (int)(t / S.ny) + 1;
+__device__ __forceinline__ void bl_outlet(const DevState& S, int j, int k) {  // :203-232 (types 1 and 2)
   const long q = hq(S, S.nx, j, k), qa = hq(S, S.nx - 1, j, k), qb = hq(S, S.nx - 2, j, k);
   double* arr[6] = {S.d, S.u, S.v, S.w, S.T, S.di};
   for (int a = 0; a < 6; a++) arr[a][q] = S.bl_outlet == 1 ? arr[a][qa] : 2.0 * arr[a][qa] - arr[a][qb];
@@ -1530,27 +1533,101 @@ __device__ __forceinline__ void face_update(const DevState& S, long q, long c) {
   S.f[c + 4 * S.ni] = Et + dd * (uu * uu + vv * vv + ww * ww) * 0.5;
 }
 
-__global__ void k_bc_faces(DevState S) {
-  const int nx = S.nx, ny = S.ny, nz = S.nz;
-  const long nxi = nx > 2 ? nx - 2 : 0, nyi = ny > 2 ? ny - 2 : 0;
-  const long n0 = (long)ny * nz, n1 = nx > 1 ? (long)ny * nz : 0;
-  const long n2 = nxi * nz, n3 = ny > 1 ? nxi * nz : 0;
-  const long n4 = nxi * nyi, n5 = nz > 1 ? nxi * nyi : 0;
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int i, j, k;
-  if (t < n0) { i = 1; j = (int)(t % ny) + 1; k = (int)(t / ny) + 1; }
-  else if ((t -= n0) < n1) { i = nx; j = (int)(t % ny) + 1; k = (int)(t / ny) + 1; }
-  else if ((t -= n1) < n2) { i = (int)(t % nxi) + 2; j = 1; k = (int)(t / nxi) + 1; }
-  else if ((t -= n2) < n3) { i = (int)(t % nxi) + 2; j = ny; k = (int)(t / nxi) + 1; }
-  else if ((t -= n3) < n4) { i = (int)(t % nxi) + 2; j = (int)(t / nxi) + 2; k = 1; }
-  else if ((t -= n4) < n5) { i = (int)(t % nxi) + 2; j = (int)(t / nxi) + 2; k = nz; }
-  else return;
+template <bool MS>
+__device__ __forceinline__ void face_cell(const DevState& S, int i, int j, int k) {
   const long q = hq(S, i, j, k), c = iq(S, i, j, k);
-  const int nf = (i == 1) + (i == nx) + (j == 1) + (j == ny) + (k == 1) + (k == nz);
+  const int nf = (i == 1) + (i == S.nx) + (j == 1) + (j == S.ny) + (k == 1) + (k == S.nz);
   for (int a = 0; a < nf; a++) {
-    if (S.ns > 1) face_update_ms(S, q, c);
+    if (MS) face_update_ms(S, q, c);
     else face_update(S, q, c);
   }
+}
+
+// One k plane: the conditions of the i and j faces in the reference's order,
+// then the faces' conserved variables.  The conditions read and write cells
+// of their own plane only, so a block does them with barriers in between.
+template <int BC, bool MS>
+__device__ void bc_plane(const DevState& S, int k) {
+  const int nx = S.nx, ny = S.ny, nz = S.nz, t0 = (int)threadIdx.x, nt = (int)blockDim.x;
+  if (BC == OCFD_BC_BOUNDARYLAYER) {
+    for (int t = t0; t < ny; t += nt) bl_inlet(S, t + 1, k);
+    __syncthreads();
+    // BcData_upper = -1: no upper data; the face keeps its values.  The wall
+    // reads rows 2 and 3, which the upper data (row ny >= 8) do not touch.
+    for (int t = t0; t < 2 * nx; t += nt) {
+      if (t >= nx) bl_wall(S, t - nx + 1, k);
+      else if (S.bl_upper >= 0) bl_upper(S, t + 1, k);
+    }
+    __syncthreads();
+    if (S.bl_outlet == 1 || S.bl_outlet == 2)
+      for (int t = t0; t < ny; t += nt) bl_outlet(S, t + 1, k);
+    __syncthreads();
+  } else if (BC == OCFD_BC_JET) {
+    for (int t = t0; t < 2 * ny; t += nt) {
+      if (t < ny) jet_inlet(S, t + 1, k);
+      else jet_outlet(S, t - ny + 1, k);
+    }
+    __syncthreads();
+  }
+  if (k > 1 && k < nz) {
+    const int n = 2 * ny + 2 * (nx - 2);
+    for (int t = t0; t < n; t += nt) {
+      int i, j;
+      if (t < 2 * ny) { i = t < ny ? 1 : nx; j = (t < ny ? t : t - ny) + 1; }
+      else { const int r = t - 2 * ny; j = r < nx - 2 ? 1 : ny; i = (r < nx - 2 ? r : r - (nx - 2)) + 2; }
+      face_cell<MS>(S, i, j, k);
+    }
+  } else {
+    // a k face: the rows and columns that the conditions write or read (rows
+    // 1-3 and ny, columns 1-2 and nx-2..nx); the rest is k_bc's last blocks'
+    const int n = 4 * nx + 5 * (ny - 4);
+    for (int t = t0; t < n; t += nt) {
+      int i, j;
+      if (t < 4 * nx) { i = t % nx + 1; j = t / nx + 1; if (j == 4) j = ny; }
+      else { const int r = t - 4 * nx, a = r % 5; j = r / 5 + 4; i = a < 2 ? a + 1 : nx - 4 + a; }
+      face_cell<MS>(S, i, j, k);
+    }
+  }
+}
+
+// All of a stage's boundary conditions in one launch: a block per k plane,
+// then blocks over the middle of the two k faces.  It also opens with the
+// negative-Et repair of stage krk (0: none to do).  That is rare, and a cell
+// may lie beside a face: if stage krk counted any, the first block repairs
+// them and does all the rest by itself.
+// Few cells, many dependent loads: bound by latency and, as launches of their
+// own (reset, repair, inlet, upper, wall, outlet, faces), by the 4 to 5 us
+// that each takes from start to start.  us a stage, before / after: boundary
+// layer 161x61x33 31 / 15, round jet 48x36x36 59 / 32, periodic box 64^3
+// 17 / 8.
+constexpr int BC_NT = 512;
+__host__ __device__ inline long bc_mid_cells(const DevState& S) { return 2L * (S.nx - 5) * (S.ny - 4); }
+template <int BC, bool MS>
+__global__ __launch_bounds__(BC_NT) void k_bc(DevState S, int krk) {
+  const bool bad = krk > 0 && S.negt[18 + krk] != 0;
+  const long nmid = bc_mid_cells(S);
+  auto mid = [&](long t) {
+    const int mx = S.nx - 5, my = S.ny - 4;
+    face_cell<MS>(S, (int)(t % mx) + 3, (int)((t / mx) % my) + 4, t < (long)mx * my ? 1 : S.nz);
+  };
+  if (!bad) {
+    if (blockIdx.x < (unsigned)S.nz) {
+      bc_plane<BC, MS>(S, (int)blockIdx.x + 1);
+    } else {
+      const long t = (long)(blockIdx.x - S.nz) * blockDim.x + threadIdx.x;
+      if (t < nmid) mid(t);
+    }
+    return;
+  }
+  if (blockIdx.x != 0) return;
+  __shared__ int idx[16];
+  if (threadIdx.x == 0) negt_repair(S, krk, idx);
+  __syncthreads();
+  for (int k = 1; k <= S.nz; k++) {
+    bc_plane<BC, MS>(S, k);
+    __syncthreads();
+  }
+  for (long t = threadIdx.x; t < nmid; t += blockDim.x) mid(t);
 }
 
 // ===========================================================================
@@ -2527,9 +2604,10 @@ bool small_stage() {
          G.col_planes < 0 && G.sweep_variant[0] == 0 && G.sweep_variant[1] == 0 && G.sweep_variant[2] == 0;
 }
 
-void enq_small_sweeps() {
+void enq_small_sweeps(int krk) {
   const DevState& S = G.S;
   StageArgs A{};
+  A.first = krk == 1;
   long grid = 0;
   auto dir = [&](int d, int np, int ts, long npen) {
     A.gx[d] = (S.n[d] + ts - 1) / ts;
@@ -2584,21 +2662,16 @@ void enq_rhybrid() {
   launch("k_sensor_norm", k_sensor_norm, grid1(S.ni), dim3(256), S);
 }
 
-void enq_bc() {
+void enq_bc(int krk) {
   const DevState& S = G.S;
-  if (G.cfg.ibc == OCFD_BC_BOUNDARYLAYER) {
-    launch("k_bl_inlet", k_bl_inlet, grid1((long)S.ny * S.nz), dim3(256), S);
-    // BcData_upper = -1: no upper data; the face keeps its values
-    if (S.bl_upper >= 0) launch("k_bl_upper", k_bl_upper, grid1((long)S.nx * S.nz), dim3(256), S);
-    launch("k_bl_wall", k_bl_wall, grid1((long)S.nx * S.nz), dim3(256), S);
-    if (S.bl_outlet == 1 || S.bl_outlet == 2) launch("k_bl_outlet", k_bl_outlet, grid1((long)S.ny * S.nz), dim3(256), S);
-  } else if (G.cfg.ibc == OCFD_BC_JET) {
-    launch("k_jet_inlet", k_jet_inlet, grid1((long)S.ny * S.nz), dim3(256), S);
-    launch("k_jet_outlet", k_jet_outlet, grid1((long)S.ny * S.nz), dim3(256), S);
-  }
-  const long nxi = S.nx > 2 ? S.nx - 2 : 0, nyi = S.ny > 2 ? S.ny - 2 : 0;
-  const long nf = 2L * S.ny * S.nz + 2L * nxi * S.nz + 2L * nxi * nyi;
-  launch("k_bc_faces", k_bc_faces, grid1(nf), dim3(256), S);
+  const dim3 grid((unsigned)(S.nz + (bc_mid_cells(S) + BC_NT - 1) / BC_NT));
+  const bool ms = S.ns > 1;
+  if (G.cfg.ibc == OCFD_BC_BOUNDARYLAYER)
+    launch("k_bc", ms ? k_bc<OCFD_BC_BOUNDARYLAYER, true> : k_bc<OCFD_BC_BOUNDARYLAYER, false>, grid, dim3(BC_NT), S, krk);
+  else if (G.cfg.ibc == OCFD_BC_JET)
+    launch("k_bc", ms ? k_bc<OCFD_BC_JET, true> : k_bc<OCFD_BC_JET, false>, grid, dim3(BC_NT), S, krk);
+  else
+    launch("k_bc", ms ? k_bc<0, true> : k_bc<0, false>, grid, dim3(BC_NT), S, krk);
   for (int f = 0; f < 6; f++)  // Flow_Ghost_boundary, OCFD_BC.f90:186
     if (G.cfg.ghost_cell[f] == 1 || G.cfg.ghost_cell[f] == 2)
       launch("k_flow_ghost", k_flow_ghost, grid1(ghost_count(f)), dim3(256), S, f);
@@ -2616,13 +2689,11 @@ void enq_stage(int krk, double dt1) {
     else launch_s(vs, "k_transport", k_transport, grid1(S.ni), dim3(256), S);
   }
   if (krk == 1 && G.cfg.scheme_invis == OCFD_SCHEME_HYBRID) enq_rhybrid();
-  if (small) enq_small_sweeps();
+  if (small) enq_small_sweeps(krk);
   else enq_sweeps();
   join_side(vs);
-  launch("k_negt_reset", k_negt_reset, dim3(1), dim3(64), S, 0);
   launch_rk(krk, dt1, flags);
-  launch("k_negt_repair", k_negt_repair, dim3(1), dim3(64), S);
-  enq_bc();
+  enq_bc(krk);
 }
 
 template <int DIR>
@@ -2685,7 +2756,7 @@ void enq_species_one(int part, int m, int krk, double dt1) {
 // recovery with Rescaling_di, negative-Et repair, boundary conditions
 void enq_stage_ms(int krk, double dt1) {
   const DevState& S = G.S;
-  launch("k_transport_ms", k_transport_ms, grid1(S.ni), dim3(256), S);
+  launch("k_transport_ms", k_transport_ms, grid1(S.ni), dim3(256), S, krk == 1 ? 1 : 0);
   if (krk == 1 && G.cfg.scheme_invis == OCFD_SCHEME_HYBRID) enq_rhybrid();
   // the species chain (sweeps, concentrations, diffusion, update of di) on
   // the second stream beside the flow sweeps, which read no di; the flow's
@@ -2702,15 +2773,13 @@ void enq_stage_ms(int krk, double dt1) {
   }
   join_side(sp);
   const int flags = (S.mass_force ? RK_MASS : 0) | (S.viscous ? RK_VISC : 0) | RK_UPDATE_F | RK_PRIMS | RK_MS;
-  launch("k_negt_reset", k_negt_reset, dim3(1), dim3(64), S, 0);
   launch_rk(krk, dt1, flags);
-  launch("k_negt_repair", k_negt_repair, dim3(1), dim3(64), S);
-  enq_bc();
+  enq_bc(krk);
 }
 
 void enq_step(double dt1) {
   const DevState& S = G.S;
-  launch("k_negt_reset", k_negt_reset, dim3(1), dim3(64), S, 1);
+  if (S.ns == 1 && !small_stage()) launch("k_negt_reset", k_negt_reset, dim3(1), dim3(64), S, 1);
   for (int krk = 1; krk <= 3; krk++) {
     if (S.ns > 1) enq_stage_ms(krk, dt1);
     else enq_stage(krk, dt1);
@@ -3521,7 +3590,7 @@ int32_t ocfd_save_stage0(void) {
 }
 int32_t ocfd_comput_amu_amk(void) {
   if (check_ready()) return 1;
-  if (G.S.ns > 1) launch("k_transport_ms", k_transport_ms, grid1(G.S.ni), dim3(256), G.S);
+  if (G.S.ns > 1) launch("k_transport_ms", k_transport_ms, grid1(G.S.ni), dim3(256), G.S, 0);
   else launch("k_transport", k_transport, grid1(G.S.ni), dim3(256), G.S);
   HIPCHK(hipGetLastError());
   return 0;
@@ -3529,7 +3598,7 @@ int32_t ocfd_comput_amu_amk(void) {
 int32_t ocfd_stage_begin(int32_t krk) {
   if (check_ready()) return 1;
   if (G.S.ns > 1) {
-    launch("k_transport_ms", k_transport_ms, grid1(G.S.ni), dim3(256), G.S);
+    launch("k_transport_ms", k_transport_ms, grid1(G.S.ni), dim3(256), G.S, 0);
   } else {
     launch("k_transport", k_transport, grid1(G.S.ni), dim3(256), G.S);
     launch("k_di_from_d", k_di_from_d, grid1(G.S.nh), dim3(256), G.S);
@@ -3659,7 +3728,7 @@ int32_t ocfd_filtering(int32_t istep, int32_t nfiltering, const double* filter) 
 
 int32_t ocfd_bc(void) {
   if (check_ready()) return 1;
-  enq_bc();
+  enq_bc(0);
   HIPCHK(hipGetLastError());
   return 0;
 }

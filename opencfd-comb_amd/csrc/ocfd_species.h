@@ -181,8 +181,10 @@ __device__ __forceinline__ void cell_ijk(const DevState& S, long c, int& i, int&
 // comput_vis_coeff (TRANSPORT_modules.f90:259-306), comput_Cp,
 // comput_thermal_conductivity (:312-372), comput_diffusion_coeff (:378-424).
 // ===========================================================================
-__global__ __launch_bounds__(256, 5) void k_transport_ms(DevState S) {
+// first: the launch opens a step and resets the negative-Et counters
+__global__ __launch_bounds__(256, 5) void k_transport_ms(DevState S, int first) {
   const long c = cell_index();
+  if (first && blockIdx.x == 0 && threadIdx.x == 0) negt_reset(S, 1);
   if (c >= S.ni) return;
   int i, j, k;
   cell_ijk(S, c, i, j, k);
@@ -615,11 +617,8 @@ __device__ __forceinline__ void face_update_ms(const DevState& S, long q, long c
 
 // ocfd_bc_jet inflow (OCFD_BC_jet.f90:22-73): Dirichlet data, or (BC_Para(1)=1)
 // the pressure of i=2 where the inflow is subsonic
-__global__ void k_jet_inlet(DevState S) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)S.ny * S.nz) return;
-  const int j = (int)(t % S.ny) + 1, k = (int)(t / S.ny) + 1;
-  const long q = hq(S, 1, j, k), pl = (long)S.ny * S.nz, r = t;
+__device__ __forceinline__ void jet_inlet(const DevState& S, int j, int k) {
+  const long q = hq(S, 1, j, k), pl = (long)S.ny * S.nz, r = (j - 1) + (long)S.ny * (k - 1);
   const double* in = S.jet_in;
   const int ns = S.ns;
   if (S.jet_iflag == 0) {
@@ -653,10 +652,7 @@ __global__ void k_jet_inlet(DevState S) {
 }
 
 // ocfd_bc_jet outflow (OCFD_BC_jet.f90:76-93): zeroth-order extrapolation
-__global__ void k_jet_outlet(DevState S) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)S.ny * S.nz) return;
-  const int j = (int)(t % S.ny) + 1, k = (int)(t / S.ny) + 1;
+__device__ __forceinline__ void jet_outlet(const DevState& S, int j, int k) {
   const long q = hq(S, S.nx, j, k), qa = hq(S, S.nx - 1, j, k);
   S.d[q] = S.d[qa]; S.u[q] = S.u[qa]; S.v[q] = S.v[qa]; S.w[q] = S.w[qa];
   S.T[q] = S.T[qa]; S.p[q] = S.p[qa]; S.Et[q] = S.Et[qa];
