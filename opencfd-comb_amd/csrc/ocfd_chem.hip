@@ -1011,11 +1011,7 @@ int32_t ocfd_chem_set_mechanism(int32_t ns, int32_t nr, int32_t rereac, const in
       for (int a = 0; a < 7; a++) h.gb[k][j][a] = gb[a];
     }
   }
-  for (int j = 0; j < 64; j++) {
-    const long double v = std::exp2((long double)j / 64.0L);
-    h.exp2t[j][0] = (double)v;
-    h.exp2t[j][1] = (double)(v - (long double)h.exp2t[j][0]);
-  }
+  chem_exp_table(h.exp2t);
   CX.h2 = rereac == 0 && nr == ChemH2::NR && n_tct == ChemH2::NT;
   for (int j = 0; CX.h2 && j < nr; j++) {
     const ChemRx& R = h.rx[j];

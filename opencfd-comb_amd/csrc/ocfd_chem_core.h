@@ -28,6 +28,8 @@
 #include <type_traits>
 #include <utility>
 
+#include "ocfd_exp.h"
+
 #define CH_NS 9
 #define CH_NR_MAX 32
 #define CH_NT_MAX 4
@@ -89,27 +91,6 @@ __device__ __forceinline__ double fm(double a, double b, double c) { return __bu
 __device__ __forceinline__ double div_r(double a, double b, double r) {
   const double q = a * r;
   return fm(fm(-b, q, a), r, q);
-}
-
-// exp(x) = 2^e T[j] (1 + p(f)), x = (64 e + j) ln2/64 + f, |f| <= ln2/128: a
-// table of 2^(j/64) in LDS (head and tail) and the Taylor polynomial of
-// e^f - 1 to degree 5 (remainder below 2^-54).  About 17 vector instructions;
-// the library's exp takes 60 to 70 here, half of them moves of its
-// polynomial's constants.  Largest error on |x| <= 700 (4e6 points against
-// 80-bit exp): 0.82 ulp.
-constexpr int CH_EXPN = 64;
-__device__ __forceinline__ double chem_exp(const double2* tab, double x) {
-  const double n = __builtin_rint(x * 92.332482616893656877);  // 64 / ln 2
-  // ln2 / 64 as a 32-bit head (its products with n are exact) and a tail
-  double f = fm(-n, 0x1.62e42fefp-7, x);
-  f = fm(-n, 0x1.473de6af278edp-40, f);
-  const int k = (int)n;
-  const double2 t = tab[k & (CH_EXPN - 1)];
-  double p = fm(f, 1.0 / 120.0, 1.0 / 24.0);
-  p = fm(f, p, 1.0 / 6.0);
-  p = fm(f, p, 0.5);
-  p = fm(f * f, p, f);
-  return __builtin_amdgcn_ldexp(t.x + fm(t.x, p, t.y), k >> 6);
 }
 
 // Fortran x**n for an integer n (repeated squaring; negative n -> 1/x**|n|)

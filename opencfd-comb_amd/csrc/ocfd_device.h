@@ -163,6 +163,20 @@ __device__ __forceinline__ double jac_at(const DevState& S, long q, int i, int j
                 xi1 * zj1 * yk1);
 }
 
+// The kernel's first argument again, out of the argument segment by a pointer
+// that the compiler cannot see through.  DevState has some 90 pointers; a
+// kernel with several branches that each use many of them has all the loads
+// hoisted to its entry otherwise, far more than the scalar registers hold, and
+// then moves them through vector lanes at every use (k_stage: 7,000 of its
+// 26,000 instructions).
+template <class T = DevState>
+__device__ __forceinline__ const T& kernarg_again() {
+  typedef const __attribute__((address_space(4))) T* Arg;
+  Arg p = (Arg)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const T*)p;
+}
+
 // XCD-aware block order.  The hardware hands workgroup b to XCD b % 8; each
 // XCD has its own L2.  Remapping so that XCD x works on one contiguous range
 // of logical blocks keeps the stencil neighbours (k +- 3 planes) of a block in

@@ -898,8 +898,7 @@ __global__ __launch_bounds__(256) void k_visc_prep(DevState S) {
 // blocks each, every launch of its own costs its ramp, its last half-empty
 // round and 2 to 4 us between launches (with the preparation on a second
 // stream 10 us a stage for the fork and join): 32^3 box, us per RK3 step, 264
-// with one launch each, 192 without the second stream, 151 in this form (27
-// us of each stage's 50 are this launch).  A large grid keeps its launches:
+// with one launch each, 192 without the second stream, 151 in this form.  A large grid keeps its launches:
 // its update is bound by memory and would read 80 B a cell more (640x120x64:
 // 5.95 against 5.51 ms per step).
 struct StageArgs {
@@ -910,7 +909,7 @@ struct StageArgs {
   int* kct[3];
 };
 template <int CD, bool MT>
-__global__ __launch_bounds__(256) void k_stage(DevState S, StageArgs A) {
+__global__ __launch_bounds__(256) void k_stage(DevState S0, StageArgs A) {
   __shared__ union Lds {
     SweepLds<0, 0> x;
     SweepLds<1, 0> y;
@@ -919,18 +918,18 @@ __global__ __launch_bounds__(256) void k_stage(DevState S, StageArgs A) {
   } U;
   const long p0 = (A.nb[0] + 7) & ~7L, p1 = p0 + ((A.nb[1] + 7) & ~7L), p2 = p1 + ((A.nb[2] + 7) & ~7L);
   const long b = (long)blockIdx.x;
-  if (A.first && b == 0 && threadIdx.x == 0) negt_reset(S, 1);
+  if (A.first && b == 0 && threadIdx.x == 0) negt_reset(S0, 1);
   if (b < p0) {
     if (b < A.nb[0])
-      sweep_tile<0, 0, false>(S, U.x, xcd_block(b, A.nb[0]), A.gx[0], A.mode[0], A.kc[0], A.kct[0], S.du);
+      sweep_tile<0, 0, false>(kernarg_again(), U.x, xcd_block(b, A.nb[0]), A.gx[0], A.mode[0], A.kc[0], A.kct[0], kernarg_again().du);
   } else if (b < p1) {
     if (b - p0 < A.nb[1])
-      sweep_tile<1, 0, false>(S, U.y, xcd_block(b - p0, A.nb[1]), A.gx[1], A.mode[1], A.kc[1], A.kct[1], S.duy);
+      sweep_tile<1, 0, false>(kernarg_again(), U.y, xcd_block(b - p0, A.nb[1]), A.gx[1], A.mode[1], A.kc[1], A.kct[1], kernarg_again().duy);
   } else if (b < p2) {
     if (b - p1 < A.nb[2])
-      sweep_tile<2, 0, false>(S, U.z, xcd_block(b - p1, A.nb[2]), A.gx[2], A.mode[2], A.kc[2], A.kct[2], S.duz);
+      sweep_tile<2, 0, false>(kernarg_again(), U.z, xcd_block(b - p1, A.nb[2]), A.gx[2], A.mode[2], A.kc[2], A.kct[2], kernarg_again().duz);
   } else {
-    visc_prep_at<CD, false, MT>(S, xcd_block(b - p2, (long)gridDim.x - p2) * blockDim.x + threadIdx.x);
+    visc_prep_at<CD, false, MT>(kernarg_again(), xcd_block(b - p2, (long)gridDim.x - p2) * blockDim.x + threadIdx.x);
   }
 }
 
@@ -1043,12 +1042,12 @@ __global__ __launch_bounds__(256) void k_visc_prep_col(DevState S, int kc) {
       }
       const YTaps yt{ys[b], lane, wv};
       if (xint && yint)
-        visc_prep_cell<CD, MS, true, true, MT>(S, c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr, &xt, &yt);
+        visc_prep_cell<CD, MS, true, true, MT>(kernarg_again(), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr, &xt, &yt);
       else if (yint)
-        visc_prep_cell<CD, MS, false, true, MT>(S, c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr,
+        visc_prep_cell<CD, MS, false, true, MT>(kernarg_again(), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr,
                                                 (const XTaps*)nullptr, &yt);
       else
-        visc_prep_cell<CD, MS, false, false, MT>(S, c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr);
+        visc_prep_cell<CD, MS, false, false, MT>(kernarg_again(), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr);
     }
 #pragma unroll
     for (int o = 0; o < W - 1; o++) {
@@ -1208,7 +1207,7 @@ __device__ __forceinline__ void rk_cell(const DevState& S, long c, long q, int i
       if (save0) {
 #pragma unroll
         for (int m = 0; m < 5; m++) S.fn[c + m * ni] = fnv[m];
-        S.din[c] = S.di[q];
+        if (!(flags & RK_MS)) S.din[c] = S.di[q];  // (N_SPEC > 1: k_species_rk's)
       }
     } else {
       const double ra = krk == 2 ? 3.0 / 4.0 : 1.0 / 3.0;
@@ -1283,7 +1282,7 @@ __global__ __launch_bounds__(256) void k_rk(DevState S, int krk, double dt, int 
         zs[m] = deriv1<CD, true>(S, 2, k, [&](int o) { return Fv[4 * o * pli]; });
       }
     }
-    rk_cell<CD, F, true, true, MT>(S, c, q, i, j, k, krk, dt, flags_rt, zs);
+    rk_cell<CD, F, true, true, MT>(kernarg_again(), c, q, i, j, k, krk, dt, flags_rt, zs);
   } else {
     if (flags & RK_VISC) {
 #pragma unroll
@@ -1295,7 +1294,7 @@ __global__ __launch_bounds__(256) void k_rk(DevState S, int krk, double dt, int 
         });
       }
     }
-    rk_cell<CD, F, false, false, MT>(S, c, q, i, j, k, krk, dt, flags_rt, zs);
+    rk_cell<CD, F, false, false, MT>(kernarg_again(), c, q, i, j, k, krk, dt, flags_rt, zs);
   }
 }
 
@@ -1348,17 +1347,17 @@ __global__ __launch_bounds__(256, (CD == 0 && F >= 0 && !(F & RK_MS)) ? 2 : 1) v
 #pragma unroll
         for (int m = 0; m < 4; m++) zs[m] = visc ? deriv1<CD>(S, 2, k, [&](int o) { return z[m][o + R]; }) : 0.0;
       }
-      if (xint && yint) rk_cell<CD, F, true, true, MT>(S, c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
-      else if (yint) rk_cell<CD, F, false, true, MT>(S, c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
-      else rk_cell<CD, F, false, false, MT>(S, c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      if (xint && yint) rk_cell<CD, F, true, true, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      else if (yint) rk_cell<CD, F, false, true, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      else rk_cell<CD, F, false, false, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
     } else if (xint && yint && central_cell(k, S.nz, R)) {
 #pragma unroll
       for (int m = 0; m < 4; m++) zs[m] = visc ? deriv1<CD, true>(S, 2, k, [&](int o) { return z[m][o + R]; }) : 0.0;
-      rk_cell<CD, F, true, true, MT>(S, c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      rk_cell<CD, F, true, true, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
     } else {
 #pragma unroll
       for (int m = 0; m < 4; m++) zs[m] = visc ? deriv1<CD>(S, 2, k, [&](int o) { return z[m][o + R]; }) : 0.0;
-      rk_cell<CD, F, false, false, MT>(S, c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      rk_cell<CD, F, false, false, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
     }
 #pragma unroll
     for (int o = 0; o < W - 1; o++)
@@ -1382,6 +1381,7 @@ __global__ void k_negt_reset(DevState S, int step) {
 // reference's (k,j,i) order by one thread: a neighbour already visited by
 // the reference loop holds its new Et, a later one (and every ghost) its old.
 // idx: 16 entries of LDS
+template <bool MS>
 __device__ __forceinline__ void negt_repair(const DevState& S, int krk, int* idx) {
   const int cnt = S.negt[18 + krk];
   if (cnt > S.negt[17]) S.negt[17] = cnt;
@@ -1393,6 +1393,7 @@ __device__ __forceinline__ void negt_repair(const DevState& S, int krk, int* idx
     while (b >= 0 && idx[b] > x) { idx[b + 1] = idx[b]; b--; }
     idx[b + 1] = x;
   }
+#pragma unroll 1
   for (int a = 0; a < n; a++) {
     const long c = idx[a];
     const int i = (int)(c % S.nx) + 1;
@@ -1410,11 +1411,17 @@ __device__ __forceinline__ void negt_repair(const DevState& S, int krk, int* idx
       return img ? S.Et_prev[iq(S, wi, wj, wk)] : S.Et[hq(S, ii, jj, kk)];
     };
     const double Et0 = S.Et[q];
-    const double En = (nb(i + 1, j, k) + nb(i - 1, j, k) + nb(i, j + 1, k) + nb(i, j - 1, k) + nb(i, j, k + 1) +
-                       nb(i, j, k - 1)) / 6.0;
+    double En = 0.0;
+#pragma unroll 1
+    for (int d = 0; d < 6; d++) {  // i + 1, i - 1, j + 1, ...
+      const int o = d & 1 ? -1 : 1, dir = d >> 1;
+      const double e = nb(i + (dir == 0 ? o : 0), j + (dir == 1 ? o : 0), k + (dir == 2 ? o : 0));
+      En = d == 0 ? e : En + e;
+    }
+    En = En / 6.0;
     S.Et[q] = En;
     S.f[c + 4 * S.ni] = S.f[c + 4 * S.ni] + (En - Et0);
-    if (S.ns > 1) {
+    if (MS) {
       double dim[OCFD_NS_MAX];
       for (int m = 0; m < S.ns; m++) dim[m] = S.di[q + (long)m * S.nh];
       const double T = gas_T(dim, En);
@@ -1428,9 +1435,10 @@ __device__ __forceinline__ void negt_repair(const DevState& S, int krk, int* idx
     S.p[q] = 0.0 + S.Ri0 * di * T;
   }
 }
+template <bool MS>
 __global__ void k_negt_repair(DevState S) {  // after comput_flow_variables
   __shared__ int idx[16];
-  if (threadIdx.x == 0 && blockIdx.x == 0) negt_repair(S, 1, idx);
+  if (threadIdx.x == 0 && blockIdx.x == 0) negt_repair<MS>(S, 1, idx);
 }
 
 // ===========================================================================
@@ -1533,60 +1541,55 @@ __device__ __forceinline__ void face_update(const DevState& S, long q, long c) {
   S.f[c + 4 * S.ni] = Et + dd * (uu * uu + vv * vv + ww * ww) * 0.5;
 }
 
+constexpr int BC_NT = 512;  // threads of k_bc
 template <bool MS>
 __device__ __forceinline__ void face_cell(const DevState& S, int i, int j, int k) {
   const long q = hq(S, i, j, k), c = iq(S, i, j, k);
   const int nf = (i == 1) + (i == S.nx) + (j == 1) + (j == S.ny) + (k == 1) + (k == S.nz);
+#pragma unroll 1
   for (int a = 0; a < nf; a++) {
     if (MS) face_update_ms(S, q, c);
     else face_update(S, q, c);
   }
 }
 
-// One k plane: the conditions of the i and j faces in the reference's order,
-// then the faces' conserved variables.  The conditions read and write cells
-// of their own plane only, so a block does them with barriers in between.
-template <int BC, bool MS>
-__device__ void bc_plane(const DevState& S, int k) {
-  const int nx = S.nx, ny = S.ny, nz = S.nz, t0 = (int)threadIdx.x, nt = (int)blockDim.x;
+// The conditions of the i and j faces in one k plane, in the reference's
+// order.  They read and write cells of their own plane only, so a block does
+// them with barriers in between.
+template <int BC>
+__device__ __forceinline__ void bc_conditions(int k) {
+  const int t0 = (int)threadIdx.x;
   if (BC == OCFD_BC_BOUNDARYLAYER) {
-    for (int t = t0; t < ny; t += nt) bl_inlet(S, t + 1, k);
-    __syncthreads();
-    // BcData_upper = -1: no upper data; the face keeps its values.  The wall
-    // reads rows 2 and 3, which the upper data (row ny >= 8) do not touch.
-    for (int t = t0; t < 2 * nx; t += nt) {
-      if (t >= nx) bl_wall(S, t - nx + 1, k);
-      else if (S.bl_upper >= 0) bl_upper(S, t + 1, k);
+    {
+      const DevState& S = kernarg_again();
+      for (int t = t0; t < S.ny; t += BC_NT) bl_inlet(S, t + 1, k);
     }
     __syncthreads();
-    if (S.bl_outlet == 1 || S.bl_outlet == 2)
-      for (int t = t0; t < ny; t += nt) bl_outlet(S, t + 1, k);
+    {
+      // BcData_upper = -1: no upper data; the face keeps its values.  The wall
+      // reads rows 2 and 3, which the upper data (row ny >= 8) do not touch.
+      const DevState& S = kernarg_again();
+      const int nx = S.nx;
+      for (int t = t0; t < 2 * nx; t += BC_NT) {
+        if (t >= nx) bl_wall(S, t - nx + 1, k);
+        else if (S.bl_upper >= 0) bl_upper(S, t + 1, k);
+      }
+    }
+    __syncthreads();
+    {
+      const DevState& S = kernarg_again();
+      if (S.bl_outlet == 1 || S.bl_outlet == 2)
+        for (int t = t0; t < S.ny; t += BC_NT) bl_outlet(S, t + 1, k);
+    }
     __syncthreads();
   } else if (BC == OCFD_BC_JET) {
-    for (int t = t0; t < 2 * ny; t += nt) {
+    const DevState& S = kernarg_again();
+    const int ny = S.ny;
+    for (int t = t0; t < 2 * ny; t += BC_NT) {
       if (t < ny) jet_inlet(S, t + 1, k);
       else jet_outlet(S, t - ny + 1, k);
     }
     __syncthreads();
-  }
-  if (k > 1 && k < nz) {
-    const int n = 2 * ny + 2 * (nx - 2);
-    for (int t = t0; t < n; t += nt) {
-      int i, j;
-      if (t < 2 * ny) { i = t < ny ? 1 : nx; j = (t < ny ? t : t - ny) + 1; }
-      else { const int r = t - 2 * ny; j = r < nx - 2 ? 1 : ny; i = (r < nx - 2 ? r : r - (nx - 2)) + 2; }
-      face_cell<MS>(S, i, j, k);
-    }
-  } else {
-    // a k face: the rows and columns that the conditions write or read (rows
-    // 1-3 and ny, columns 1-2 and nx-2..nx); the rest is k_bc's last blocks'
-    const int n = 4 * nx + 5 * (ny - 4);
-    for (int t = t0; t < n; t += nt) {
-      int i, j;
-      if (t < 4 * nx) { i = t % nx + 1; j = t / nx + 1; if (j == 4) j = ny; }
-      else { const int r = t - 4 * nx, a = r % 5; j = r / 5 + 4; i = a < 2 ? a + 1 : nx - 4 + a; }
-      face_cell<MS>(S, i, j, k);
-    }
   }
 }
 
@@ -1598,36 +1601,58 @@ __device__ void bc_plane(const DevState& S, int k) {
 // Few cells, many dependent loads: bound by latency and, as launches of their
 // own (reset, repair, inlet, upper, wall, outlet, faces), by the 4 to 5 us
 // that each takes from start to start.  us a stage, before / after: boundary
-// layer 161x61x33 31 / 15, round jet 48x36x36 59 / 32, periodic box 64^3
-// 17 / 8.
-constexpr int BC_NT = 512;
+// layer 161x61x33 31 / 15, round jet 48x36x36 59 / 24, periodic box 32^3
+// 17 / 5.
 __host__ __device__ inline long bc_mid_cells(const DevState& S) { return 2L * (S.nx - 5) * (S.ny - 4); }
 template <int BC, bool MS>
 __global__ __launch_bounds__(BC_NT) void k_bc(DevState S, int krk) {
-  const bool bad = krk > 0 && S.negt[18 + krk] != 0;
-  const long nmid = bc_mid_cells(S);
-  auto mid = [&](long t) {
-    const int mx = S.nx - 5, my = S.ny - 4;
-    face_cell<MS>(S, (int)(t % mx) + 3, (int)((t / mx) % my) + 4, t < (long)mx * my ? 1 : S.nz);
-  };
-  if (!bad) {
-    if (blockIdx.x < (unsigned)S.nz) {
-      bc_plane<BC, MS>(S, (int)blockIdx.x + 1);
-    } else {
-      const long t = (long)(blockIdx.x - S.nz) * blockDim.x + threadIdx.x;
-      if (t < nmid) mid(t);
-    }
-    return;
-  }
-  if (blockIdx.x != 0) return;
   __shared__ int idx[16];
-  if (threadIdx.x == 0) negt_repair(S, krk, idx);
-  __syncthreads();
-  for (int k = 1; k <= S.nz; k++) {
-    bc_plane<BC, MS>(S, k);
+  const int nx = S.nx, ny = S.ny, nz = S.nz;
+  const int mx = nx - 5, my = ny - 4;  // the middle of a k face
+  const bool bad = krk > 0 && S.negt[18 + krk] != 0;
+  if (bad) {
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x == 0) negt_repair<MS>(kernarg_again(), krk, idx);
     __syncthreads();
   }
-  for (long t = threadIdx.x; t < nmid; t += blockDim.x) mid(t);
+  const int b1 = bad ? (int)gridDim.x : (int)blockIdx.x + 1;
+#pragma unroll 1
+  for (int b = (int)blockIdx.x; b < b1; b++) {
+    const int k = b + 1;  // the plane of a block below nz
+    const bool mid = b >= nz, kface = k == 1 || k == nz;
+    const long m0 = (long)(b - nz) * BC_NT;
+    long n;
+    if (!mid) {
+      bc_conditions<BC>(k);
+      // a k face: the rows and columns that the conditions write or read (rows
+      // 1-3 and ny, columns 1-2 and nx-2..nx); the last blocks do the rest
+      n = kface ? 4 * nx + 5 * (ny - 4) : 2 * ny + 2 * (nx - 2);
+    } else {
+      n = min((long)BC_NT, 2L * mx * my - m0);
+    }
+#pragma unroll 1
+    for (int t = (int)threadIdx.x; t < n; t += BC_NT) {
+      int i, j, kk = k;
+      if (mid) {
+        const long c = m0 + t, l = c / mx;
+        i = (int)(c - l * mx) + 3;
+        kk = l < my ? 1 : nz;
+        j = (int)(l < my ? l : l - my) + 4;
+      } else if (kface) {
+        if (t < 4 * nx) { i = t % nx + 1; j = t / nx + 1; if (j == 4) j = ny; }
+        else { const int r = t - 4 * nx, a = r % 5; j = r / 5 + 4; i = a < 2 ? a + 1 : nx - 4 + a; }
+      } else if (t < 2 * ny) {
+        i = t < ny ? 1 : nx;
+        j = (t < ny ? t : t - ny) + 1;
+      } else {
+        const int r = t - 2 * ny;
+        j = r < nx - 2 ? 1 : ny;
+        i = (r < nx - 2 ? r : r - (nx - 2)) + 2;
+      }
+      face_cell<MS>(kernarg_again(), i, j, kk);
+    }
+    if (bad) __syncthreads();
+  }
 }
 
 // ===========================================================================
@@ -2466,7 +2491,7 @@ void launch_rk_f(int krk, double dt, int flags) {
 template <int CD>
 void launch_rk_cd(int krk, double dt, int flags) {
   constexpr int STEP1 = RK_SAVE0 | RK_VISC | RK_UPDATE_F | RK_PRIMS | RK_DI_FROM_D;
-  constexpr int STEPMS = RK_VISC | RK_UPDATE_F | RK_PRIMS | RK_MS;
+  constexpr int STEPMS = RK_SAVE0 | RK_VISC | RK_UPDATE_F | RK_PRIMS | RK_MS;
   if (flags & RK_DU3) {  // small grids: one thread per cell
     constexpr int STEPS = STEP1 | RK_DU3;
     const DevState& S = G.S;
@@ -2595,7 +2620,8 @@ void enq_sweeps() {
 // RK3 step, k_stage / separate launches, on periodic boxes: 48^3 253 / 348,
 // 64^3 504 / 535, 80^3 946 / 976, 88^3 1201 / 1184, 96^3 1473 / 1412; on
 // plates: 161x61x33 605 / 678, 200x61x40 844 / 900, 240x81x33 (642,000
-// cells) 1163 / 1165, 320x80x33 1443 / 1365.  Above the line the update's
+// cells) 1163 / 1165, 320x80x33 1443 / 1365 (before kernarg_again took a
+// tenth off the first).  Above the line the update's
 // 80 B a cell more outweigh the ramps and gaps saved.  Only the default tiles
 // have a form in k_stage, and a timed run shows the kernels one by one.
 constexpr long SMALL_CELLS = 1L << 19;
@@ -2696,34 +2722,67 @@ void enq_stage(int krk, double dt1) {
   enq_bc(krk);
 }
 
+// Blocks that share the species of a cell or tile, where `blocks` blocks of
+// four wavefronts would do all of them: the species follow one another
+// otherwise, and a small grid has too few wavefronts to cover their latency.
+// Every share repeats the work on the point itself (metrics, masks, split
+// velocity), so a large grid takes one.  us per RK3 step with 1 / 2 / 3
+// shares, jets: 48x36x36 (243 blocks of cells) 812 / 642 / 615, 64x48x40 (480)
+// 950 / 851 / 888, 80x56x48 (840) 1415 / 1332 / 1348, 96x64x56 (1344) 1941 /
+// 1940 / 1975, 160x112x64 (4480) 5397 / 5407 / 5535.
+int species_groups(long blocks, int nm) { return blocks >= 1344 ? 1 : std::min(nm, blocks >= 400 ? 2 : 3); }
+
 template <int DIR>
 void launch_species_sweep(hipStream_t st, int m0, int m1) {
   const DevState& S = G.S;
   constexpr int NP = SpTile<DIR>::NP, TS = SpTile<DIR>::TS;
   const long npen = DIR == 0 ? (long)S.ny * S.nz : DIR == 1 ? (long)S.nx * S.nz : (long)S.nx * S.ny;
   dim3 g((unsigned)((S.n[DIR] + TS - 1) / TS), (unsigned)((npen + NP - 1) / NP));
+  const int ns = species_groups((long)g.x * g.y, m1 - m0), ng = (m1 - m0 + ns - 1) / ns;
+  g.z = (unsigned)((m1 - m0 + ng - 1) / ng);
   static const char* names[3] = {"k_species_sweep_x", "k_species_sweep_y", "k_species_sweep_z"};
-  launch_s(st, names[DIR], k_species_sweep<DIR>, g, dim3(256), S, m0, m1);
+  launch_s(st, names[DIR], k_species_sweep<DIR>, g, dim3(256), S, m0, m1, ng);
+}
+
+// first: reset the negative-Et counters; conc: also the concentrations
+void launch_transport_ms(int first, int conc) {
+  const DevState& S = G.S;
+  launch("k_transport_ms", S.ns == OCFD_NS_MAX ? k_transport_ms<true> : k_transport_ms<false>, grid1(S.ni), dim3(256),
+         S, first, conc);
+}
+
+void launch_species_rk(hipStream_t st, int krk, double dt, int visc, int save, int m0, int m1) {
+  const DevState& S = G.S;
+  dim3 g = grid1(S.ni);
+  const int ns = species_groups(g.x, m1 - m0), ng = (m1 - m0 + ns - 1) / ns;
+  g.y = (unsigned)((m1 - m0 + ng - 1) / ng);
+  launch_s(st, "k_species_rk", S.cd8 ? k_species_rk<1> : k_species_rk<0>, g, dim3(256), S, krk, dt, visc, save, m0, m1,
+           ng);
 }
 
 // species right-hand sides (krk = 0: leave them in dus) or the species RK3
 // stage (OCFD_Time_Adv.f90:64-71)
 // on stream st (default: the library stream); after_prep, if given, is
-// recorded once Qp (species viscous preparation) is written
-void enq_species(int krk, double dt1, hipStream_t st = nullptr, hipEvent_t after_prep = nullptr) {
+// recorded once Qp (species viscous preparation) is written.  step: a stage
+// of a step, which has the concentrations from the transport coefficients'
+// kernel and whose first one keeps din.
+void enq_species(int krk, double dt1, hipStream_t st = nullptr, hipEvent_t after_prep = nullptr, bool step = false) {
   const DevState& S = G.S;
   if (!st) st = G.stream;
   launch_species_sweep<0>(st, 0, S.ns);
   launch_species_sweep<1>(st, 0, S.ns);
   launch_species_sweep<2>(st, 0, S.ns);
   if (S.viscous) {
-    launch_s(st, "k_species_conc", k_species_conc, grid1(S.ni), dim3(256), S, 0, S.ns);
-    launch_s(st, "k_species_visc_prep", S.cd8 ? k_species_visc_prep<1> : k_species_visc_prep<0>, grid1(S.ni),
-             dim3(256), S, 0, S.ns);
+    if (!step) launch_s(st, "k_species_conc", k_species_conc, grid1(S.ni), dim3(256), S, 0, S.ns);
+    if (species_groups(grid1(S.ni).x, S.ns) > 1)
+      launch_s(st, "k_species_visc_prep", S.cd8 ? k_species_visc_prep3<1> : k_species_visc_prep3<0>,
+               dim3((unsigned)((S.ni + 63) / 64)), dim3(192), S);
+    else
+      launch_s(st, "k_species_visc_prep", S.cd8 ? k_species_visc_prep<1> : k_species_visc_prep<0>, grid1(S.ni),
+               dim3(256), S, 0, S.ns);
   }
   if (after_prep) hipEventRecord(after_prep, st);
-  launch_s(st, "k_species_rk", S.cd8 ? k_species_rk<1> : k_species_rk<0>, grid1(S.ni), dim3(256), S, krk, dt1,
-           S.viscous, 0, S.ns);
+  launch_species_rk(st, krk, dt1, S.viscous, step && krk == 1, 0, S.ns);
 }
 
 // One species m (0-based) of the reference's species loop
@@ -2743,11 +2802,9 @@ void enq_species_one(int part, int m, int krk, double dt1) {
     launch_s(st, "k_species_conc", k_species_conc, grid1(S.ni), dim3(256), S, m, m + 1);
     launch_s(st, "k_species_visc_prep", S.cd8 ? k_species_visc_prep<1> : k_species_visc_prep<0>, grid1(S.ni),
              dim3(256), S, m, m + 1);
-    launch_s(st, "k_species_rk", S.cd8 ? k_species_rk<1> : k_species_rk<0>, grid1(S.ni), dim3(256), S, 0, 0.0, 1,
-             m, m + 1);
+    launch_species_rk(st, 0, 0.0, 1, 0, m, m + 1);
   } else {
-    launch_s(st, "k_species_rk", S.cd8 ? k_species_rk<1> : k_species_rk<0>, grid1(S.ni), dim3(256), S, krk, dt1, 0,
-             m, m + 1);
+    launch_species_rk(st, krk, dt1, 0, 0, m, m + 1);
   }
 }
 
@@ -2756,23 +2813,20 @@ void enq_species_one(int part, int m, int krk, double dt1) {
 // recovery with Rescaling_di, negative-Et repair, boundary conditions
 void enq_stage_ms(int krk, double dt1) {
   const DevState& S = G.S;
-  launch("k_transport_ms", k_transport_ms, grid1(S.ni), dim3(256), S, krk == 1 ? 1 : 0);
+  launch_transport_ms(krk == 1 ? 1 : 0, S.viscous);
   if (krk == 1 && G.cfg.scheme_invis == OCFD_SCHEME_HYBRID) enq_rhybrid();
   // the species chain (sweeps, concentrations, diffusion, update of di) on
   // the second stream beside the flow sweeps, which read no di; the flow's
   // viscous preparation waits for Qp, k_rk (Rescaling_di) for the whole chain
   const hipStream_t sp = fork_side();
-  // the step's saved solution: din is first read by the species update on
-  // the second stream, fn by k_rk after the join
-  if (krk == 1) launch_s(sp, "k_save0", k_save0, grid1(S.ni), dim3(256), S);
-  enq_species(krk, dt1, sp, sp != G.stream ? G.ev_qp : nullptr);
+  enq_species(krk, dt1, sp, sp != G.stream ? G.ev_qp : nullptr, true);
   enq_sweeps();
   if (S.viscous) {
     if (sp != G.stream) hipStreamWaitEvent(G.stream, G.ev_qp, 0);
     launch_visc_prep(true);
   }
   join_side(sp);
-  const int flags = (S.mass_force ? RK_MASS : 0) | (S.viscous ? RK_VISC : 0) | RK_UPDATE_F | RK_PRIMS | RK_MS;
+  const int flags = (S.mass_force ? RK_MASS : 0) | (S.viscous ? RK_VISC : 0) | RK_SAVE0 | RK_UPDATE_F | RK_PRIMS | RK_MS;
   launch_rk(krk, dt1, flags);
   enq_bc(krk);
 }
@@ -3199,6 +3253,15 @@ int32_t ocfd_set_species(int32_t n_tct, const double* tct, double tct_max, const
                         h.ect[k][j];
     }
   }
+  for (int j = 0; j < GAS_NT_MAX; j++)
+    for (int k = 0; k < ns; k++) {
+      const bool on = j < h.n_tct;
+      h.ev[j][0][k] = on ? (h.coef[k][j][0] - 1.0) * h.Ri[k] : 0.0;
+      for (int a = 1; a < 5; a++) h.ev[j][a][k] = on ? h.coef[k][j][a] * h.Ri[k] : 0.0;
+      h.ev[j][5][k] = on ? h.ect[k][j] * h.Ri[k] : 0.0;
+    }
+  for (int k = 0; k < ns; k++) h.rcv[k] = 2.5 * h.Ri[k];
+  chem_exp_table(h.exp2t);
   return upload_gas();
 }
 
@@ -3590,7 +3653,7 @@ int32_t ocfd_save_stage0(void) {
 }
 int32_t ocfd_comput_amu_amk(void) {
   if (check_ready()) return 1;
-  if (G.S.ns > 1) launch("k_transport_ms", k_transport_ms, grid1(G.S.ni), dim3(256), G.S, 0);
+  if (G.S.ns > 1) launch_transport_ms(0, 0);
   else launch("k_transport", k_transport, grid1(G.S.ni), dim3(256), G.S);
   HIPCHK(hipGetLastError());
   return 0;
@@ -3598,7 +3661,7 @@ int32_t ocfd_comput_amu_amk(void) {
 int32_t ocfd_stage_begin(int32_t krk) {
   if (check_ready()) return 1;
   if (G.S.ns > 1) {
-    launch("k_transport_ms", k_transport_ms, grid1(G.S.ni), dim3(256), G.S, 0);
+    launch_transport_ms(0, 0);
   } else {
     launch("k_transport", k_transport, grid1(G.S.ni), dim3(256), G.S);
     launch("k_di_from_d", k_di_from_d, grid1(G.S.nh), dim3(256), G.S);
@@ -3663,7 +3726,7 @@ int32_t ocfd_comput_flow_variables(void) {
   if (check_ready()) return 1;
   launch("k_negt_reset", k_negt_reset, dim3(1), dim3(64), G.S, 0);
   launch_rk(1, 0.0, (int)(G.S.ns > 1 ? RK_PRIMS | RK_MS : RK_PRIMS));
-  launch("k_negt_repair", k_negt_repair, dim3(1), dim3(64), G.S);
+  launch("k_negt_repair", G.S.ns > 1 ? k_negt_repair<true> : k_negt_repair<false>, dim3(1), dim3(64), G.S);
   hipMemcpyAsync(G.h_negt, G.S.negt + 17, sizeof(int), hipMemcpyDeviceToHost, G.stream);
   HIPCHK(hipGetLastError());
   return 0;

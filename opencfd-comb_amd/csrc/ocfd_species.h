@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "ocfd_device.h"
+#include "ocfd_exp.h"
 
 #define GAS_NT_MAX 4
 #define GAS_R0 8.314       // CHEM_modules.f90:20
@@ -22,6 +23,10 @@ struct FlowGas {
   double tct[GAS_NT_MAX], tct_max;
   double Mi[OCFD_NS_MAX], Ri[OCFD_NS_MAX];
   double coef[OCFD_NS_MAX][GAS_NT_MAX][7], ect[OCFD_NS_MAX][GAS_NT_MAX];
+  // (A-1) R, B R, C R, D R, E R, Ect R of each range, and 2.5 R: the products
+  // that the mixture's sums of energy start with
+  double ev[GAS_NT_MAX][6][OCFD_NS_MAX], rcv[OCFD_NS_MAX];
+  double exp2t[CH_EXPN][2];  // chem_exp's table
   double mu_an[OCFD_NS_MAX][4], k_an[OCFD_NS_MAX][4], D_an[OCFD_NS_MAX][OCFD_NS_MAX][4];
   // Wilke factors that depend only on the molar masses, evaluated on the
   // host: wq = (M_j/M_k)^(1/4) and wrec = 1/sqrt(8 (1 + M_k/M_j))
@@ -29,80 +34,113 @@ struct FlowGas {
 };
 __constant__ FlowGas fg;
 
+// The bank by a pointer that the compiler cannot see through, taken afresh by
+// every function below: in a loop the hundreds of constants of an inlined
+// gas_T would be hoisted out and spilled (5,400 register moves in k_bc).
+typedef const __attribute__((address_space(4))) FlowGas* Gas;
+__device__ __forceinline__ Gas gas_bank() {
+  Gas g = (Gas)&fg;
+  asm volatile("" : "+s"(g));
+  return g;
+}
+
 __device__ __forceinline__ double gp3(double x) { double x2 = x * x; return x2 * x; }
 __device__ __forceinline__ double gp4(double x) { double x2 = x * x; return x2 * x2; }
 __device__ __forceinline__ double gp5(double x) { double x2 = x * x; return (x2 * x2) * x; }
 
-__device__ __forceinline__ int gas_range(double T) {
+__device__ __forceinline__ int gas_range(Gas g, double T) {
   int jc = 0;
-  for (int j = 0; j < fg.n_tct - 1; j++)
-    if (T > fg.tct[j]) jc = j + 1;
+  for (int j = 0; j < g->n_tct - 1; j++)
+    if (T > g->tct[j]) jc = j + 1;
   return jc;
 }
 
+// The species loops below run to the fixed bound, fully unrolled: with all
+// species present (FULL) without a test, so that the scalar loads of the bank
+// and the loads of the partial densities are all in flight together; with
+// fewer, a uniform branch each.  As loops of ns passes each pass waited for
+// its own loads: k_bc of a 48x36x36 jet 33 us against 24, k_comput_T_P 13
+// against 7.
+template <class F>
+__device__ __forceinline__ void each_species(F f) {
+  if (fg.ns == OCFD_NS_MAX) {
+#pragma unroll
+    for (int k = 0; k < OCFD_NS_MAX; k++) f(k);
+  } else {
+#pragma unroll
+    for (int k = 0; k < OCFD_NS_MAX; k++)
+      if (k < fg.ns) f(k);
+  }
+}
+
+// sum over the species of the energy polynomial's coefficients 0 .. N-1 in
+// range j (a uniform index)
+template <int N>
+__device__ __forceinline__ void gas_sums(Gas g, const double* di, int j, double* s) {
+#pragma unroll
+  for (int a = 0; a < N; a++) s[a] = 0.0;
+  each_species([&](int k) {
+#pragma unroll
+    for (int a = 0; a < N; a++) s[a] = s[a] + g->ev[j][a][k] * di[k];
+  });
+}
+
+// ... in range jc of each lane: the lanes of one range at a time, so that the
+// coefficients stay scalar loads
+template <int N>
+__device__ __forceinline__ void gas_sums_lane(Gas g, const double* di, int jc, double* s) {
+#pragma unroll
+  for (int a = 0; a < N; a++) s[a] = 0.0;
+  for (int j = 0; j < g->n_tct; j++)
+    if (jc == j) gas_sums<N>(g, di, j, s);
+}
+
 // comput_E_pgas (CHEM_thermdyn.f90:114-122) / comput_E_rgas (:203-231)
-__device__ double gas_E(const double* di, double T) {
-  const int ns = fg.ns;
-  if (!fg.real_gas) {
+__device__ __forceinline__ double gas_E(const double* di, double T) {
+  const Gas g = gas_bank();
+  if (!g->real_gas) {
     double E = 0.0;
-    for (int k = 0; k < ns; k++) E = E + 2.5 * fg.Ri[k] * di[k] * T;
+    each_species([&](int k) { E = E + g->rcv[k] * di[k] * T; });
     return E;
   }
-  double A1 = 0, B1 = 0, C1 = 0, D1 = 0, E1 = 0, Ect = 0;
-  const int jc = gas_range(T);
-  for (int k = 0; k < ns; k++) {
-    const double R1 = fg.Ri[k];
-    A1 = A1 + (fg.coef[k][jc][0] - 1.0) * R1 * di[k];
-    B1 = B1 + fg.coef[k][jc][1] * R1 * di[k];
-    C1 = C1 + fg.coef[k][jc][2] * R1 * di[k];
-    D1 = D1 + fg.coef[k][jc][3] * R1 * di[k];
-    E1 = E1 + fg.coef[k][jc][4] * R1 * di[k];
-    Ect = Ect + fg.ect[k][jc] * R1 * di[k];
-  }
-  if (T <= fg.tct_max) return A1 * T + B1 * (T * T) / 2.0 + C1 * gp3(T) / 3.0 + D1 * gp4(T) / 4.0 + E1 * gp5(T) / 5.0 + Ect;
-  const double tm = fg.tct_max;
+  double s[6];
+  gas_sums_lane<6>(g, di, gas_range(g, T), s);
+  const double A1 = s[0], B1 = s[1], C1 = s[2], D1 = s[3], E1 = s[4], Ect = s[5];
+  if (T <= g->tct_max) return A1 * T + B1 * (T * T) / 2.0 + C1 * gp3(T) / 3.0 + D1 * gp4(T) / 4.0 + E1 * gp5(T) / 5.0 + Ect;
+  const double tm = g->tct_max;
   const double Cv2 = A1 + B1 * tm + C1 * (tm * tm) + D1 * gp3(tm) + E1 * gp4(tm);
   return A1 * tm + B1 * (tm * tm) / 2.0 + C1 * gp3(tm) / 3.0 + D1 * gp4(tm) / 4.0 + E1 * gp5(tm) / 5.0 + Ect +
          Cv2 * (T - tm);
 }
 
 // comput_T_pgas (CHEM_thermdyn.f90:157-168) / comput_T_rgas (:326-382)
-__device__ double gas_T(const double* di, double E) {
-  const int ns = fg.ns;
-  if (!fg.real_gas) {
+__device__ __forceinline__ double gas_T(const double* di, double E) {
+  const Gas g = gas_bank();
+  if (!g->real_gas) {
     double rCv = 0.0;
-    for (int k = 0; k < ns; k++) rCv = rCv + 2.5 * fg.Ri[k] * di[k];
+    each_species([&](int k) { rCv = rCv + g->rcv[k] * di[k]; });
     return E / rCv;
   }
-  double A1[GAS_NT_MAX], B1[GAS_NT_MAX], C1[GAS_NT_MAX], D1[GAS_NT_MAX], E1[GAS_NT_MAX], Ect[GAS_NT_MAX];
+  double s[GAS_NT_MAX][6];
 #pragma unroll
   for (int j = 0; j < GAS_NT_MAX; j++) {
-    A1[j] = B1[j] = C1[j] = D1[j] = E1[j] = Ect[j] = 0.0;
-    if (j < fg.n_tct) {
-      for (int k = 0; k < ns; k++) {
-        const double R1 = fg.Ri[k];
-        A1[j] = A1[j] + (fg.coef[k][j][0] - 1.0) * R1 * di[k];
-        B1[j] = B1[j] + fg.coef[k][j][1] * R1 * di[k];
-        C1[j] = C1[j] + fg.coef[k][j][2] * R1 * di[k];
-        D1[j] = D1[j] + fg.coef[k][j][3] * R1 * di[k];
-        E1[j] = E1[j] + fg.coef[k][j][4] * R1 * di[k];
-        Ect[j] = Ect[j] + fg.ect[k][j] * R1 * di[k];
-      }
-    }
+#pragma unroll
+    for (int a = 0; a < 6; a++) s[j][a] = 0.0;
+    if (j < g->n_tct) gas_sums<6>(g, di, j, s[j]);
   }
-  double T1 = E / A1[0], T2 = T1;
+  double T1 = E / s[0][0], T2 = T1;
   for (int ks = 0; ks <= 30; ks++) {
-    const int jc = gas_range(T1);
-    double a = A1[0], b = B1[0], c = C1[0], d = D1[0], e = E1[0], ect = Ect[0];
+    const int jc = gas_range(g, T1);
+    double a = s[0][0], b = s[0][1], c = s[0][2], d = s[0][3], e = s[0][4], ect = s[0][5];
 #pragma unroll
     for (int j = 1; j < GAS_NT_MAX; j++)
-      if (jc == j) { a = A1[j]; b = B1[j]; c = C1[j]; d = D1[j]; e = E1[j]; ect = Ect[j]; }
+      if (jc == j) { a = s[j][0]; b = s[j][1]; c = s[j][2]; d = s[j][3]; e = s[j][4]; ect = s[j][5]; }
     double Et1, Ex;
-    if (T1 <= fg.tct_max) {
+    if (T1 <= g->tct_max) {
       Et1 = a * T1 + b * (T1 * T1) / 2.0 + c * gp3(T1) / 3.0 + d * gp4(T1) / 4.0 + e * gp5(T1) / 5.0 + ect;
       Ex = a + b * T1 + c * (T1 * T1) + d * gp3(T1) + e * gp4(T1);
     } else {
-      const double tm = fg.tct_max;
+      const double tm = g->tct_max;
       Ex = a + b * tm + c * (tm * tm) + d * gp3(tm) + e * gp4(tm);
       Et1 = a * tm + b * (tm * tm) / 2.0 + c * gp3(tm) / 3.0 + d * gp4(tm) / 4.0 + e * gp5(tm) / 5.0 + ect +
             Ex * (T1 - tm);
@@ -117,57 +155,61 @@ __device__ double gas_T(const double* di, double E) {
 
 // comput_P, CHEM_thermdyn.f90:385-395
 __device__ __forceinline__ double gas_P(const double* di, double T) {
+  const Gas g = gas_bank();
   double p = 0.0;
-  for (int k = 0; k < fg.ns; k++) p = p + fg.Ri[k] * di[k] * T;
+  each_species([&](int k) { p = p + g->Ri[k] * di[k] * T; });
   return p;
 }
 
 // comput_d, CHEM_thermdyn.f90:399-409 (ai = mass fractions)
 __device__ __forceinline__ double gas_d(const double* ai, double T, double p) {
+  const Gas g = gas_bank();
   double R1 = 0.0;
-  for (int k = 0; k < fg.ns; k++) R1 = R1 + fg.Ri[k] * ai[k];
+  each_species([&](int k) { R1 = R1 + g->Ri[k] * ai[k]; });
   return p / (T * R1);
 }
 
 // comput_Cp_pgas (CHEM_thermdyn.f90:125-136) / comput_Cp_rgas (:234-266)
-__device__ double gas_Cp(double d, const double* di, double T) {
-  const int ns = fg.ns;
-  if (!fg.real_gas) {
+__device__ __forceinline__ double gas_Cp(double d, const double* di, double T) {
+  const Gas g = gas_bank();
+  if (!g->real_gas) {
     double Cp = 0.0;
-    for (int k = 0; k < ns; k++) Cp = Cp + 3.5 * fg.Ri[k] * di[k];
+    each_species([&](int k) { Cp = Cp + 3.5 * g->Ri[k] * di[k]; });
     return Cp / d;
   }
-  double A1 = 0, B1 = 0, C1 = 0, D1 = 0, E1 = 0;
-  const int jc = gas_range(T);
-  for (int k = 0; k < ns; k++) {
-    const double R1 = fg.Ri[k];
-    A1 = A1 + fg.coef[k][jc][0] * R1 * di[k];
-    B1 = B1 + fg.coef[k][jc][1] * R1 * di[k];
-    C1 = C1 + fg.coef[k][jc][2] * R1 * di[k];
-    D1 = D1 + fg.coef[k][jc][3] * R1 * di[k];
-    E1 = E1 + fg.coef[k][jc][4] * R1 * di[k];
-  }
-  const double t = T <= fg.tct_max ? T : fg.tct_max;
-  return (A1 + B1 * t + C1 * (t * t) + D1 * gp3(t) + E1 * gp4(t)) / d;
+  double s[5];
+  gas_sums_lane<5>(g, di, gas_range(g, T), s);
+  const double t = T <= g->tct_max ? T : g->tct_max;
+  return (s[0] + s[1] * t + s[2] * (t * t) + s[3] * gp3(t) + s[4] * gp4(t)) / d;
 }
 
 // comput_hi_pgas (CHEM_thermdyn.f90:176-182) / comput_hi_rgas (:271-293)
 __device__ double gas_hi(int k, double T) {
-  if (!fg.real_gas) return 3.5 * fg.Ri[k] * T;
-  const int jc = gas_range(T);
-  const double c0 = fg.coef[k][jc][0], c1 = fg.coef[k][jc][1], c2 = fg.coef[k][jc][2], c3 = fg.coef[k][jc][3],
-               c4 = fg.coef[k][jc][4], ect = fg.ect[k][jc];
-  if (T <= fg.tct_max)
-    return (c0 * T + c1 * (T * T) / 2.0 + c2 * gp3(T) / 3.0 + c3 * gp4(T) / 4.0 + c4 * gp5(T) / 5.0 + ect) * fg.Ri[k];
-  const double tm = fg.tct_max;
+  const Gas g = gas_bank();
+  if (!g->real_gas) return 3.5 * g->Ri[k] * T;
+  const int jc = gas_range(g, T);
+  double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0, c4 = 0.0, ect = 0.0;
+  for (int j = 0; j < g->n_tct; j++)  // the lanes of one range at a time: scalar loads
+    if (jc == j) {
+      c0 = g->coef[k][j][0];
+      c1 = g->coef[k][j][1];
+      c2 = g->coef[k][j][2];
+      c3 = g->coef[k][j][3];
+      c4 = g->coef[k][j][4];
+      ect = g->ect[k][j];
+    }
+  if (T <= g->tct_max)
+    return (c0 * T + c1 * (T * T) / 2.0 + c2 * gp3(T) / 3.0 + c3 * gp4(T) / 4.0 + c4 * gp5(T) / 5.0 + ect) * g->Ri[k];
+  const double tm = g->tct_max;
   const double Cp_max = c0 + c1 * tm + c2 * (tm * tm) + c3 * gp3(tm) + c4 * gp4(tm);
   return (c0 * tm + c1 * (tm * tm) / 2.0 + c2 * gp3(tm) / 3.0 + c3 * gp4(tm) / 4.0 + c4 * gp5(tm) / 5.0 + ect +
-          Cp_max * (T - tm)) * fg.Ri[k];
+          Cp_max * (T - tm)) * g->Ri[k];
 }
 
-// Chemkin fit exp(a1 + a2 lnT + a3 lnT^2 + a4 lnT^3), TRANSPORT_modules.f90:276-277
+// exponent of the Chemkin fit exp(a1 + a2 lnT + a3 lnT^2 + a4 lnT^3),
+// TRANSPORT_modules.f90:276-277
 __device__ __forceinline__ double chemkin_fit(const double* a, double lT) {
-  return exp(a[0] + a[1] * lT + a[2] * (lT * lT) + a[3] * gp3(lT));
+  return __builtin_fma(__builtin_fma(__builtin_fma(a[3], lT, a[2]), lT, a[1]), lT, a[0]);
 }
 
 __device__ __forceinline__ void cell_ijk(const DevState& S, long c, int& i, int& j, int& k) {
@@ -181,49 +223,68 @@ __device__ __forceinline__ void cell_ijk(const DevState& S, long c, int& i, int&
 // comput_vis_coeff (TRANSPORT_modules.f90:259-306), comput_Cp,
 // comput_thermal_conductivity (:312-372), comput_diffusion_coeff (:378-424).
 // ===========================================================================
-// first: the launch opens a step and resets the negative-Et counters
-__global__ __launch_bounds__(256, 5) void k_transport_ms(DevState S, int first) {
+// conc: also c_m = di_m / d for the species diffusion (du_scaler_viscous),
+// whose di and d are at hand here.
+// Bound by its arithmetic: 9 + 9 + 36 exponentials a cell.  The fits are
+// Horner FMAs and chem_exp; a fit that the mixture rules divide by is the
+// exponential of the negative exponent, and the square roots of the
+// viscosities and their inverses come from the half exponent.  Largest
+// (mean) relative error of the H2 mixture's fits against 80-bit arithmetic,
+// 250 to 3500 K: viscosity 2.7e-15 (5.3e-16), conductivity 5.6e-15 (7.8e-16),
+// 1/D 5.2e-15 (9.2e-16); with powers, exp and divisions 5.6e-15 (8.6e-16),
+// 1.7e-14 (1.6e-15), 9.6e-15 (1.3e-15).  us before / now: 48x36x36 40 / 21,
+// 160x112x64 210 (and 57 for the concentrations) / 119.  first: the launch
+// opens a step and resets the negative-Et counters.
+template <bool FULL>
+__global__ __launch_bounds__(256, 4) void k_transport_ms(DevState S, int first, int conc) {
+  __shared__ double2 tab[CH_EXPN];
+  if (threadIdx.x < CH_EXPN) tab[threadIdx.x] = make_double2(fg.exp2t[threadIdx.x][0], fg.exp2t[threadIdx.x][1]);
+  __syncthreads();
   const long c = cell_index();
   if (first && blockIdx.x == 0 && threadIdx.x == 0) negt_reset(S, 1);
   if (c >= S.ni) return;
   int i, j, k;
   cell_ijk(S, c, i, j, k);
   const long q = hq(S, i, j, k);
-  const int ns = fg.ns;
+  const int ns = FULL ? OCFD_NS_MAX : fg.ns;
   // species loops run to the fixed bound with guards, fully unrolled, so the
   // per-species arrays stay in registers
   double di0[OCFD_NS_MAX], Xi[OCFD_NS_MAX];
+#pragma unroll
+  for (int m = 0; m < OCFD_NS_MAX; m++) di0[m] = m < ns ? S.di[q + (long)m * S.nh] : 0.0;
+  const double T = S.T[q];
+  if (conc) {
+    const double d = S.d[q];
+#pragma unroll
+    for (int m = 0; m < OCFD_NS_MAX; m++)
+      if (m < ns) S.cs[c + (long)m * S.ni] = di0[m] / d;
+  }
   double X0 = 0.0;
 #pragma unroll
   for (int m = 0; m < OCFD_NS_MAX; m++) {
-    di0[m] = m < ns ? S.di[q + (long)m * S.nh] : 0.0;
     Xi[m] = m < ns ? di0[m] / fg.Mi[m] : 0.0;
     if (m < ns) X0 = X0 + Xi[m];
   }
 #pragma unroll
   for (int m = 0; m < OCFD_NS_MAX; m++)
     if (m < ns) Xi[m] = Xi[m] / X0;
-  const double T = S.T[q];
+  const double lT = log(T);
   double amu;
   if (fg.flag_vis == 0) {
     const double TA = 288.15, TC = 110.4;
     const double tr = T / TA;
     amu = S.amu0 * sqrt(gp3(tr)) * (TA + TC) / (TC + T);
   } else {
-    const double lT = log(T);
-    double mui[OCFD_NS_MAX];
-#pragma unroll
-    for (int m = 0; m < OCFD_NS_MAX; m++) mui[m] = m < ns ? chemkin_fit(fg.mu_an[m], lT) * 0.1 : 1.0;
     // Wilke's Phi_kj = (1 + sqrt(mu_k/mu_j) (M_j/M_k)^(1/4))^2 / sqrt(8 (1 +
     // M_k/M_j)) (comput_vis_coeff, TRANSPORT_modules.f90:296-305) with
-    // sqrt(mu_k/mu_j) = sqrt(mu_k) / sqrt(mu_j): 9 square roots and 9
-    // divisions per cell instead of 81 and 162 (a few ulps from the
-    // reference's evaluation)
+    // sqrt(mu_k/mu_j) = sqrt(mu_k) / sqrt(mu_j), up to the fits' common
+    // factor 0.1
     double smu[OCFD_NS_MAX], rmu[OCFD_NS_MAX];
 #pragma unroll
     for (int m = 0; m < OCFD_NS_MAX; m++) {
-      smu[m] = sqrt(mui[m]);
-      rmu[m] = 1.0 / smu[m];
+      const double e = 0.5 * chemkin_fit(fg.mu_an[m], lT);
+      smu[m] = m < ns ? chem_exp(tab, e) : 1.0;
+      rmu[m] = m < ns ? chem_exp(tab, -e) : 1.0;
     }
     double mu = 0.0;
 #pragma unroll
@@ -233,31 +294,28 @@ __global__ __launch_bounds__(256, 5) void k_transport_ms(DevState S, int first) 
 #pragma unroll
         for (int jj = 0; jj < OCFD_NS_MAX; jj++) {
           if (jj < ns) {
-            const double a = 1.0 + smu[kk] * rmu[jj] * fg.wq[kk][jj];
-            const double Pkj = (a * a) * fg.wrec[kk][jj];
-            Pk0 = Pk0 + Xi[jj] * Pkj;
+            const double a = __builtin_fma(smu[kk] * rmu[jj], fg.wq[kk][jj], 1.0);
+            Pk0 = __builtin_fma(Xi[jj] * (a * a), fg.wrec[kk][jj], Pk0);
           }
         }
-        mu = mu + Xi[kk] * mui[kk] / Pk0;
+        mu = mu + Xi[kk] * (smu[kk] * smu[kk]) / Pk0;
       }
     }
-    amu = mu;
+    amu = mu * 0.1;
   }
-  const double Cp = gas_Cp(S.d[q], di0, T);
   double amk;
   if (fg.flag_cond == 0) {
-    amk = amu * Cp / S.pr;
+    amk = amu * gas_Cp(S.d[q], di0, T) / S.pr;
   } else {
-    const double lT = log(T);
     double Amk1 = 0.0, Amk2 = 0.0;
 #pragma unroll
     for (int m = 0; m < OCFD_NS_MAX; m++)
       if (m < ns) {
-        const double ki = chemkin_fit(fg.k_an[m], lT) * 1.0e-5;
-        Amk1 = Amk1 + Xi[m] * ki;
-        Amk2 = Amk2 + Xi[m] / ki;
+        const double e = chemkin_fit(fg.k_an[m], lT);
+        Amk1 = __builtin_fma(Xi[m], chem_exp(tab, e), Amk1);
+        Amk2 = __builtin_fma(Xi[m], chem_exp(tab, -e), Amk2);
       }
-    amk = 0.5 * (Amk1 + 1.0 / Amk2);
+    amk = 0.5 * (Amk1 + 1.0 / Amk2) * 1.0e-5;
   }
   S.Amu[c] = amu;
   S.Amk[c] = amk;
@@ -275,8 +333,7 @@ __global__ __launch_bounds__(256, 5) void k_transport_ms(DevState S, int first) 
     // reference fills the lower triangle from the upper one), each evaluated
     // once.  Visiting the pairs (a, b), a < b, with a outer and b inner adds
     // the terms of every ds_k in increasing j, the reference's order.
-    const double lT = log(T);
-    const double pq = S.p[q];
+    const double pq = GAS_ATM / S.p[q];
     double ds[OCFD_NS_MAX];
 #pragma unroll
     for (int m = 0; m < OCFD_NS_MAX; m++) ds[m] = 0.0;
@@ -285,14 +342,14 @@ __global__ __launch_bounds__(256, 5) void k_transport_ms(DevState S, int first) 
 #pragma unroll
       for (int b = a + 1; b < OCFD_NS_MAX; b++)
         if (b < ns) {
-          const double rD = 1.0 / (chemkin_fit(fg.D_an[a][b], lT) * 1.0e-4);
-          ds[a] = ds[a] + Xi[b] * rD;
-          ds[b] = ds[b] + Xi[a] * rD;
+          const double rD = chem_exp(tab, -chemkin_fit(fg.D_an[a][b], lT));
+          ds[a] = __builtin_fma(Xi[b], rD, ds[a]);
+          ds[b] = __builtin_fma(Xi[a], rD, ds[b]);
         }
 #pragma unroll
     for (int kk = 0; kk < OCFD_NS_MAX; kk++) {
       if (kk < ns)
-        S.AmD[c + (long)kk * S.ni] = (1.0 - Xi[kk]) / (ds[kk] + 1.0e-20) * GAS_ATM / pq;
+        S.AmD[c + (long)kk * S.ni] = (1.0 - Xi[kk]) / __builtin_fma(ds[kk], 1.0e4, 1.0e-20) * pq;
     }
   }
 }
@@ -309,8 +366,10 @@ template <> struct SpTile<0> { static constexpr int NP = 4, TS = 64; };
 template <> struct SpTile<1> { static constexpr int NP = 8, TS = 32; };
 template <> struct SpTile<2> { static constexpr int NP = 8, TS = 32; };
 
+// gridDim.z blocks share the species of a tile, ng each: see species_groups.
 template <int DIR>
-__global__ __launch_bounds__(256) void k_species_sweep(DevState S, int m0, int m1) {
+__global__ __launch_bounds__(256) void k_species_sweep(DevState S, int ma, int me, int ng) {
+  const int m0 = ma + (int)blockIdx.z * ng, m1 = min(me, m0 + ng);
   constexpr int NP = SpTile<DIR>::NP, TS = SpTile<DIR>::TS;
   constexpr int NPT = TS + 8, NIF = TS + 1;
   // one species at a time through small LDS buffers: the split velocity,
@@ -425,14 +484,13 @@ __global__ __launch_bounds__(256) void k_species_conc(DevState S, int m0, int m1
   for (int m = m0; m < m1; m++) S.cs[c + (long)m * S.ni] = S.di[q + (long)m * S.nh] / d;
 }
 
-// INT: every stencil of the cell is central (no wrap, no closure), so each
-// species' derivatives are straight-line code whose loads issue together.
-// Species m0 .. m1-1; Qp starts from zero at the first species (m0 = 0) and
-// from its stored value otherwise, so species taken one at a time add up in
-// the same order as all at once.
-template <int CD, bool IX, bool IY, bool IZ>
+// IX, IY, IZ: the stencils of the cell are central there (no wrap, no
+// closure), so each species' derivatives are straight-line code whose loads
+// issue together.  Species m0, m0 + step, .. < m1; out takes each one's share
+// of Qp.
+template <int CD, bool IX, bool IY, bool IZ, class Out>
 __device__ __forceinline__ void species_visc_prep_cell(const DevState& S, long c, long q, int i, int j, int k, int m0,
-                                                       int m1) {
+                                                       int m1, int step, Out out) {
   const double T0 = S.T[q], d0 = S.d[q];
   const double Akx = S.Akx[q], Aky = S.Aky[q], Akz = S.Akz[q];
   const double Aix = S.Aix[q], Aiy = S.Aiy[q], Aiz = S.Aiz[q];
@@ -441,13 +499,7 @@ __device__ __forceinline__ void species_visc_prep_cell(const DevState& S, long c
   const double Aix1 = S.Aix1[q], Aiy1 = S.Aiy1[q], Aiz1 = S.Aiz1[q];
   const double Asx1 = S.Asx1[q], Asy1 = S.Asy1[q], Asz1 = S.Asz1[q];
   const long ni = S.ni;
-  double Qpx = 0.0, Qpy = 0.0, Qpz = 0.0;
-  if (m0 > 0) {
-    Qpx = S.Qp[c];
-    Qpy = S.Qp[c + ni];
-    Qpz = S.Qp[c + 2 * ni];
-  }
-  for (int m = m0; m < m1; m++) {
+  for (int m = m0; m < m1; m += step) {
     const double* C = S.cs + (long)m * ni + c;
     auto dc = [&](auto central, int dir, int s) {
       const long st = S.si[dir];
@@ -468,23 +520,16 @@ __device__ __forceinline__ void species_visc_prep_cell(const DevState& S, long c
     const double ciy = uk * Aky + ui * Aiy + us * Asy;
     const double ciz = uk * Akz + ui * Aiz + us * Asz;
     const double E1 = dD * cix, E2 = dD * ciy, E3 = dD * ciz;
-    Qpx = Qpx + E1 * hi;
-    Qpy = Qpy + E2 * hi;
-    Qpz = Qpz + E3 * hi;
+    out(m, E1 * hi, E2 * hi, E3 * hi);
     S.Evs[c + (long)(3 * m) * ni] = E1 * Akx1 + E2 * Aky1 + E3 * Akz1;
     S.Evs[c + (long)(3 * m + 1) * ni] = E1 * Aix1 + E2 * Aiy1 + E3 * Aiz1;
     S.Evs[c + (long)(3 * m + 2) * ni] = E1 * Asx1 + E2 * Asy1 + E3 * Asz1;
   }
-  S.Qp[c] = Qpx;
-  S.Qp[c + ni] = Qpy;
-  S.Qp[c + 2 * ni] = Qpz;
 }
 
-template <int CD>
-__global__ __launch_bounds__(256) void k_species_visc_prep(DevState S, int m0, int m1) {
+template <int CD, class Out>
+__device__ __forceinline__ void species_visc_prep_at(const DevState& S, long c, int m0, int m1, int step, Out out) {
   constexpr int R = CD == 1 ? 4 : 3;
-  const long c = cell_index();
-  if (c >= S.ni) return;
   int i, j, k;
   cell_ijk(S, c, i, j, k);
   const long q = hq(S, i, j, k);
@@ -492,9 +537,53 @@ __global__ __launch_bounds__(256) void k_species_visc_prep(DevState S, int m0, i
   // central eta and zeta forms
   const bool ix = wave_all(central_cell(i, S.nx, R));
   const bool iyz = wave_all(central_cell(j, S.ny, R) && central_cell(k, S.nz, R));
-  if (ix && iyz) species_visc_prep_cell<CD, true, true, true>(S, c, q, i, j, k, m0, m1);
-  else if (iyz) species_visc_prep_cell<CD, false, true, true>(S, c, q, i, j, k, m0, m1);
-  else species_visc_prep_cell<CD, false, false, false>(S, c, q, i, j, k, m0, m1);
+  if (ix && iyz) species_visc_prep_cell<CD, true, true, true>(kernarg_again(), c, q, i, j, k, m0, m1, step, out);
+  else if (iyz) species_visc_prep_cell<CD, false, true, true>(kernarg_again(), c, q, i, j, k, m0, m1, step, out);
+  else species_visc_prep_cell<CD, false, false, false>(kernarg_again(), c, q, i, j, k, m0, m1, step, out);
+}
+
+// Species m0 .. m1-1, one thread per cell.  Qp starts from zero at the first
+// species (m0 = 0) and from its stored value otherwise, so species taken one
+// at a time add up in the same order as all at once.
+template <int CD>
+__global__ __launch_bounds__(256) void k_species_visc_prep(DevState S, int m0, int m1) {
+  const long c = cell_index();
+  if (c >= S.ni) return;
+  double Q[3] = {0.0, 0.0, 0.0};
+  if (m0 > 0) {
+#pragma unroll
+    for (int a = 0; a < 3; a++) Q[a] = S.Qp[c + a * S.ni];
+  }
+  species_visc_prep_at<CD>(S, c, m0, m1, 1, [&](int, double x, double y, double z) {
+    Q[0] = Q[0] + x;
+    Q[1] = Q[1] + y;
+    Q[2] = Q[2] + z;
+  });
+#pragma unroll
+  for (int a = 0; a < 3; a++) S.Qp[c + a * S.ni] = Q[a];
+}
+
+// ... all species of 64 cells by three wavefronts, every third species each:
+// for grids that would leave most wavefront slots empty (species_groups;
+// 48x36x36: 36 us with one thread a cell, 25 so).  The shares of Qp meet in
+// LDS and are added in the species' order, one component a wavefront.
+template <int CD>
+__global__ __launch_bounds__(192) void k_species_visc_prep3(DevState S) {
+  __shared__ double sQ[OCFD_NS_MAX][3][64];
+  const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+  const long c = xcd_block(blockIdx.x, gridDim.x) * 64 + lane;
+  const bool in = c < S.ni;
+  if (in)
+    species_visc_prep_at<CD>(S, c, w, S.ns, 3, [&](int m, double x, double y, double z) {
+      sQ[m][0][lane] = x;
+      sQ[m][1][lane] = y;
+      sQ[m][2][lane] = z;
+    });
+  __syncthreads();
+  if (!in) return;
+  double Q = 0.0;
+  for (int m = 0; m < S.ns; m++) Q = Q + sQ[m][w][lane];
+  S.Qp[c + w * S.ni] = Q;
 }
 
 // Species update: Dus += div(diffusive flux) Ajac (OCFD_scaler_viscous.f90:67-77)
@@ -502,7 +591,7 @@ __global__ __launch_bounds__(256) void k_species_visc_prep(DevState S, int m0, i
 // krk = 0 stores the complete right-hand side in dus instead.
 template <int CD, bool IX, bool IY, bool IZ>
 __device__ __forceinline__ void species_rk_cell(const DevState& S, long c, long q, int i, int j, int k, int krk,
-                                                double dt, int visc, int m0, int m1) {
+                                                double dt, int visc, int save, int m0, int m1) {
   const long ni = S.ni;
   const double ajac = S.Ajac[q];
   auto dv = [&](auto central, const double* F, int dir, int s) {
@@ -522,7 +611,8 @@ __device__ __forceinline__ void species_rk_cell(const DevState& S, long c, long 
   for (int m = m0; m < m1; m++) {
     const long qm = q + (long)m * S.nh, cm = c + (long)m * ni;
     // the stage's old values, read with the stencil loads
-    const double dn = krk >= 1 ? S.din[cm] : 0.0;
+    const double dn = save ? S.di[qm] : krk >= 1 ? S.din[cm] : 0.0;
+    if (save) S.din[cm] = dn;
     const double dold = krk >= 2 ? S.di[qm] : 0.0;
     double val = S.dus[cm];
     if (visc) {
@@ -540,9 +630,13 @@ __device__ __forceinline__ void species_rk_cell(const DevState& S, long c, long 
   }
 }
 
+// save: the stage opens a step, which starts from din = di, kept here from the
+// di that the update reads.  gridDim.y blocks share the species, ng each.
 template <int CD>
-__global__ __launch_bounds__(256) void k_species_rk(DevState S, int krk, double dt, int visc, int m0, int m1) {
+__global__ __launch_bounds__(256) void k_species_rk(DevState S, int krk, double dt, int visc, int save, int ma, int me,
+                                                    int ng) {
   constexpr int R = CD == 1 ? 4 : 3;
+  const int m0 = ma + (int)blockIdx.y * ng, m1 = min(me, m0 + ng);
   const long c = cell_index();
   if (c >= S.ni) return;
   int i, j, k;
@@ -550,9 +644,9 @@ __global__ __launch_bounds__(256) void k_species_rk(DevState S, int krk, double 
   const long q = hq(S, i, j, k);
   const bool ix = wave_all(central_cell(i, S.nx, R));
   const bool iyz = wave_all(central_cell(j, S.ny, R) && central_cell(k, S.nz, R));
-  if (ix && iyz) species_rk_cell<CD, true, true, true>(S, c, q, i, j, k, krk, dt, visc, m0, m1);
-  else if (iyz) species_rk_cell<CD, false, true, true>(S, c, q, i, j, k, krk, dt, visc, m0, m1);
-  else species_rk_cell<CD, false, false, false>(S, c, q, i, j, k, krk, dt, visc, m0, m1);
+  if (ix && iyz) species_rk_cell<CD, true, true, true>(kernarg_again(), c, q, i, j, k, krk, dt, visc, save, m0, m1);
+  else if (iyz) species_rk_cell<CD, false, true, true>(kernarg_again(), c, q, i, j, k, krk, dt, visc, save, m0, m1);
+  else species_rk_cell<CD, false, false, false>(kernarg_again(), c, q, i, j, k, krk, dt, visc, save, m0, m1);
 }
 
 // Rescaling_di (Comput_flow_variables.f90:101-121) and comput_T_P (:32-46)
@@ -560,17 +654,17 @@ __global__ __launch_bounds__(256) void k_species_rk(DevState S, int krk, double 
 __device__ __forceinline__ void ms_prims(const DevState& S, long q, double dd, double Et, double& T, double& p) {
   double di[OCFD_NS_MAX];
   double d0 = 0.0;
-  for (int m = 0; m < S.ns; m++) {
+  each_species([&](int m) {
     double x = S.di[q + (long)m * S.nh];
     if (x < 0.0) x = 0.0;
     di[m] = x;
     d0 = d0 + x;
-  }
+  });
   const double tmp = dd / d0;
-  for (int m = 0; m < S.ns; m++) {
+  each_species([&](int m) {
     di[m] = di[m] * tmp;
     S.di[q + (long)m * S.nh] = di[m];
-  }
+  });
   T = gas_T(di, Et);
   p = gas_P(di, T);
 }
@@ -583,7 +677,7 @@ __global__ __launch_bounds__(256) void k_comput_T_P(DevState S) {
   cell_ijk(S, c, i, j, k);
   const long q = hq(S, i, j, k);
   double di[OCFD_NS_MAX];
-  for (int m = 0; m < S.ns; m++) di[m] = S.di[q + (long)m * S.nh];
+  each_species([&](int m) { di[m] = S.di[q + (long)m * S.nh]; });
   const double T = gas_T(di, S.Et[q]);
   S.T[q] = T;
   S.p[q] = gas_P(di, T);
@@ -593,15 +687,15 @@ __global__ __launch_bounds__(256) void k_comput_T_P(DevState S) {
 __device__ __forceinline__ void face_update_ms(const DevState& S, long q, long c) {
   double di[OCFD_NS_MAX];
   double d0 = 0.0;
-  for (int m = 0; m < S.ns; m++) {
+  each_species([&](int m) {
     di[m] = S.di[q + (long)m * S.nh];
     d0 = d0 + di[m];
-  }
+  });
   const double dtmp = S.d[q] / d0;
-  for (int m = 0; m < S.ns; m++) {
+  each_species([&](int m) {
     di[m] = di[m] * dtmp;
     S.di[q + (long)m * S.nh] = di[m];
-  }
+  });
   const double T = S.T[q];
   const double Et = gas_E(di, T);
   const double p = gas_P(di, T);
@@ -620,21 +714,20 @@ __device__ __forceinline__ void face_update_ms(const DevState& S, long q, long c
 __device__ __forceinline__ void jet_inlet(const DevState& S, int j, int k) {
   const long q = hq(S, 1, j, k), pl = (long)S.ny * S.nz, r = (j - 1) + (long)S.ny * (k - 1);
   const double* in = S.jet_in;
-  const int ns = S.ns;
   if (S.jet_iflag == 0) {
     S.d[q] = in[r]; S.u[q] = in[r + pl]; S.v[q] = in[r + 2 * pl]; S.w[q] = in[r + 3 * pl]; S.T[q] = in[r + 4 * pl];
-    for (int m = 0; m < ns; m++) S.di[q + (long)m * S.nh] = in[r + (5L + m) * pl];
+    each_species([&](int m) { S.di[q + (long)m * S.nh] = in[r + (5L + m) * pl]; });
     return;
   }
   S.u[q] = in[r + pl]; S.v[q] = in[r + 2 * pl]; S.w[q] = in[r + 3 * pl]; S.T[q] = in[r + 4 * pl];
   const double d1 = in[r];
   double di1[OCFD_NS_MAX], ai1[OCFD_NS_MAX];
   double d0 = 0.0;
-  for (int m = 0; m < ns; m++) {
+  each_species([&](int m) {
     di1[m] = in[r + (5L + m) * pl];
     d0 = d0 + di1[m];
-  }
-  for (int m = 0; m < ns; m++) ai1[m] = di1[m] / d0;
+  });
+  each_species([&](int m) { ai1[m] = di1[m] / d0; });
   const double T1 = S.T[q];
   const double p1 = gas_P(di1, T1);
   const double Et1 = gas_E(di1, T1);
@@ -644,10 +737,10 @@ __device__ __forceinline__ void jet_inlet(const DevState& S, int j, int k) {
     S.p[q] = S.p[hq(S, 2, j, k)];
     const double d1new = gas_d(ai1, T1, S.p[q]);
     S.d[q] = d1new;
-    for (int m = 0; m < ns; m++) S.di[q + (long)m * S.nh] = d1new * ai1[m];
+    each_species([&](int m) { S.di[q + (long)m * S.nh] = d1new * ai1[m]; });
   } else {
     S.d[q] = d1;
-    for (int m = 0; m < ns; m++) S.di[q + (long)m * S.nh] = di1[m];
+    each_species([&](int m) { S.di[q + (long)m * S.nh] = di1[m]; });
   }
 }
 
@@ -656,7 +749,7 @@ __device__ __forceinline__ void jet_outlet(const DevState& S, int j, int k) {
   const long q = hq(S, S.nx, j, k), qa = hq(S, S.nx - 1, j, k);
   S.d[q] = S.d[qa]; S.u[q] = S.u[qa]; S.v[q] = S.v[qa]; S.w[q] = S.w[qa];
   S.T[q] = S.T[qa]; S.p[q] = S.p[qa]; S.Et[q] = S.Et[qa];
-  for (int m = 0; m < S.ns; m++) S.di[q + (long)m * S.nh] = S.di[qa + (long)m * S.nh];
+  each_species([&](int m) { S.di[q + (long)m * S.nh] = S.di[qa + (long)m * S.nh]; });
 }
 
 // Chemistry coupling (Chemical_time_advance, OCFD_Time_Adv.f90:169-196):
