@@ -16,6 +16,10 @@
 //   B(k,n) = TB ? B[n*ldb + k] : B[k*ldb + n]
 // Split-K writes per-split partial tiles that a second kernel sums in a fixed
 // order, so training is deterministic.
+//
+// Gradients of networks of at most 256 wide take k_net (ocfd_mlp_net.h)
+// instead, from a single sample up: the GEMMs' chain of launches costs 390 us
+// before any batch is large.  Wider networks do not fit its LDS tile.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -53,6 +57,8 @@ __device__ __forceinline__ float dgelu_f(float z) {
   const float s = gelu_sig(z);
   return s + z * s * (1.0f - s) * 2.0f * 0.7978845608028654f * (1.0f + 3.0f * 0.044715f * z * z);
 }
+
+#include "ocfd_mlp_net.h"
 
 template <bool TA, bool TB>
 __global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, int kchunk, const bf16* __restrict__ A, long lda,
@@ -221,8 +227,24 @@ __global__ __launch_bounds__(256) void k_loss_final(int nb, long count, const fl
   if (threadIdx.x == 0) loss[0] = (float)(red[0] / (double)count);
 }
 
+// The bf16 copies of a weight matrix [doutp][dinp]: row-major, and (networks
+// that k_net takes) W and its transpose in MFMA operand order.
+struct WeightCopies {
+  bf16 *Wb, *Wf, *Wt;
+  int dinp, doutp;
+  __device__ __forceinline__ void put(long i, float v) const {
+    if (!Wb) return;  // a bias
+    const bf16 h = (bf16)v;
+    Wb[i] = h;
+    if (!Wf) return;
+    const int o = (int)(i / dinp), k = (int)(i % dinp);
+    Wf[net_frag(o, k, dinp)] = h;
+    Wt[net_frag(k, o, doutp)] = h;
+  }
+};
+
 __global__ void k_adam(long n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, bf16* __restrict__ pb, float lr, float b1, float b2, float eps, float c1,
+                       float* __restrict__ v, WeightCopies pb, float lr, float b1, float b2, float eps, float c1,
                        float c2) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -233,12 +255,12 @@ __global__ void k_adam(long n, float* __restrict__ p, const float* __restrict__ 
   v[i] = vi;
   const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   p[i] = pi;
-  if (pb) pb[i] = (bf16)pi;
+  pb.put(i, pi);
 }
 
-__global__ void k_to_bf16(long n, const float* __restrict__ a, bf16* __restrict__ b) {
+__global__ void k_to_bf16(long n, const float* __restrict__ a, WeightCopies b) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = (bf16)a[i];
+  if (i < n) b.put(i, a[i]);
 }
 
 int pad_to(int x, int m) { return (x + m - 1) / m * m; }
@@ -247,7 +269,8 @@ struct Layer {
   int din = 0, dout = 0, dinp = 0, doutp = 0;
   float *W = nullptr, *b = nullptr, *gW = nullptr, *gb = nullptr;
   float *mW = nullptr, *vW = nullptr, *mb = nullptr, *vb = nullptr;
-  bf16* Wb = nullptr;
+  bf16 *Wb = nullptr, *Wf = nullptr, *Wt = nullptr;
+  WeightCopies copies() const { return {Wb, Wf, Wt, dinp, doutp}; }
   float* Z = nullptr;   // [Bp][doutp] pre-activation (output of the last layer)
   bf16* Ab = nullptr;   // [Bp][doutp] GELU(Z) (hidden layers)
   float* dZ = nullptr;  // [Bp][doutp]
@@ -262,6 +285,9 @@ struct MlpCtx {
   bf16* Xb = nullptr;
   float* part = nullptr;  // split-K partials
   long part_cap = 0;
+  bool net = false;        // every padded width at most NET_W: k_net
+  char* nws = nullptr;     // its workspace
+  size_t nws_cap = 0;
   float* lpart = nullptr;  // loss partials
   long lpart_cap = 0;
   float* loss = nullptr;  // device scalar
@@ -295,7 +321,10 @@ void free_batch() {
     l.dZb = nullptr;
   }
   hipFree(X.Xb);
+  hipFree(X.nws);
   X.Xb = nullptr;
+  X.nws = nullptr;
+  X.nws_cap = 0;
   X.Bcap = 0;
 }
 
@@ -311,6 +340,8 @@ void free_all() {
     hipFree(l.mb);
     hipFree(l.vb);
     hipFree(l.Wb);
+    hipFree(l.Wf);
+    hipFree(l.Wt);
   }
   X.lay.clear();
   hipFree(X.part);
@@ -415,6 +446,72 @@ int backward(long B, long Bp, const float* y) {
   return hipGetLastError() == hipSuccess ? 0 : mfail("ocfd_mlp: launch failed");
 }
 
+// k_net, k_net_dw, k_net_sum: gradients into gW, gb and, if given, the flat
+// array; the loss into X.loss and loss (may be NULL)
+int net_gradients(long B, const float* x, const float* y, float* grad, float* loss) {
+  NetArgs P{};
+  P.L = X.L;
+  P.B = B;
+  P.nblk = (int)((B + NET_R - 1) / NET_R);
+  P.x = x;
+  P.y = y;
+  P.grad = grad;
+  P.loss = X.loss;
+  P.loss2 = loss;
+  // the parts of the workspace, each a multiple of 256 bytes
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at += (bytes + 255) / 256 * 256;
+    return o;
+  };
+  size_t oA[MLP_MAX_LAYERS], oD[MLP_MAX_LAYERS], oG[MLP_MAX_LAYERS], oC[MLP_MAX_LAYERS];
+  const size_t rows = (size_t)P.nblk * NET_R;
+  long flat = 0;
+  for (int l = 0; l < X.L; l++) {
+    const Layer& s = X.lay[l];
+    NetLayer& d = P.l[l];
+    d.din = s.din;
+    d.dout = s.dout;
+    d.dinp = s.dinp;
+    d.doutp = s.doutp;
+    d.Wf = s.Wf;
+    d.Wt = s.Wt;
+    d.b = s.b;
+    d.gW = s.gW;
+    d.gb = s.gb;
+    d.flat = flat;
+    d.tile0 = P.tiles;
+    flat += (long)s.din * s.dout + s.dout;
+    P.tiles += (s.dinp / 64) * (s.doutp / 64);
+    P.bias_blocks += s.doutp / 64;
+    oA[l] = take(rows * s.dinp * sizeof(bf16));
+    oD[l] = take(rows * s.doutp * sizeof(bf16));
+    oG[l] = take(l + 1 < X.L ? rows * s.doutp * sizeof(float) : 0);
+    oC[l] = take((size_t)P.nblk * s.doutp * sizeof(float));
+  }
+  const size_t oL = take((size_t)P.nblk * sizeof(double)), oP = take((size_t)P.tiles * NET_S * 4096 * sizeof(float));
+  if (at > X.nws_cap) {
+    hipFree(X.nws);
+    X.nws = nullptr;
+    X.nws_cap = 0;
+    if (!dalloc(&X.nws, at)) return mfail("ocfd_mlp: out of device memory for the batch");
+    X.nws_cap = at;
+  }
+  for (int l = 0; l < X.L; l++) {
+    P.l[l].At = (bf16*)(X.nws + oA[l]);
+    P.l[l].Dt = (bf16*)(X.nws + oD[l]);
+    P.l[l].gp = (float*)(X.nws + oG[l]);
+    P.l[l].cs = (float*)(X.nws + oC[l]);
+  }
+  P.lp = (double*)(X.nws + oL);
+  P.part = (float*)(X.nws + oP);
+  hipLaunchKernelGGL(k_net, dim3(P.nblk), dim3(64 * NET_NW), 0, X.stream, P);
+  hipLaunchKernelGGL(k_net_dw, dim3(NET_S, P.tiles), dim3(256), 0, X.stream, P);
+  hipLaunchKernelGGL(k_net_sum, dim3(4 * P.tiles + P.bias_blocks + 1), dim3(256), 0, X.stream, P);
+  return hipGetLastError() == hipSuccess ? 0 : mfail("ocfd_mlp: launch failed");
+}
+
 int pack_input(long B, const float* x) {
   if (reserve(B)) return 1;
   const long Bp = pad_to((int)B, 64);
@@ -453,6 +550,8 @@ int32_t ocfd_mlp_create(int32_t n_layers, const int32_t* dims) {
   free_all();
   X.L = n_layers;
   X.lay.resize(n_layers);
+  X.net = true;
+  for (int l = 0; l <= n_layers; l++) X.net = X.net && dims[l] <= NET_W;
   for (int l = 0; l < n_layers; l++) {
     Layer& y = X.lay[l];
     y.din = dims[l];
@@ -466,6 +565,9 @@ int32_t ocfd_mlp_create(int32_t n_layers, const int32_t* dims) {
     if (hipMemset(y.W, 0, nw * 4) || hipMemset(y.mW, 0, nw * 4) || hipMemset(y.vW, 0, nw * 4) ||
         hipMemset(y.Wb, 0, nw * 2) || hipMemset(y.b, 0, y.doutp * 4) || hipMemset(y.mb, 0, y.doutp * 4) ||
         hipMemset(y.vb, 0, y.doutp * 4) || hipMemset(y.gW, 0, nw * 4) || hipMemset(y.gb, 0, y.doutp * 4))
+      return mfail("ocfd_mlp_create: memset failed");
+    if (X.net && (!dalloc(&y.Wf, nw) || !dalloc(&y.Wt, nw))) return mfail("ocfd_mlp_create: out of device memory");
+    if (X.net && (hipMemset(y.Wf, 0, nw * 2) || hipMemset(y.Wt, 0, nw * 2)))
       return mfail("ocfd_mlp_create: memset failed");
   }
   if (!X.stream && hipStreamCreateWithFlags(&X.stream, hipStreamNonBlocking) != hipSuccess)
@@ -505,7 +607,7 @@ int32_t ocfd_mlp_set_params(const float* flat) {
         hipMemcpy(l.b, b.data(), b.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
       return mfail("ocfd_mlp_set_params: copy failed");
     const long nw = (long)w.size();
-    hipLaunchKernelGGL(k_to_bf16, dim3(blocks(nw)), dim3(256), 0, X.stream, nw, l.W, l.Wb);
+    hipLaunchKernelGGL(k_to_bf16, dim3(blocks(nw)), dim3(256), 0, X.stream, nw, l.W, l.copies());
     if (hipMemsetAsync(l.mW, 0, nw * 4, X.stream) || hipMemsetAsync(l.vW, 0, nw * 4, X.stream) ||
         hipMemsetAsync(l.mb, 0, l.doutp * 4, X.stream) || hipMemsetAsync(l.vb, 0, l.doutp * 4, X.stream))
       return mfail("ocfd_mlp_set_params: memset failed");
@@ -555,6 +657,7 @@ int32_t ocfd_mlp_forward(int64_t B, const float* x, float* y) {
 int32_t ocfd_mlp_gradients(int64_t B, const float* x, const float* y, float* grad, float* loss) {
   if (!X.ready) return mfail("ocfd_mlp_gradients: no network");
   if (B <= 0) return mfail("ocfd_mlp_gradients: empty batch");
+  if (X.net) return net_gradients(B, x, y, grad, loss);
   if (pack_input(B, x)) return 1;
   const long Bp = pad_to((int)B, 64);
   if (forward(Bp) || backward(B, Bp, y)) return 1;
@@ -579,20 +682,24 @@ int32_t ocfd_mlp_train_step(int64_t B, const float* x, const float* y, float lr,
                             float* loss) {
   if (!X.ready) return mfail("ocfd_mlp_train_step: no network");
   if (B <= 0) return mfail("ocfd_mlp_train_step: empty batch");
-  if (pack_input(B, x)) return 1;
-  const long Bp = pad_to((int)B, 64);
-  if (forward(Bp) || backward(B, Bp, y)) return 1;
+  if (X.net) {
+    if (net_gradients(B, x, y, nullptr, loss)) return 1;
+  } else {
+    if (pack_input(B, x)) return 1;
+    const long Bp = pad_to((int)B, 64);
+    if (forward(Bp) || backward(B, Bp, y)) return 1;
+  }
   X.step++;
   X.version++;
   const float c1 = 1.f - powf(beta1, (float)X.step), c2 = 1.f - powf(beta2, (float)X.step);
   for (auto& l : X.lay) {
     const long nw = (long)l.doutp * l.dinp;
-    hipLaunchKernelGGL(k_adam, dim3(blocks(nw)), dim3(256), 0, X.stream, nw, l.W, l.gW, l.mW, l.vW, l.Wb, lr, beta1,
+    hipLaunchKernelGGL(k_adam, dim3(blocks(nw)), dim3(256), 0, X.stream, nw, l.W, l.gW, l.mW, l.vW, l.copies(), lr, beta1,
                        beta2, eps, c1, c2);
     hipLaunchKernelGGL(k_adam, dim3(blocks(l.doutp)), dim3(256), 0, X.stream, (long)l.doutp, l.b, l.gb, l.mb, l.vb,
-                       (bf16*)nullptr, lr, beta1, beta2, eps, c1, c2);
+                       WeightCopies{}, lr, beta1, beta2, eps, c1, c2);
   }
-  if (loss && hipMemcpyAsync(loss, X.loss, 4, hipMemcpyDeviceToDevice, X.stream) != hipSuccess)
+  if (loss && !X.net && hipMemcpyAsync(loss, X.loss, 4, hipMemcpyDeviceToDevice, X.stream) != hipSuccess)
     return mfail("ocfd_mlp_train_step: copy failed");
   return hipGetLastError() == hipSuccess ? 0 : mfail("ocfd_mlp_train_step: launch failed");
 }
