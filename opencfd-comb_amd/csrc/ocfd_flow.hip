@@ -3238,6 +3238,7 @@ int32_t ocfd_set_species(int32_t n_tct, const double* tct, double tct_max, const
     }
   for (int k = 0; k < ns; k++) {
     h.Mi[k] = mi[k];
+    h.rMi[k] = 1.0 / mi[k];
     h.Ri[k] = GAS_R0 / mi[k];
     for (int j = 0; j < GAS_NT_MAX; j++)
       for (int a = 0; a < 7; a++) h.coef[k][j][a] = (coef && j < h.n_tct) ? coef[((long)k * h.n_tct + j) * 7 + a] : 0.0;

@@ -21,7 +21,7 @@
 struct FlowGas {
   int ns, n_tct, real_gas, flag_vis, flag_cond, flag_diff;
   double tct[GAS_NT_MAX], tct_max;
-  double Mi[OCFD_NS_MAX], Ri[OCFD_NS_MAX];
+  double Mi[OCFD_NS_MAX], rMi[OCFD_NS_MAX], Ri[OCFD_NS_MAX];  // rMi = 1 / Mi
   double coef[OCFD_NS_MAX][GAS_NT_MAX][7], ect[OCFD_NS_MAX][GAS_NT_MAX];
   // (A-1) R, B R, C R, D R, E R, Ect R of each range, and 2.5 R: the products
   // that the mixture's sums of energy start with
@@ -44,6 +44,12 @@ __device__ __forceinline__ Gas gas_bank() {
   return g;
 }
 
+// a / b to the last bit, given r = 1 / b correctly rounded: the quotient's
+// remainder corrects it (Markstein).  3 instructions against a division's 11.
+__device__ __forceinline__ double quot(double a, double b, double r) {
+  const double q = a * r;
+  return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+}
 __device__ __forceinline__ double gp3(double x) { double x2 = x * x; return x2 * x; }
 __device__ __forceinline__ double gp4(double x) { double x2 = x * x; return x2 * x2; }
 __device__ __forceinline__ double gp5(double x) { double x2 = x * x; return (x2 * x2) * x; }
@@ -106,10 +112,10 @@ __device__ __forceinline__ double gas_E(const double* di, double T) {
   double s[6];
   gas_sums_lane<6>(g, di, gas_range(g, T), s);
   const double A1 = s[0], B1 = s[1], C1 = s[2], D1 = s[3], E1 = s[4], Ect = s[5];
-  if (T <= g->tct_max) return A1 * T + B1 * (T * T) / 2.0 + C1 * gp3(T) / 3.0 + D1 * gp4(T) / 4.0 + E1 * gp5(T) / 5.0 + Ect;
+  if (T <= g->tct_max) return A1 * T + B1 * (T * T) / 2.0 + quot(C1 * gp3(T), 3.0, 1.0 / 3.0) + D1 * gp4(T) / 4.0 + quot(E1 * gp5(T), 5.0, 0.2) + Ect;
   const double tm = g->tct_max;
   const double Cv2 = A1 + B1 * tm + C1 * (tm * tm) + D1 * gp3(tm) + E1 * gp4(tm);
-  return A1 * tm + B1 * (tm * tm) / 2.0 + C1 * gp3(tm) / 3.0 + D1 * gp4(tm) / 4.0 + E1 * gp5(tm) / 5.0 + Ect +
+  return A1 * tm + B1 * (tm * tm) / 2.0 + quot(C1 * gp3(tm), 3.0, 1.0 / 3.0) + D1 * gp4(tm) / 4.0 + quot(E1 * gp5(tm), 5.0, 0.2) + Ect +
          Cv2 * (T - tm);
 }
 
@@ -137,12 +143,12 @@ __device__ __forceinline__ double gas_T(const double* di, double E) {
       if (jc == j) { a = s[j][0]; b = s[j][1]; c = s[j][2]; d = s[j][3]; e = s[j][4]; ect = s[j][5]; }
     double Et1, Ex;
     if (T1 <= g->tct_max) {
-      Et1 = a * T1 + b * (T1 * T1) / 2.0 + c * gp3(T1) / 3.0 + d * gp4(T1) / 4.0 + e * gp5(T1) / 5.0 + ect;
+      Et1 = a * T1 + b * (T1 * T1) / 2.0 + quot(c * gp3(T1), 3.0, 1.0 / 3.0) + d * gp4(T1) / 4.0 + quot(e * gp5(T1), 5.0, 0.2) + ect;
       Ex = a + b * T1 + c * (T1 * T1) + d * gp3(T1) + e * gp4(T1);
     } else {
       const double tm = g->tct_max;
       Ex = a + b * tm + c * (tm * tm) + d * gp3(tm) + e * gp4(tm);
-      Et1 = a * tm + b * (tm * tm) / 2.0 + c * gp3(tm) / 3.0 + d * gp4(tm) / 4.0 + e * gp5(tm) / 5.0 + ect +
+      Et1 = a * tm + b * (tm * tm) / 2.0 + quot(c * gp3(tm), 3.0, 1.0 / 3.0) + d * gp4(tm) / 4.0 + quot(e * gp5(tm), 5.0, 0.2) + ect +
             Ex * (T1 - tm);
     }
     T2 = T1 - (Et1 - E) / Ex;
@@ -199,10 +205,10 @@ __device__ double gas_hi(int k, double T) {
       ect = g->ect[k][j];
     }
   if (T <= g->tct_max)
-    return (c0 * T + c1 * (T * T) / 2.0 + c2 * gp3(T) / 3.0 + c3 * gp4(T) / 4.0 + c4 * gp5(T) / 5.0 + ect) * g->Ri[k];
+    return (c0 * T + c1 * (T * T) / 2.0 + quot(c2 * gp3(T), 3.0, 1.0 / 3.0) + c3 * gp4(T) / 4.0 + quot(c4 * gp5(T), 5.0, 0.2) + ect) * g->Ri[k];
   const double tm = g->tct_max;
   const double Cp_max = c0 + c1 * tm + c2 * (tm * tm) + c3 * gp3(tm) + c4 * gp4(tm);
-  return (c0 * tm + c1 * (tm * tm) / 2.0 + c2 * gp3(tm) / 3.0 + c3 * gp4(tm) / 4.0 + c4 * gp5(tm) / 5.0 + ect +
+  return (c0 * tm + c1 * (tm * tm) / 2.0 + quot(c2 * gp3(tm), 3.0, 1.0 / 3.0) + c3 * gp4(tm) / 4.0 + quot(c4 * gp5(tm), 5.0, 0.2) + ect +
           Cp_max * (T - tm)) * g->Ri[k];
 }
 
@@ -233,7 +239,7 @@ __device__ __forceinline__ void cell_ijk(const DevState& S, long c, int& i, int&
 // 250 to 3500 K: viscosity 2.7e-15 (5.3e-16), conductivity 5.6e-15 (7.8e-16),
 // 1/D 5.2e-15 (9.2e-16); with powers, exp and divisions 5.6e-15 (8.6e-16),
 // 1.7e-14 (1.6e-15), 9.6e-15 (1.3e-15).  us before / now: 48x36x36 40 / 21,
-// 160x112x64 210 (and 57 for the concentrations) / 119.  first: the launch
+// 160x112x64 210 (and 57 for the concentrations) / 112.  first: the launch
 // opens a step and resets the negative-Et counters.
 template <bool FULL>
 __global__ __launch_bounds__(256, 4) void k_transport_ms(DevState S, int first, int conc) {
@@ -254,20 +260,21 @@ __global__ __launch_bounds__(256, 4) void k_transport_ms(DevState S, int first, 
   for (int m = 0; m < OCFD_NS_MAX; m++) di0[m] = m < ns ? S.di[q + (long)m * S.nh] : 0.0;
   const double T = S.T[q];
   if (conc) {
-    const double d = S.d[q];
+    const double d = S.d[q], rd = 1.0 / d;
 #pragma unroll
     for (int m = 0; m < OCFD_NS_MAX; m++)
-      if (m < ns) S.cs[c + (long)m * S.ni] = di0[m] / d;
+      if (m < ns) S.cs[c + (long)m * S.ni] = quot(di0[m], d, rd);
   }
   double X0 = 0.0;
 #pragma unroll
   for (int m = 0; m < OCFD_NS_MAX; m++) {
-    Xi[m] = m < ns ? di0[m] / fg.Mi[m] : 0.0;
+    Xi[m] = m < ns ? quot(di0[m], fg.Mi[m], fg.rMi[m]) : 0.0;
     if (m < ns) X0 = X0 + Xi[m];
   }
+  const double rX0 = 1.0 / X0;
 #pragma unroll
   for (int m = 0; m < OCFD_NS_MAX; m++)
-    if (m < ns) Xi[m] = Xi[m] / X0;
+    if (m < ns) Xi[m] = quot(Xi[m], X0, rX0);
   const double lT = log(T);
   double amu;
   if (fg.flag_vis == 0) {
@@ -361,10 +368,35 @@ __global__ __launch_bounds__(256, 4) void k_transport_ms(DevState S, int first, 
 // Each species only reads its own di, so doing them together equals the
 // reference's one-species-at-a-time order.
 // ===========================================================================
+// A tile's points, NP (TS + 8), and its interfaces, NP (TS + 1), fit the 256
+// threads: a thread owns one point and one interface for the whole species
+// loop, and what belongs to them (addresses, split velocities, kinds, old
+// interface values) stays in registers.  The sweeps are bound by their vector
+// instructions (vector units 0.7 to 0.9 busy); with tiles of 64 and 32 cells
+// the loops over points and interfaces took their indexes apart again for
+// every species, more than half of the instructions.  160x112x64, nine
+// species, us x / y / z: 228 / 202 / 162, now 170 / 151 / 134.
 template <int DIR> struct SpTile;
-template <> struct SpTile<0> { static constexpr int NP = 4, TS = 64; };
-template <> struct SpTile<1> { static constexpr int NP = 8, TS = 32; };
-template <> struct SpTile<2> { static constexpr int NP = 8, TS = 32; };
+template <> struct SpTile<0> { static constexpr int NP = 4, TS = 56; };
+template <> struct SpTile<1> { static constexpr int NP = 8, TS = 24; };
+template <> struct SpTile<2> { static constexpr int NP = 8, TS = 24; };
+
+// Reconstruction where the wavefront's lanes mostly agree: ku is their common
+// kind (a scalar branch) or -1.
+__device__ __forceinline__ double recon_wave(int ku, int kind, const double* w, const double* ud7l) {
+  switch (ku) {
+    case K_UD7L: return recon(K_UD7L, w, ud7l);
+    case K_WENO7: return recon_weno7(w);
+    case K_WENO5: return recon_weno5(w, 1);
+    case K_OMP6: return recon_omp6(w);
+  }
+  return recon(kind, w, ud7l);
+}
+__device__ __forceinline__ int common_kind(int kind, bool on) {
+  const unsigned long long m = __ballot(on);
+  const int k0 = __builtin_amdgcn_readlane(kind, m ? __builtin_ctzll(m) : 0);
+  return wave_all(!on || kind == k0) ? k0 : -1;
+}
 
 // gridDim.z blocks share the species of a tile, ng each: see species_groups.
 template <int DIR>
@@ -372,15 +404,12 @@ __global__ __launch_bounds__(256) void k_species_sweep(DevState S, int ma, int m
   const int m0 = ma + (int)blockIdx.z * ng, m1 = min(me, m0 + ng);
   constexpr int NP = SpTile<DIR>::NP, TS = SpTile<DIR>::TS;
   constexpr int NPT = TS + 8, NIF = TS + 1;
-  // one species at a time through small LDS buffers: the split velocity,
-  // the point index and the reconstruction kind are formed once
-  __shared__ double sV[NP * NPT];
-  __shared__ long sQ[NP * NPT];
-  __shared__ double sF[2 * NP * NPT];
-  __shared__ double sH[2 * NP * NIF];
-  __shared__ uint8_t sK[2 * NP * NIF];
+  constexpr int LPS = DIR == 0 ? 1 : NP;  // LDS distance of neighbours along the pencil
+  static_assert(NP * NPT <= 256 && NP * NIF <= 256, "one point and one interface a thread");
+  // one species at a time: split fluxes of the points, values at the interfaces
+  __shared__ double sF[2][NP * NPT];
+  __shared__ double sH[2][NP * NIF];
   __shared__ PencilBase<DIR, NP> PB;
-  const int ns = S.ns;
   const int n = S.n[DIR];
   const long nb = (long)gridDim.x * gridDim.y;
   const long lb = xcd_block((long)blockIdx.y * gridDim.x + blockIdx.x, nb);
@@ -390,79 +419,75 @@ __global__ __launch_bounds__(256) void k_species_sweep(DevState S, int ma, int m
   const int ncell = min(TS, n - c0 + 1);
   const long npen = DIR == 0 ? (long)S.ny * S.nz : DIR == 1 ? (long)S.nx * S.nz : (long)S.nx * S.ny;
   const long pen0 = by * NP;
-  auto lp = [](int pl, int s) { return DIR == 0 ? pl * NPT + s : s * NP + pl; };
-  auto lh = [](int pl, int l) { return DIR == 0 ? pl * NIF + l : l * NP + pl; };
-  const double* M1 = DIR == 0 ? S.Akx1 : DIR == 1 ? S.Aix1 : S.Asx1;
-  const double* M2 = DIR == 0 ? S.Aky1 : DIR == 1 ? S.Aiy1 : S.Asy1;
-  const double* M3 = DIR == 0 ? S.Akz1 : DIR == 1 ? S.Aiz1 : S.Asz1;
   const int tid = threadIdx.x;
   pencil_bases<DIR, NP>(S, pen0, npen, PB);
   __syncthreads();
-  for (int t = tid; t < NP * NPT; t += blockDim.x) {
-    const int pl = DIR == 0 ? t / NPT : t % NP;
-    const int sl = DIR == 0 ? t % NPT : t / NP;
-    const long pen = pen0 + pl;
-    if (pen >= npen || sl > ncell + 7) continue;
-    const long q = PB.hq1[pl] + (long)(wrap(c0 - 4 + sl, n, S.per[DIR]) - 1) * S.sh[DIR];
-    sQ[lp(pl, sl)] = q;
-    sV[lp(pl, sl)] = M1[q] * S.u[q] + M2[q] * S.v[q] + M3[q] * S.w[q];
+  // the thread's point
+  const int ppl = DIR == 0 ? tid / NPT : tid % NP, psl = DIR == 0 ? tid % NPT : tid / NP;
+  const bool pon = tid < NP * NPT && pen0 + ppl < npen && psl <= ncell + 7;
+  double vp = 0.0, vm = 0.0;
+  const double* Dp = S.di;
+  if (pon) {
+    const double* M1 = DIR == 0 ? S.Akx1 : DIR == 1 ? S.Aix1 : S.Asx1;
+    const double* M2 = DIR == 0 ? S.Aky1 : DIR == 1 ? S.Aiy1 : S.Asy1;
+    const double* M3 = DIR == 0 ? S.Akz1 : DIR == 1 ? S.Aiz1 : S.Asz1;
+    const long q = PB.hq1[ppl] + (long)(wrap(c0 - 4 + psl, n, S.per[DIR]) - 1) * S.sh[DIR];
+    const double vs = M1[q] * S.u[q] + M2[q] * S.v[q] + M3[q] * S.w[q];
+    vp = 0.5 * (vs + fabs(vs));
+    vm = 0.5 * (vs - fabs(vs));
+    Dp = S.di + q + (long)m0 * S.nh;
   }
-  const bool hyb = S.scheme == OCFD_SCHEME_HYBRID;
-  for (int t = tid; t < 2 * NP * NIF; t += blockDim.x) {
-    const int side = t / (NP * NIF);
-    const int r = t % (NP * NIF);
-    const int pl = DIR == 0 ? r / NIF : r % NP;
-    const int l = DIR == 0 ? r % NIF : r / NP;
-    const long pen = pen0 + pl;
-    if (pen >= npen || l > ncell) continue;
+  // the thread's interface, and the cell above it
+  const int pl = DIR == 0 ? tid / NIF : tid % NP, l = DIR == 0 ? tid % NIF : tid / NP;
+  const bool on = tid < NP * NIF && pen0 + pl < npen && l <= ncell;
+  const bool out = on && l < ncell;
+  int kp = 0, km = 0;
+  double* U = S.dus;
+  double aj = 0.0;
+  if (on) {
     const int s_if = c0 - 1 + l;
-    const int mask = hyb ? (int)S.mask[DIR][PB.mb[pl] + (long)s_if * mask_stride<DIR>(S)] : 0;
-    sK[t] = (uint8_t)recon_kind(S, DIR, s_if, side, mask);
+    const int mask = S.scheme == OCFD_SCHEME_HYBRID
+                         ? (int)S.mask[DIR][PB.mb[pl] + (long)s_if * mask_stride<DIR>(S)] : 0;
+    kp = recon_kind(S, DIR, s_if, 0, mask);
+    km = recon_kind(S, DIR, s_if, 1, mask);
+    if (out) {
+      U = S.dus + PB.iq1[pl] + (long)(c0 + l - 1) * S.si[DIR] + (long)m0 * S.ni;
+      if (DIR == 2) aj = S.Ajac[PB.hq1[pl] + (long)(c0 + l - 1) * S.sh[DIR]];
+    }
   }
+  const int kup = common_kind(kp, on), kum = common_kind(km, on);
   const double h1 = S.h_1[DIR];
-  (void)ns;
-  for (int m = m0; m < m1; m++) {
-    const double* Di = S.di + (long)m * S.nh;
-    for (int t = tid; t < NP * NPT; t += blockDim.x) {
-      const int pl = DIR == 0 ? t / NPT : t % NP;
-      const int sl = DIR == 0 ? t % NPT : t / NP;
-      if (pen0 + pl >= npen || sl > ncell + 7) continue;
-      const int a = lp(pl, sl);
-      const double vs = sV[a], fs = Di[sQ[a]];
-      sF[a] = 0.5 * (vs + fabs(vs)) * fs;
-      sF[NP * NPT + a] = 0.5 * (vs - fabs(vs)) * fs;
+  const double* Fp = &sF[0][DIR == 0 ? pl * NPT + l : l * NP + pl];
+  const double* Fm = Fp + NP * NPT;
+  double* Hp = &sH[0][tid];
+  for (int m = m0; m < m1; m++, Dp += S.nh, U += S.ni) {
+    double old = 0.0;
+    if (DIR != 0 && out) old = *U;  // in flight until the end of the pass
+    if (pon) {
+      const double fs = *Dp;
+      sF[0][tid] = vp * fs;
+      sF[1][tid] = vm * fs;
     }
     __syncthreads();  // sF complete; the previous species' outputs have read sH
-    for (int t = tid; t < 2 * NP * NIF; t += blockDim.x) {
-      const int side = t / (NP * NIF);
-      const int r = t % (NP * NIF);
-      const int pl = DIR == 0 ? r / NIF : r % NP;
-      const int l = DIR == 0 ? r % NIF : r / NP;
-      if (pen0 + pl >= npen || l > ncell) continue;
-      const double* F = sF + side * NP * NPT;
+    double hp0 = 0.0, hm0 = 0.0;
+    if (on) {
       double w[8];
 #pragma unroll
-      for (int qq = 0; qq < 8; qq++) w[qq] = F[lp(pl, side ? l + 7 - qq : l + qq)];
-      sH[t] = recon(sK[t], w, S.ud7l);
+      for (int qq = 0; qq < 8; qq++) w[qq] = Fp[qq * LPS];
+      hp0 = recon_wave(kup, kp, w, S.ud7l);
+#pragma unroll
+      for (int qq = 0; qq < 8; qq++) w[qq] = Fm[(7 - qq) * LPS];
+      hm0 = recon_wave(kum, km, w, S.ud7l);
+      Hp[0] = hp0;
+      Hp[NP * NIF] = hm0;
     }
     __syncthreads();  // sH complete; sF may be overwritten
-    for (int t = tid; t < NP * TS; t += blockDim.x) {
-      const int pl = DIR == 0 ? t / TS : t % NP;
-      const int c = DIR == 0 ? t % TS : t / NP;
-      const long pen = pen0 + pl;
-      if (pen >= npen || c >= ncell) continue;
-      const double hp1 = sH[lh(pl, c + 1)], hp0 = sH[lh(pl, c)];
-      const double hm1 = sH[NP * NIF + lh(pl, c + 1)], hm0 = sH[NP * NIF + lh(pl, c)];
+    if (out) {
+      const double hp1 = Hp[LPS], hm1 = Hp[NP * NIF + LPS];
       const double val = (hp1 - hp0 + hm1 - hm0) * h1;
-      const long ci = PB.iq1[pl] + (long)(c0 + c - 1) * S.si[DIR] + (long)m * S.ni;
-      if (DIR == 0) {
-        S.dus[ci] = val;
-      } else if (DIR == 1) {
-        S.dus[ci] = S.dus[ci] + val;
-      } else {
-        const long q = sQ[lp(pl, c + 4)];
-        S.dus[ci] = -(S.dus[ci] + val) * S.Ajac[q];
-      }
+      if (DIR == 0) *U = val;
+      else if (DIR == 1) *U = old + val;
+      else *U = -(old + val) * aj;
     }
   }
 }
