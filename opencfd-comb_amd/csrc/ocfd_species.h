@@ -674,6 +674,210 @@ __global__ __launch_bounds__(256) void k_species_rk(DevState S, int krk, double 
   else species_rk_cell<CD, false, false, false>(kernarg_again(), c, q, i, j, k, krk, dt, visc, save, m0, m1);
 }
 
+// The two kernels above for large grids, all species: a workgroup takes 32 x
+// 8 cells of a plane and fetches a species' values once, its own by every
+// thread and the R cells around the tile by most; the xi and eta taps come
+// from LDS.  With every tap a load of its own the kernels were bound by the
+// address and data path of the vector cache (19 loads a species and cell, and
+// each wavefront load of 512 bytes off a line's start takes twice the cycles).
+// The next species' values are in flight while this one's are used; two
+// buffers, so one barrier a species.  Tiles in the order of bricks
+// (brick_cell), so that the planes of the zeta taps are in the L2 together.
+// 160x112x64, nine species, us before / now: viscous preparation 303 / 197,
+// update 240 / 145 (of which the order of the tiles is about a tenth).
+constexpr int ST_X = 32, ST_Y = 8;
+template <int R>
+struct SpeciesTile {
+  static constexpr int LX = ST_X + 2 * R, LY = ST_Y + 2 * R, NH = 2 * R * (ST_X + ST_Y), NT = (NH + 255) / 256;
+  int i, j, k;
+  bool act;            // a cell of the grid
+  long own;            // source of the thread's position (periodic images included), -1: none
+  long src[NT];        // ... of its positions around the tile: eta below ST_X * 2 R, then xi
+  int pos[NT];         // their places in an LY x LX array
+  __device__ __forceinline__ void init(const DevState& S) {
+    const int nti = (S.nx + ST_X - 1) / ST_X, ntj = (S.ny + ST_Y - 1) / ST_Y;
+    const int lb = (int)xcd_block((long)blockIdx.x, (long)gridDim.x);
+    const int zg = lb / (nti * ntj * BRICK_Z), r = lb - zg * (nti * ntj * BRICK_Z);
+    const int zc = min(BRICK_Z, S.nz - zg * BRICK_Z);
+    const int tj = r / (nti * zc), r2 = r - tj * (nti * zc), kk = r2 / nti;
+    k = zg * BRICK_Z + kk + 1;
+    const int i0 = (r2 - kk * nti) * ST_X + 1, j0 = tj * ST_Y + 1;
+    auto source = [&](int a, int b) {
+      const int ii = wrap(a, S.nx, S.per[0]), jj = wrap(b, S.ny, S.per[1]);
+      return ii >= 1 && ii <= S.nx && jj >= 1 && jj <= S.ny ? iq(S, ii, jj, k) : -1L;
+    };
+    const int lx = (int)threadIdx.x % ST_X, ly = (int)threadIdx.x / ST_X;
+    i = i0 + lx;
+    j = j0 + ly;
+    act = i <= S.nx && j <= S.ny;
+    own = source(i, j);
+#pragma unroll
+    for (int a = 0; a < NT; a++) {
+      const int e = (int)threadIdx.x + 256 * a;
+      int x, y;
+      if (e < 2 * R * ST_X) {
+        const int h = e / ST_X;
+        x = e % ST_X;
+        y = h < R ? h - R : ST_Y + h - R;
+      } else {
+        const int f = e - 2 * R * ST_X, h = f % (2 * R);
+        y = f / (2 * R);
+        x = h < R ? h - R : ST_X + h - R;
+      }
+      src[a] = e < NH ? source(i0 + x, j0 + y) : -1L;
+      pos[a] = (y + R) * LX + x + R;
+    }
+  }
+  __device__ __forceinline__ static bool eta_item(int a) { return (int)threadIdx.x + 256 * a < 2 * R * ST_X; }
+  __device__ __forceinline__ static int place() {
+    return ((int)threadIdx.x / ST_X + R) * LX + (int)threadIdx.x % ST_X + R;
+  }
+};
+inline dim3 species_tiles(const DevState& S) {
+  return dim3((unsigned)((long)((S.nx + ST_X - 1) / ST_X) * ((S.ny + ST_Y - 1) / ST_Y) * S.nz));
+}
+
+// the zeta taps -R .. R of the field at C, ahead of their use (central cells)
+template <int CD, int R>
+__device__ __forceinline__ void zeta_taps(const double* C, long st, double* z) {
+#pragma unroll
+  for (int o = -R; o <= R; o++)
+    if (o != 0) z[o + R] = C[o * st];
+}
+
+template <int CD>
+__global__ __launch_bounds__(256) void k_species_visc_tile(DevState S) {
+  constexpr int R = CD == 1 ? 4 : 3;
+  typedef SpeciesTile<R> Tile;
+  __shared__ double sC[2][Tile::LY * Tile::LX];
+  Tile t;
+  t.init(S);
+  const int i = t.i, j = t.j, k = t.k, at = Tile::place();
+  // lanes beyond the grid compute on the plane's first cell and write nothing
+  const long ni = S.ni, c = t.act ? t.own : iq(S, 1, 1, k), q = t.act ? hq(S, i, j, k) : hq(S, 1, 1, k);
+  const bool ix = wave_all(!t.act || S.per[0] || central_cell(i, S.nx, R));
+  const bool iy = wave_all(!t.act || S.per[1] || central_cell(j, S.ny, R));
+  const bool iz = central_cell(k, S.nz, R);
+  const double T0 = S.T[q], d0 = S.d[q];
+  const double Akx = S.Akx[q], Aky = S.Aky[q], Akz = S.Akz[q];
+  const double Aix = S.Aix[q], Aiy = S.Aiy[q], Aiz = S.Aiz[q];
+  const double Asx = S.Asx[q], Asy = S.Asy[q], Asz = S.Asz[q];
+  const double Akx1 = S.Akx1[q], Aky1 = S.Aky1[q], Akz1 = S.Akz1[q];
+  const double Aix1 = S.Aix1[q], Aiy1 = S.Aiy1[q], Aiz1 = S.Aiz1[q];
+  const double Asx1 = S.Asx1[q], Asy1 = S.Asy1[q], Asz1 = S.Asz1[q];
+  double own = 0.0, halo[Tile::NT];
+  auto fetch = [&](int m) {
+    const double* F = S.cs + (long)m * ni;
+    own = t.own >= 0 ? F[t.own] : 0.0;
+#pragma unroll
+    for (int a = 0; a < Tile::NT; a++) halo[a] = t.src[a] >= 0 ? F[t.src[a]] : 0.0;
+  };
+  fetch(0);
+  double Qx = 0.0, Qy = 0.0, Qz = 0.0;
+  for (int m = 0; m < S.ns; m++) {
+    double* B = sC[m & 1];
+    B[at] = own;
+#pragma unroll
+    for (int a = 0; a < Tile::NT; a++)
+      if ((int)threadIdx.x + 256 * a < Tile::NH) B[t.pos[a]] = halo[a];
+    if (m + 1 < S.ns) fetch(m + 1);
+    const double* C = S.cs + (long)m * ni + c;
+    double z[2 * R + 1];
+    if (iz) zeta_taps<CD, R>(C, S.si[2], z);
+    const double AmD = S.AmD[c + (long)m * ni];
+    __syncthreads();
+    auto tx = [&](int o) { return B[at + o]; };
+    auto ty = [&](int o) { return B[at + o * Tile::LX]; };
+    const double uk = ix ? deriv1<CD, true>(S, 0, i, tx) : deriv1<CD>(S, 0, i, tx);
+    const double ui = iy ? deriv1<CD, true>(S, 1, j, ty) : deriv1<CD>(S, 1, j, ty);
+    const double us = iz ? deriv1<CD, true>(S, 2, k, [&](int o) { return z[o + R]; })
+                         : deriv1<CD>(S, 2, k, [&](int o) {
+                             const int s = wrap(k + o, S.nz, S.per[2]);
+                             return C[(s - k) * S.si[2]];
+                           });
+    const double dD = d0 * AmD;
+    const double hi = gas_hi(m, T0);
+    const double cix = uk * Akx + ui * Aix + us * Asx;
+    const double ciy = uk * Aky + ui * Aiy + us * Asy;
+    const double ciz = uk * Akz + ui * Aiz + us * Asz;
+    const double E1 = dD * cix, E2 = dD * ciy, E3 = dD * ciz;
+    Qx = Qx + E1 * hi;
+    Qy = Qy + E2 * hi;
+    Qz = Qz + E3 * hi;
+    if (t.act) {
+      S.Evs[c + (long)(3 * m) * ni] = E1 * Akx1 + E2 * Aky1 + E3 * Akz1;
+      S.Evs[c + (long)(3 * m + 1) * ni] = E1 * Aix1 + E2 * Aiy1 + E3 * Aiz1;
+      S.Evs[c + (long)(3 * m + 2) * ni] = E1 * Asx1 + E2 * Asy1 + E3 * Asz1;
+    }
+  }
+  if (!t.act) return;
+  S.Qp[c] = Qx;
+  S.Qp[c + ni] = Qy;
+  S.Qp[c + 2 * ni] = Qz;
+}
+
+template <int CD>
+__global__ __launch_bounds__(256) void k_species_rk_tile(DevState S, int krk, double dt, int save) {
+  constexpr int R = CD == 1 ? 4 : 3;
+  typedef SpeciesTile<R> Tile;
+  __shared__ double sE[2][2][Tile::LY * Tile::LX];  // the xi and the eta flux
+  Tile t;
+  t.init(S);
+  const int i = t.i, j = t.j, k = t.k, at = Tile::place();
+  // lanes beyond the grid compute on the plane's first cell and write nothing
+  const long ni = S.ni, c = t.act ? t.own : iq(S, 1, 1, k), q = t.act ? hq(S, i, j, k) : hq(S, 1, 1, k);
+  const bool ix = wave_all(!t.act || S.per[0] || central_cell(i, S.nx, R));
+  const bool iy = wave_all(!t.act || S.per[1] || central_cell(j, S.ny, R));
+  const bool iz = central_cell(k, S.nz, R);
+  const double ajac = S.Ajac[q];
+  const double ra = krk == 2 ? 3.0 / 4.0 : 1.0 / 3.0;
+  const double rb = krk == 2 ? 1.0 / 4.0 : 2.0 / 3.0;
+  double ox = 0.0, oy = 0.0, halo[Tile::NT];
+  auto fetch = [&](int m) {
+    const double* X = S.Evs + (long)(3 * m) * ni;
+    const double* Y = X + ni;
+    ox = t.own >= 0 ? X[t.own] : 0.0;
+    oy = t.own >= 0 ? Y[t.own] : 0.0;
+#pragma unroll
+    for (int a = 0; a < Tile::NT; a++) halo[a] = t.src[a] >= 0 ? (Tile::eta_item(a) ? Y : X)[t.src[a]] : 0.0;
+  };
+  fetch(0);
+  for (int m = 0; m < S.ns; m++) {
+    double(*B)[Tile::LY * Tile::LX] = sE[m & 1];
+    B[0][at] = ox;
+    B[1][at] = oy;
+#pragma unroll
+    for (int a = 0; a < Tile::NT; a++)
+      if ((int)threadIdx.x + 256 * a < Tile::NH) B[Tile::eta_item(a)][t.pos[a]] = halo[a];
+    if (m + 1 < S.ns) fetch(m + 1);
+    const long qm = q + (long)m * S.nh, cm = c + (long)m * ni;
+    const double* Z = S.Evs + (long)(3 * m + 2) * ni + c;
+    double z[2 * R + 1];
+    if (iz) zeta_taps<CD, R>(Z, S.si[2], z);
+    // the stage's old values
+    const double dn = save ? S.di[qm] : krk >= 1 ? S.din[cm] : 0.0;
+    const double dold = krk >= 2 ? S.di[qm] : 0.0;
+    double val = S.dus[cm];
+    __syncthreads();
+    auto tx = [&](int o) { return B[0][at + o]; };
+    auto ty = [&](int o) { return B[1][at + o * Tile::LX]; };
+    const double uk = ix ? deriv1<CD, true>(S, 0, i, tx) : deriv1<CD>(S, 0, i, tx);
+    const double ui = iy ? deriv1<CD, true>(S, 1, j, ty) : deriv1<CD>(S, 1, j, ty);
+    const double us = iz ? deriv1<CD, true>(S, 2, k, [&](int o) { return z[o + R]; })
+                         : deriv1<CD>(S, 2, k, [&](int o) {
+                             const int s = wrap(k + o, S.nz, S.per[2]);
+                             return Z[(s - k) * S.si[2]];
+                           });
+    val = val + (uk + ui + us) * ajac;
+    if (t.act) {
+      if (save) S.din[cm] = dn;
+      if (krk == 0) S.dus[cm] = val;  // right-hand side only
+      else if (krk == 1) S.di[qm] = dn + dt * val;
+      else S.di[qm] = ra * dn + rb * (dold + dt * val);
+    }
+  }
+}
+
 // Rescaling_di (Comput_flow_variables.f90:101-121) and comput_T_P (:32-46)
 // of one cell, given the new density and internal energy.
 __device__ __forceinline__ void ms_prims(const DevState& S, long q, double dd, double Et, double& T, double& p) {
