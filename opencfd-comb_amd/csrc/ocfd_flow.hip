@@ -2731,11 +2731,11 @@ void enq_stage(int krk, double dt1) {
 // four wavefronts would do all of them: the species follow one another
 // otherwise, and a small grid has too few wavefronts to cover their latency.
 // Every share repeats the work on the point itself (metrics, masks, split
-// velocity), so a large grid takes one.  us per RK3 step with 1 / 2 / 3
-// shares, jets: 48x36x36 (243 blocks of cells) 812 / 642 / 615, 64x48x40 (480)
-// 950 / 851 / 888, 80x56x48 (840) 1415 / 1332 / 1348, 96x64x56 (1344) 1941 /
-// 1940 / 1975, 160x112x64 (4480) 5397 / 5407 / 5535.
-int species_groups(long blocks, int nm) { return blocks >= 1344 ? 1 : std::min(nm, blocks >= 400 ? 2 : 3); }
+// velocity), so other grids take one, and the LDS tiles.  us per RK3 step with
+// 1 / 2 / 3 shares, jets: 48x36x36 (243 blocks of cells) 670 / 594 / 577,
+// 64x48x40 (480) 745 / 815 / 821, 80x56x48 (840) 1085 / 1178 / 1223,
+// 160x112x64 (4480) 4365 / 5094 / 5150.
+int species_groups(long blocks, int nm) { return blocks >= 400 ? 1 : std::min(nm, 3); }
 
 template <int DIR>
 void launch_species_sweep(hipStream_t st, int m0, int m1) {
