@@ -446,7 +446,8 @@ int32_t ocfd_chem_timeadv_batch(int64_t n, double* rho, double* E, const double*
  * not reached dt by then counts as unfinished (ocfd_chem_unfinished).
  * nsub_out [n] (device, may be NULL) receives the accepted substeps per
  * cell.  scheduler 0: one cell per thread; 1: a persistent kernel whose
- * lanes take cells from a device work queue; 2: the work queue, where a cell
+ * lanes take cells from a device work queue, and whose wavefronts finish
+ * their last cells one at a time with all lanes; 2: the work queue, where a cell
  * still running after a budget of attempts (OCFD_CHEM_OPT_COOP_BUDGET) moves
  * to a cooperative kernel that
  * integrates one cell per wavefront (lower latency for the few cells that
@@ -472,7 +473,8 @@ int32_t ocfd_chem_adaptive_batch_noalloc(int64_t n, double* rho, double* E, cons
 
 /* Chemistry options: OCFD_CHEM_OPT_COOP_BUDGET = attempts a cell may take on
  * one lane before scheduler 2 moves it to the cooperative kernel (default
- * 128, the fastest of 16..1024 on a 2^21-cell jet-flame batch);
+ * 128, within a few percent of the fastest on a 2^21-cell jet-flame batch;
+ * smaller batches gain from less);
  * OCFD_CHEM_OPT_FALLBACK_SCHEDULER = scheduler (1 or 2) of the
  * surrogate's fallback (default 2); OCFD_CHEM_OPT_COOP_DIRECT_MAX = a
  * fallback list of at most this many cells hands every cell that needs more

@@ -186,15 +186,25 @@ __device__ __forceinline__ long xcd_block(long b, long nb) {
   const long x = b & 7, r = b >> 3;
   return x * q + (x < rem ? x : rem) + r;
 }
+// linear cell index of this thread for a 1-D launch of 256-thread blocks
+__device__ __forceinline__ long cell_index() {
+  return xcd_block((long)blockIdx.x, (long)gridDim.x) * blockDim.x + threadIdx.x;
+}
 // Cell of this thread for a launch of brick_blocks(S) blocks of 256 threads: a
 // plane's cells in blocks of 256, and the blocks in bricks of about BRICK_R
 // rows and BRICK_Z planes, so that what an XCD has in flight, some 25,000
 // cells, is a compact body whose eta and zeta taps meet in its L2 (in plane
 // order the planes of a zeta tap lie 3 x 8 MB of other arrays apart).  S.ni
-// where there is none.
+// where there is none.  Grids of up to 2^18 cells keep the linear order: they
+// gain nothing (64^3), and the divisions here cost a small grid 2 us a stage
+// (32^3 114 us per step, 120 in bricks; 161x61x33 518 linear, 506 in bricks).
 constexpr int BRICK_R = 8, BRICK_Z = 16;
-inline long brick_blocks(const DevState& S) { return ((long)S.nx * S.ny + 255) / 256 * S.nz; }
+constexpr long BRICK_CELLS = 1L << 18;
+inline long brick_blocks(const DevState& S) {
+  return S.ni > BRICK_CELLS ? ((long)S.nx * S.ny + 255) / 256 * S.nz : (S.ni + 255) / 256;
+}
 __device__ __forceinline__ long brick_cell(const DevState& S) {
+  if (S.ni <= BRICK_CELLS) return cell_index();
   const int P = S.nx * S.ny, np = (P + 255) >> 8;
   const int B = max(1, (BRICK_R * S.nx + 128) >> 8);
   const int lb = (int)xcd_block((long)blockIdx.x, (long)gridDim.x);
@@ -202,10 +212,6 @@ __device__ __forceinline__ long brick_cell(const DevState& S) {
   const int bg = r / (B * zc), r2 = r - bg * (B * zc), bc = min(B, np - bg * B);
   const int k = r2 / bc, pc = (bg * B + (r2 - k * bc)) * 256 + (int)threadIdx.x;
   return pc < P ? (long)(zg * BRICK_Z + k) * P + pc : S.ni;
-}
-// linear cell index of this thread for a 1-D launch of 256-thread blocks
-__device__ __forceinline__ long cell_index() {
-  return xcd_block((long)blockIdx.x, (long)gridDim.x) * blockDim.x + threadIdx.x;
 }
 
 // ---------------------------------------------------------------------------

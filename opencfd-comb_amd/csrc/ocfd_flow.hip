@@ -2731,11 +2731,15 @@ void enq_stage(int krk, double dt1) {
 // four wavefronts would do all of them: the species follow one another
 // otherwise, and a small grid has too few wavefronts to cover their latency.
 // Every share repeats the work on the point itself (metrics, masks, split
-// velocity), so other grids take one, and the LDS tiles.  us per RK3 step with
-// 1 / 2 / 3 shares, jets: 48x36x36 (243 blocks of cells) 670 / 594 / 577,
-// 64x48x40 (480) 745 / 815 / 821, 80x56x48 (840) 1085 / 1178 / 1223,
-// 160x112x64 (4480) 4365 / 5094 / 5150.
+// velocity), so a large grid takes one.  The viscous preparation and update
+// take three shares below 400 blocks of cells and the LDS tiles above; us per
+// RK3 step, all kernels with 1 / 2 / 3 shares, jets: 48x36x36 (243 blocks of
+// cells, 324 to 432 of sweep tiles) 670 / 594 / 577, 64x48x40 (480) 745 / 815 /
+// 821, 80x56x48 (840) 1085 / 1178 / 1223, 160x112x64 (4480) 4365 / 5094 / 5150.
+// The sweeps alone keep two shares up to 1344 blocks (48x36x36 jet case, 432
+// blocks in y and z: 11.0 ms, 11.3 with one).
 int species_groups(long blocks, int nm) { return blocks >= 400 ? 1 : std::min(nm, 3); }
+int sweep_groups(long blocks, int nm) { return blocks >= 1344 ? 1 : std::min(nm, blocks >= 400 ? 2 : 3); }
 
 template <int DIR>
 void launch_species_sweep(hipStream_t st, int m0, int m1) {
@@ -2743,7 +2747,7 @@ void launch_species_sweep(hipStream_t st, int m0, int m1) {
   constexpr int NP = SpTile<DIR>::NP, TS = SpTile<DIR>::TS;
   const long npen = DIR == 0 ? (long)S.ny * S.nz : DIR == 1 ? (long)S.nx * S.nz : (long)S.nx * S.ny;
   dim3 g((unsigned)((S.n[DIR] + TS - 1) / TS), (unsigned)((npen + NP - 1) / NP));
-  const int ns = species_groups((long)g.x * g.y, m1 - m0), ng = (m1 - m0 + ns - 1) / ns;
+  const int ns = sweep_groups((long)g.x * g.y, m1 - m0), ng = (m1 - m0 + ns - 1) / ns;
   g.z = (unsigned)((m1 - m0 + ng - 1) / ng);
   static const char* names[3] = {"k_species_sweep_x", "k_species_sweep_y", "k_species_sweep_z"};
   launch_s(st, names[DIR], k_species_sweep<DIR>, g, dim3(256), S, m0, m1, ng);
@@ -3083,9 +3087,18 @@ int32_t ocfd_init(const ocfd_cfg* cfg) {
       {&S.Aiz1, nh, 1.0}, {&S.Asx1, nh, 1.0}, {&S.Asy1, nh, 1.0}, {&S.Asz1, nh, 1.0},
       {&S.Rh, nh, 0.0}, {&S.Ev, 12 * ni, 0.0}, {&S.red, 8, 0.0}};
   G.inited = true;  // so that finalize frees partial allocations on error
+  // one allocation for all of them, every array on a 2 KB boundary: an
+  // allocation and its release cost about 2 ms each, and the address
+  // translations of neighbouring arrays are larger (640x120x64, 16 steps with
+  // their copies: 105.1 ms with an allocation an array, 100.5 so)
+  long words = 0;
+  auto padded = [](long n) { return (std::max(n, 1L) + 255) / 256 * 256; };
+  for (auto& a : arrs) words += padded(a.n);
+  double* base = dalloc(words);
+  if (!base) return fail("ocfd_init: hipMalloc failed");
   for (auto& a : arrs) {
-    *a.p = dalloc(a.n);
-    if (!*a.p) return fail("ocfd_init: hipMalloc failed");
+    *a.p = base;
+    base += padded(a.n);
     if (a.n > 0) hipLaunchKernelGGL(k_fill, grid1(a.n), dim3(256), 0, G.stream, *a.p, a.n, a.v);
   }
   for (int d = 0; d < 3; d++) {
