@@ -2829,7 +2829,7 @@ void enq_stage_ms(int krk, double dt1) {
   const DevState& S = G.S;
   launch_transport_ms(krk == 1 ? 1 : 0, S.viscous);
   if (krk == 1 && G.cfg.scheme_invis == OCFD_SCHEME_HYBRID) enq_rhybrid();
-  // the species chain (sweeps, concentrations, diffusion, update of di) on
+  // the species chain (sweeps, diffusion, update of di) on
   // the second stream beside the flow sweeps, which read no di; the flow's
   // viscous preparation waits for Qp, k_rk (Rescaling_di) for the whole chain
   const hipStream_t sp = fork_side();
