@@ -3156,7 +3156,8 @@ int32_t ocfd_init(const ocfd_cfg* cfg) {
   const long nup = 6L * (blbc && S.bl_upper == 2 ? (long)S.nx * S.nz : blbc && S.bl_upper == 1 ? (long)S.nx : 1L);
   G.bl_nin = nin;
   G.bl_nup = nup;
-  double* bl = dalloc(nin + nup + (long)S.nx * S.nz);
+  const long nbl = nin + nup + (long)S.nx * S.nz;
+  double* bl = dalloc(nbl);
   void* nr = nullptr;
   if (!G.part || !bl || hipMalloc(&nr, sizeof(int) * (size_t)S.nx * S.nz) != hipSuccess) return fail("ocfd_init: hipMalloc failed");
   G.allocs.push_back(nr);
@@ -3171,8 +3172,7 @@ int32_t ocfd_init(const ocfd_cfg* cfg) {
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, G.stream, htp, 1L, 1.0);
     S.bl_ht = htp;
   }
-  hipLaunchKernelGGL(k_fill, grid1(nin + nup + (long)S.nx * S.nz), dim3(256), 0, G.stream, bl,
-                     (long)S.ny * 6 + 6 + (long)S.nx * S.nz, 0.0);
+  hipLaunchKernelGGL(k_fill, grid1(nbl), dim3(256), 0, G.stream, bl, nbl, 0.0);
   if (hipHostMalloc((void**)&G.h_negt, sizeof(int)) != hipSuccess) return fail("ocfd_init: hipHostMalloc failed");
   *G.h_negt = 0;
   {
