@@ -2965,6 +2965,8 @@ int32_t ocfd_finalize(void) {
   return 0;
 }
 
+static int upload_gas();
+
 int32_t ocfd_init(const ocfd_cfg* cfg) {
   ocfd_finalize();
   G.err.clear();
@@ -3195,6 +3197,12 @@ int32_t ocfd_init(const ocfd_cfg* cfg) {
     S.mt_zj = t + 2 * nxy + 2 * nxz + nyz;
     S.mt_on = 0;
     G.mt_valid = false;
+  }
+  // The kernels' species loops run to the bank's count (each_species) and
+  // write DI: the count of an earlier context must not outlive it.
+  if (S.ns > 1 && G.hg.ns != S.ns) {
+    G.hg.ns = S.ns;
+    if (upload_gas()) return 1;
   }
   HIPCHK(hipStreamSynchronize(G.stream));
   return 0;
