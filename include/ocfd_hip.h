@@ -118,9 +118,9 @@ enum {
   OCFD_OPT_KERNEL_TIMING = 3,
   /* k planes walked by one block of the viscous-flux and update kernels
    * (their z-stencil windows stay in registers); 0 = one thread per cell;
-   * -1 (default) = 4 for N_SPEC = 1 (up to 2^19 cells of a viscous run:
-   * sweeps and viscous preparation in one launch, one thread per cell), one
-   * thread per cell for N_SPEC > 1.
+   * -1 (default) = 4 for N_SPEC = 1 above 2^19 cells, one thread per cell
+   * below (a viscous run's step: sweeps and viscous preparation in one
+   * launch) and for N_SPEC > 1.
    * Results are bitwise independent of the value. */
   OCFD_OPT_COLUMN_PLANES = 4,
   /* 1 (default) = the viscous-flux preparation of each stage runs on a

@@ -2472,11 +2472,27 @@ inline long ghost_count(int f) {
   return (long)OCFD_LAP * (dir == 0 ? S.ny : S.nx) * (dir == 2 ? S.ny : S.nz);
 }
 
+// Grids up to this many cells take the small grid's stage (k_stage).  us per
+// RK3 step, k_stage / separate launches, on periodic boxes: 48^3 253 / 348,
+// 64^3 504 / 535, 80^3 946 / 976, 88^3 1201 / 1184, 96^3 1473 / 1412; on
+// plates: 161x61x33 605 / 678, 200x61x40 844 / 900, 240x81x33 (642,000
+// cells) 1163 / 1165, 320x80x33 1443 / 1365 (before kernarg_again took a
+// tenth off the first).  Above the line the update's
+// 80 B a cell more outweigh the ramps and gaps saved.  Only the default tiles
+// have a form in k_stage, and a timed run shows the kernels one by one.
+constexpr long SMALL_CELLS = 1L << 19;
+
 // Planes per block of the marching kernels.  Automatic choice: 4 for N_SPEC
-// = 1; one thread per cell for N_SPEC > 1, whose per-cell bodies (species
+// = 1 on grids above SMALL_CELLS; one thread per cell below, where blocks of
+// four planes are too few to cover their latency (the stage entries' RK3 step
+// with 4 planes / one thread per cell, us: box 16^3 384 / 258, 32^3 373 / 275,
+// 64^3 647 / 570, 80^3 1182 / 999, plate 161x61x33 759 / 679; a step of the
+// 256x96x64 plate 2038 / 2058), and for N_SPEC > 1, whose per-cell bodies (species
 // loops, Rescaling_di, Newton temperature) leave no registers for the z
 // windows (measured on a 256x192x128 jet: 1.26 vs 1.09 ms per k_rk launch).
-inline int col_planes() { return G.col_planes >= 0 ? G.col_planes : (G.S.ns > 1 ? 0 : 4); }
+inline int col_planes() {
+  return G.col_planes >= 0 ? G.col_planes : (G.S.ns > 1 || G.S.ni <= SMALL_CELLS ? 0 : 4);
+}
 
 // k_rk with the viscous scheme and (for the stepping path's flag sets) the
 // flags fixed at compile time, flat or marching
@@ -2621,15 +2637,6 @@ void enq_sweeps() {
   G.du_parts = false;
 }
 
-// Grids up to this many cells take the small grid's stage (k_stage).  us per
-// RK3 step, k_stage / separate launches, on periodic boxes: 48^3 253 / 348,
-// 64^3 504 / 535, 80^3 946 / 976, 88^3 1201 / 1184, 96^3 1473 / 1412; on
-// plates: 161x61x33 605 / 678, 200x61x40 844 / 900, 240x81x33 (642,000
-// cells) 1163 / 1165, 320x80x33 1443 / 1365 (before kernarg_again took a
-// tenth off the first).  Above the line the update's
-// 80 B a cell more outweigh the ramps and gaps saved.  Only the default tiles
-// have a form in k_stage, and a timed run shows the kernels one by one.
-constexpr long SMALL_CELLS = 1L << 19;
 bool small_stage() {
   return G.S.ns == 1 && G.S.viscous && G.S.ni <= SMALL_CELLS && !G.cfg.if_scheme_character && !G.timing &&
          G.col_planes < 0 && G.sweep_variant[0] == 0 && G.sweep_variant[1] == 0 && G.sweep_variant[2] == 0;
