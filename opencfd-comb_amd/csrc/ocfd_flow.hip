@@ -687,11 +687,13 @@ __global__ __launch_bounds__(256) void k_du_sum(DevState S) {
 
 // Negative-Et bookkeeping (Num_NegT=0, Comput_flow_variables.f90:8): negt[18 +
 // krk] counts the bad cells of stage krk, negt[1..16] lists the first of them,
-// negt[17] is the step's largest count.  Every stage has its own counter, so
-// one reset serves a step: the counter of a stage is read by every block of
-// its boundary kernel, which could not clear it.
+// negt[17] is the step's largest count; negt[21 + krk] counts the blocks of
+// the stage's boundary kernel that came to a repair, negt[24 + krk] tells them
+// that it is done.  Every stage has its own, so one reset serves a step: a
+// stage's words are read by every block of its boundary kernel, which could
+// not clear them.
 __device__ __forceinline__ void negt_reset(const DevState& S, int step) {
-  for (int krk = 1; krk <= 3; krk++) S.negt[18 + krk] = 0;
+  for (int krk = 1; krk <= 3; krk++) S.negt[18 + krk] = S.negt[21 + krk] = S.negt[24 + krk] = 0;
   if (step) S.negt[17] = 0;
 }
 
@@ -1598,65 +1600,73 @@ __device__ __forceinline__ void bc_conditions(int k) {
   }
 }
 
+// The repair of stage krk before any face is done (a bad cell may lie beside
+// one), once for all blocks of the boundary kernel.  The block that comes
+// first does it and the others wait for it.  The one they wait for is running
+// and waits for nobody, so every wait ends, in whatever order blocks start.
+template <bool MS>
+__device__ __forceinline__ void negt_repair_first(const DevState& S, int krk, int* idx) {
+  if (threadIdx.x == 0) {
+    int* done = S.negt + 24 + krk;
+    if (atomicAdd(S.negt + 21 + krk, 1) == 0) {
+      negt_repair<MS>(S, krk, idx);
+      __hip_atomic_store(done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      while (__hip_atomic_load(done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == 0) __builtin_amdgcn_s_sleep(8);
+    }
+  }
+  __syncthreads();
+}
+
 // All of a stage's boundary conditions in one launch: a block per k plane,
 // then blocks over the middle of the two k faces.  It also opens with the
-// negative-Et repair of stage krk (0: none to do).  That is rare, and a cell
-// may lie beside a face: if stage krk counted any, the first block repairs
-// them and does all the rest by itself.
+// negative-Et repair of stage krk (0: none to do), which is rare.
 // Few cells, many dependent loads: bound by latency and, as launches of their
 // own (reset, repair, inlet, upper, wall, outlet, faces), by the 4 to 5 us
 // that each takes from start to start.  us a stage, before / after: boundary
 // layer 161x61x33 31 / 15, round jet 48x36x36 59 / 24, periodic box 32^3
-// 17 / 5.
+// 17 / 5.  A stage with a bad cell on a 256x96x64 plate takes 18 us more than
+// one without (870 us with all faces left to the block that repairs).
 __host__ __device__ inline long bc_mid_cells(const DevState& S) { return 2L * (S.nx - 5) * (S.ny - 4); }
 template <int BC, bool MS>
 __global__ __launch_bounds__(BC_NT) void k_bc(DevState S, int krk) {
   __shared__ int idx[16];
   const int nx = S.nx, ny = S.ny, nz = S.nz;
   const int mx = nx - 5, my = ny - 4;  // the middle of a k face
-  const bool bad = krk > 0 && S.negt[18 + krk] != 0;
-  if (bad) {
-    if (blockIdx.x != 0) return;
-    if (threadIdx.x == 0) negt_repair<MS>(kernarg_again(), krk, idx);
-    __syncthreads();
+  if (krk > 0 && S.negt[18 + krk] != 0) negt_repair_first<MS>(kernarg_again(), krk, idx);
+  const int b = (int)blockIdx.x;
+  const int k = b + 1;  // the plane of a block below nz
+  const bool mid = b >= nz, kface = k == 1 || k == nz;
+  const long m0 = (long)(b - nz) * BC_NT;
+  long n;
+  if (!mid) {
+    bc_conditions<BC>(k);
+    // a k face: the rows and columns that the conditions write or read (rows
+    // 1-3 and ny, columns 1-2 and nx-2..nx); the last blocks do the rest
+    n = kface ? 4 * nx + 5 * (ny - 4) : 2 * ny + 2 * (nx - 2);
+  } else {
+    n = min((long)BC_NT, 2L * mx * my - m0);
   }
-  const int b1 = bad ? (int)gridDim.x : (int)blockIdx.x + 1;
 #pragma unroll 1
-  for (int b = (int)blockIdx.x; b < b1; b++) {
-    const int k = b + 1;  // the plane of a block below nz
-    const bool mid = b >= nz, kface = k == 1 || k == nz;
-    const long m0 = (long)(b - nz) * BC_NT;
-    long n;
-    if (!mid) {
-      bc_conditions<BC>(k);
-      // a k face: the rows and columns that the conditions write or read (rows
-      // 1-3 and ny, columns 1-2 and nx-2..nx); the last blocks do the rest
-      n = kface ? 4 * nx + 5 * (ny - 4) : 2 * ny + 2 * (nx - 2);
+  for (int t = (int)threadIdx.x; t < n; t += BC_NT) {
+    int i, j, kk = k;
+    if (mid) {
+      const long c = m0 + t, l = c / mx;
+      i = (int)(c - l * mx) + 3;
+      kk = l < my ? 1 : nz;
+      j = (int)(l < my ? l : l - my) + 4;
+    } else if (kface) {
+      if (t < 4 * nx) { i = t % nx + 1; j = t / nx + 1; if (j == 4) j = ny; }
+      else { const int r = t - 4 * nx, a = r % 5; j = r / 5 + 4; i = a < 2 ? a + 1 : nx - 4 + a; }
+    } else if (t < 2 * ny) {
+      i = t < ny ? 1 : nx;
+      j = (t < ny ? t : t - ny) + 1;
     } else {
-      n = min((long)BC_NT, 2L * mx * my - m0);
+      const int r = t - 2 * ny;
+      j = r < nx - 2 ? 1 : ny;
+      i = (r < nx - 2 ? r : r - (nx - 2)) + 2;
     }
-#pragma unroll 1
-    for (int t = (int)threadIdx.x; t < n; t += BC_NT) {
-      int i, j, kk = k;
-      if (mid) {
-        const long c = m0 + t, l = c / mx;
-        i = (int)(c - l * mx) + 3;
-        kk = l < my ? 1 : nz;
-        j = (int)(l < my ? l : l - my) + 4;
-      } else if (kface) {
-        if (t < 4 * nx) { i = t % nx + 1; j = t / nx + 1; if (j == 4) j = ny; }
-        else { const int r = t - 4 * nx, a = r % 5; j = r / 5 + 4; i = a < 2 ? a + 1 : nx - 4 + a; }
-      } else if (t < 2 * ny) {
-        i = t < ny ? 1 : nx;
-        j = (t < ny ? t : t - ny) + 1;
-      } else {
-        const int r = t - 2 * ny;
-        j = r < nx - 2 ? 1 : ny;
-        i = (r < nx - 2 ? r : r - (nx - 2)) + 2;
-      }
-      face_cell<MS>(kernarg_again(), i, j, kk);
-    }
-    if (bad) __syncthreads();
+    face_cell<MS>(kernarg_again(), i, j, kk);
   }
 }
 
@@ -2703,13 +2713,12 @@ void enq_rhybrid() {
 void enq_bc(int krk) {
   const DevState& S = G.S;
   const dim3 grid((unsigned)(S.nz + (bc_mid_cells(S) + BC_NT - 1) / BC_NT));
-  const bool ms = S.ns > 1;
-  if (G.cfg.ibc == OCFD_BC_BOUNDARYLAYER)
-    launch("k_bc", ms ? k_bc<OCFD_BC_BOUNDARYLAYER, true> : k_bc<OCFD_BC_BOUNDARYLAYER, false>, grid, dim3(BC_NT), S, krk);
-  else if (G.cfg.ibc == OCFD_BC_JET)
-    launch("k_bc", ms ? k_bc<OCFD_BC_JET, true> : k_bc<OCFD_BC_JET, false>, grid, dim3(BC_NT), S, krk);
-  else
-    launch("k_bc", ms ? k_bc<0, true> : k_bc<0, false>, grid, dim3(BC_NT), S, krk);
+  // (ocfd_init: the boundary layer has one species, the jet several)
+  const auto kern = G.cfg.ibc == OCFD_BC_BOUNDARYLAYER ? k_bc<OCFD_BC_BOUNDARYLAYER, false>
+                    : G.cfg.ibc == OCFD_BC_JET         ? k_bc<OCFD_BC_JET, true>
+                    : S.ns > 1                         ? k_bc<0, true>
+                                                       : k_bc<0, false>;
+  launch("k_bc", kern, grid, dim3(BC_NT), S, krk);
   for (int f = 0; f < 6; f++)  // Flow_Ghost_boundary, OCFD_BC.f90:186
     if (G.cfg.ghost_cell[f] == 1 || G.cfg.ghost_cell[f] == 2)
       launch("k_flow_ghost", k_flow_ghost, grid1(ghost_count(f)), dim3(256), S, f);
