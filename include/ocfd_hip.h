@@ -378,9 +378,12 @@ int32_t ocfd_ana_box(double* out);
  * The inviscid sweeps come in several workgroup tile shapes (pencils per
  * workgroup x cells per pencil).  ocfd_autotune times each shape per
  * direction on the current state with HIP events (reps launches each) and
- * keeps the fastest; ocfd_set_tile forces one.  Results are bit-identical
- * for every shape.  ocfd_tile_choice returns the chosen variant index and
- * its shape, and the measured ms per launch of every variant (4 floats). */
+ * keeps the fastest; ocfd_set_tile forces one.  A step of a viscous N_SPEC =
+ * 1 run of up to 2^19 cells has its sweeps in one launch with the default
+ * shapes whatever the tuner chose; ocfd_set_tile of another shape takes the
+ * separate launches there too.  Results are bit-identical for every shape.
+ * ocfd_tile_choice returns the chosen variant index and its shape, and the
+ * measured ms per launch of every variant (4 floats). */
 int32_t ocfd_autotune(int32_t reps);
 int32_t ocfd_set_tile(int32_t dir, int32_t variant);
 int32_t ocfd_tile_choice(int32_t dir, int32_t* np, int32_t* ts, float* ms_per_variant);

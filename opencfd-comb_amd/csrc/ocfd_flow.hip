@@ -2367,6 +2367,7 @@ struct Ctx {
   double hyb_eta0 = 0.0;      // certificate band before OCFD_OPT_HYBRID_CERT_WIDEN
   bool hyb_cert_ran = false;
   int sweep_variant[3] = {0, 0, 0};
+  bool tile_asked[3] = {false, false, false};  // by ocfd_set_tile, not the tuner
   float tune_ms[3][8] = {};
   int col_planes = -1;    // k planes per block of the marching kernels (0: one thread per cell, -1: auto)
   unsigned short* kc[3] = {nullptr, nullptr, nullptr};  // sweep kind lists per direction
@@ -2489,7 +2490,12 @@ inline long ghost_count(int f) {
 // cells) 1163 / 1165, 320x80x33 1443 / 1365 (before kernarg_again took a
 // tenth off the first).  Above the line the update's
 // 80 B a cell more outweigh the ramps and gaps saved.  Only the default tiles
-// have a form in k_stage, and a timed run shows the kernels one by one.
+// have a form in k_stage: a shape that ocfd_set_tile asks for takes the
+// separate launches, one that the tuner prefers is theirs only: the tuner times
+// a sweep by itself, and the one launch stays the faster (us a step, k_stage /
+// separate launches with the tuner's shapes: 64^3 441 / 476, 72^3 566 / 619,
+// 80^3 847 / 859).
+// A timed run shows the kernels one by one.
 constexpr long SMALL_CELLS = 1L << 19;
 
 // Planes per block of the marching kernels.  Automatic choice: 4 for N_SPEC
@@ -2648,8 +2654,10 @@ void enq_sweeps() {
 }
 
 bool small_stage() {
+  for (int d = 0; d < 3; d++)
+    if (G.tile_asked[d] && G.sweep_variant[d] != 0) return false;
   return G.S.ns == 1 && G.S.viscous && G.S.ni <= SMALL_CELLS && !G.cfg.if_scheme_character && !G.timing &&
-         G.col_planes < 0 && G.sweep_variant[0] == 0 && G.sweep_variant[1] == 0 && G.sweep_variant[2] == 0;
+         G.col_planes < 0;
 }
 
 void enq_small_sweeps(int krk) {
@@ -4022,6 +4030,7 @@ int32_t ocfd_autotune(int32_t reps) {
       if (v == 0 || ms < 0.90f * best) { best = ms; bestv = v; }
     }
     G.sweep_variant[dir] = bestv;
+    G.tile_asked[dir] = false;
   }
   hipEventDestroy(a);
   hipEventDestroy(b);
@@ -4051,6 +4060,7 @@ int32_t ocfd_tile_choice(int32_t dir, int32_t* np, int32_t* ts, float* ms_per_va
 int32_t ocfd_set_tile(int32_t dir, int32_t variant) {
   if (dir < 0 || dir > 2 || variant < 0 || variant >= OCFD_SWEEP_VARIANTS) return fail("ocfd_set_tile: bad argument");
   G.sweep_variant[dir] = variant;
+  G.tile_asked[dir] = true;
   drop_graph();
   return 0;
 }
