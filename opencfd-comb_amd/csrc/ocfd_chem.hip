@@ -794,6 +794,12 @@ int order_list_longest_first(long n, long cap, const int* list, const unsigned l
   return 0;
 }
 
+// the kernels for the mechanism's structure
+template <class F>
+auto chem_kernel(F f) {
+  return CX.h2 ? f(ChemH2{}) : CX.h.rereac != 0 ? f(ChemRev{}) : f(ChemAny{});
+}
+
 // the adaptive integrator over cells 0..n-1, or over list[0 .. *list_count)
 // when list is given; counters [0,1,3,4] must be zero.  scheduler 0: one
 // cell per thread; 1: per-lane work queue; 2: work queue with the cooperative
@@ -805,11 +811,12 @@ int launch_adaptive(long n, double* rho, double* E, const double* dt, const Chem
                     unsigned long long* counter = nullptr) {
   if (!counter) counter = CX.counter;
   if (scheduler == 0 && !list) {
-    hipLaunchKernelGGL(CX.h2 ? k_chem_adaptive<ChemH2> : k_chem_adaptive<ChemAny>, dim3((unsigned)((n + CH_BLOCK - 1) / CH_BLOCK)), dim3(CH_BLOCK), 0, CX.stream, n, rho, E, dt, ctl,
-                       nsub_out, counter);
+    const auto kern = chem_kernel([](auto st) { return &k_chem_adaptive<decltype(st)>; });
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n + CH_BLOCK - 1) / CH_BLOCK)), dim3(CH_BLOCK), 0, CX.stream, n, rho, E, dt,
+                       ctl, nsub_out, counter);
     return hipGetLastError() == hipSuccess ? 0 : cfail("chemistry: launch failed");
   }
-  const auto queue = CX.h2 ? k_chem_queue<ChemH2> : k_chem_queue<ChemAny>;
+  const auto queue = chem_kernel([](auto st) { return &k_chem_queue<decltype(st)>; });
   int dev = 0, ncu = 0, per = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
@@ -824,7 +831,7 @@ int launch_adaptive(long n, double* rho, double* E, const double* dt, const Chem
                      counter, list, list_count, coop ? CX.coop_budget : 0, direct ? CX.coop_direct_max : 0,
                      coop ? CX.heavy : HeavyBuf{});
   if (coop) {
-    const auto coopk = CX.h2 ? k_chem_coop<ChemH2> : k_chem_coop<ChemAny>;
+    const auto coopk = chem_kernel([](auto st) { return &k_chem_coop<decltype(st)>; });
     int per2 = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per2, coopk, 64, 0) != hipSuccess)
       return cfail("chemistry: device query failed");
@@ -1054,10 +1061,10 @@ int32_t ocfd_chem_timeadv_batch(int64_t n, double* rho, double* E, const double*
   if (nsub < 1) return cfail("ocfd_chem_timeadv_batch: nsub must be >= 1");
   dim3 g((unsigned)((n + CH_BLOCK - 1) / CH_BLOCK)), b(CH_BLOCK);
   switch (mode) {
-    case 1: hipLaunchKernelGGL((CX.h2 ? k_chem_fixed<1, ChemH2> : k_chem_fixed<1, ChemAny>), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
-    case 2: hipLaunchKernelGGL((CX.h2 ? k_chem_fixed<2, ChemH2> : k_chem_fixed<2, ChemAny>), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
-    case 3: hipLaunchKernelGGL((CX.h2 ? k_chem_fixed<3, ChemH2> : k_chem_fixed<3, ChemAny>), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
-    case -1: hipLaunchKernelGGL((CX.h2 ? k_chem_fixed<-1, ChemH2> : k_chem_fixed<-1, ChemAny>), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
+    case 1: hipLaunchKernelGGL(chem_kernel([](auto st) { return &k_chem_fixed<1, decltype(st)>; }), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
+    case 2: hipLaunchKernelGGL(chem_kernel([](auto st) { return &k_chem_fixed<2, decltype(st)>; }), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
+    case 3: hipLaunchKernelGGL(chem_kernel([](auto st) { return &k_chem_fixed<3, decltype(st)>; }), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
+    case -1: hipLaunchKernelGGL(chem_kernel([](auto st) { return &k_chem_fixed<-1, decltype(st)>; }), g, b, 0, CX.stream, (long)n, rho, E, dt, nsub); break;
     default: return cfail("ocfd_chem_timeadv_batch: CHEM_TimeAdv must be 1, 2, 3 or -1");
   }
   if (hipGetLastError() != hipSuccess) return cfail("ocfd_chem_timeadv_batch: launch failed");

@@ -109,7 +109,8 @@ __device__ __forceinline__ double ipow(double x, int n) {
 
 // ---------------------------------------------------------------------------
 // Stoichiometry known when the kernels are compiled.  The kernels take it as
-// a template argument: ChemAny reads the bank (any mechanism), ChemH2 is the
+// a template argument: ChemAny reads the bank (any mechanism with Gibbs reverse
+// rates), ChemRev is ChemAny for the other reverse rates, ChemH2 is the
 // structure of the shipped 9-species / 19-reaction H2-O2 mechanism -- which
 // species take part in which reaction, its third bodies and falloffs, and
 // which Arrhenius exponents are zero, two temperature ranges.  The numbers (A, b, E, efficiencies,
@@ -123,11 +124,16 @@ __device__ __forceinline__ double ipow(double x, int n) {
 // 0.037 / 0.096.  Both give the same bits (what is left out adds zeros).
 // ---------------------------------------------------------------------------
 struct ChemAny {
-  static constexpr bool FIXED = false;
+  static constexpr bool FIXED = false, ANYT = false;
   static constexpr int NR = 0, NA = CH_NS, NT = 0;
 };
+// ReReac 1 and 2 give numbers at temperatures that are no ordinary ones (chem_arr);
+// kernels of their own, since the loop for them costs the others up to 5%
+struct ChemRev : ChemAny {
+  static constexpr bool ANYT = true;
+};
 struct ChemH2 {
-  static constexpr bool FIXED = true;
+  static constexpr bool FIXED = true, ANYT = false;
   static constexpr int NR = 19, NA = 8, NT = 2;  // reactions; species 0 .. NA-1 react (N2 does not); T ranges
   // af_type, third body, bits: 1 b0, 2 e0, 4 b1, 8 e1 not zero
   static constexpr int af[NR] = {0, 0, 0, 0, 0, 0, 0, 0, 1, 0, 0, 0, 0, 2, 1, 0, 0, 0, 2};
@@ -245,7 +251,20 @@ __device__ __forceinline__ double chem_arr_s(double a, double b, double e, const
   const double k = a * chem_exp(t.tab, s);
   return fm(k, lo, k);
 }
+// Whether ln T, 1/T and the exponent are ordinary numbers.  They are not for a
+// cell without energy (T = 0), of negative energy or NaN: there the expression
+// itself decides, since T^b exists for whole b and exp(-e/T) is 0 where e/T is
+// infinite.  (The ln T of Gibbs reverse rates makes every rate NaN there, so
+// ReReac = 0 needs no test.)
+__device__ __forceinline__ bool chem_T_ordinary(double T) { return T >= 1.0e-12 && T <= 1.0e300; }
+__device__ __noinline__ double chem_arr_expr(double a, double b, double e, double T) {
+  return a * pow(T, b) * exp(-e / T);
+}
+// ANYT: the temperature may not be an ordinary number
+template <bool ANYT>
 __device__ __forceinline__ double chem_arr(double a, double b, double e, const ChemTp& t) {
+  if constexpr (ANYT)
+    if (!chem_T_ordinary(t.T)) return chem_arr_expr(a, b, e, t.T);
   if (b == 0.0 && e == 0.0) return a;
   return chem_arr_s<true, true>(a, b, e, t);
 }
@@ -294,19 +313,19 @@ __device__ __noinline__ double chem_gibbs_high(Mech m, int i, double T) {
 // (CHEM_reactions.f90:130-197) and the mass-action products of
 // Reaction_rate_and_Matrix (:246-250).  g(i) = G_i / (R T), c(s) =
 // concentration of species s, c(CH_NS) = 1.
-template <class RX, class G, class C>
+template <bool ANYT = false, class RX, class G, class C>
 __device__ __forceinline__ void chem_reaction(RX R, int rereac, const ChemTp& t, G g, C c, double& wf1, double& wr1) {
   double ctrb = 0.0;
   if (R->tb == 1) {
 #pragma unroll
     for (int i = 0; i < CH_NS; i++) ctrb = fm(c(i), R->eff[i], ctrb);
   }
-  const double k1 = chem_arr(R->a0, R->b0, R->e0, t);
+  const double k1 = chem_arr<ANYT>(R->a0, R->b0, R->e0, t);
   double wf, wr;
   if (R->af_type == 0) {
     wf = k1;
   } else {
-    const double k2 = chem_arr(R->a1, R->b1, R->e1, t);
+    const double k2 = chem_arr<ANYT>(R->a1, R->b1, R->e1, t);
     if (R->af_type == 2) wf = k1 + k2;
     else wf = chem_troe(R, k1, k2, ctrb, t);
   }
@@ -320,7 +339,7 @@ __device__ __forceinline__ void chem_reaction(RX R, int rereac, const ChemTp& t,
     if (sgm > 0) wr = wr * ipow(t.rs, sgm);
     else if (sgm < 0) wr = wr * ipow(t.irs, -sgm);
   } else if (rereac == 1) {
-    wr = chem_arr(R->r[0], R->r[1], R->r[2], t);  // Arrhenius reverse rate (:180-181)
+    wr = chem_arr<ANYT>(R->r[0], R->r[1], R->r[2], t);  // Arrhenius reverse rate (:180-181)
   } else {
     // ParkCurveFit (:113-118) with the 1e-30 floor (:182-186)
     const double z = 10000.0 / t.T;
@@ -478,25 +497,34 @@ __device__ __forceinline__ void lane_rates(Mech m, LDS& L, double T, const doubl
     });
     return;
   }
+  auto reactions = [&](auto anyt) {
 #pragma unroll 1
-  for (int k = 0; k < nr; k++) {
-    const CH_CONST ChemRx* R = &m->rx[k];
-    double wf1, wr1;
-    chem_reaction(R, rereac, t, gibbs, conc, wf1, wr1);
-    const double w = wf1 - wr1;
+    for (int k = 0; k < nr; k++) {
+      const CH_CONST ChemRx* R = &m->rx[k];
+      double wf1, wr1;
+      chem_reaction<decltype(anyt)::value>(R, rereac, t, gibbs, conc, wf1, wr1);
+      const double w = wf1 - wr1;
 #pragma unroll
-    for (int i = 0; i < CH_NS; i++) ri[i] = fm(w, R->nu[i], ri[i]);
-    if constexpr (JAC) {
-      const int part = R->part;
+      for (int i = 0; i < CH_NS; i++) ri[i] = fm(w, R->nu[i], ri[i]);
+      if constexpr (JAC) {
+        const int part = R->part;
 #pragma unroll
-      for (int j = 0; j < CH_NS; j++)
-        if ((part >> j) & 1) {
-          const double dA = chem_dA(R->vf[j], R->vr[j], wf1, wr1, L.rc[j][tid]);
+        for (int j = 0; j < CH_NS; j++)
+          if ((part >> j) & 1) {
+            const double dA = chem_dA(R->vf[j], R->vr[j], wf1, wr1, L.rc[j][tid]);
 #pragma unroll
-          for (int i = 0; i < CH_NS; i++) A[i][j] = fm(dA, R->nu[i], A[i][j]);
-        }
+            for (int i = 0; i < CH_NS; i++) A[i][j] = fm(dA, R->nu[i], A[i][j]);
+          }
+      }
+    }
+  };
+  if constexpr (ST::ANYT) {
+    if (__any(!chem_T_ordinary(T))) {
+      reactions(std::true_type{});
+      return;
     }
   }
+  reactions(std::false_type{});
 }
 
 // Gauss elimination with partial pivoting (CHEM_reactions.f90:523-567),
@@ -787,9 +815,14 @@ __device__ __forceinline__ bool coop_attempt(Mech m, CoopLds& L, const double2* 
   for (int i = 0; i < CH_NS; i++) gi[i] = bcast(gl, i);
   __syncthreads();
   double wf1 = 0.0, wr1 = 0.0;
-  if (lane < nr)
-    chem_reaction((const ChemRx*)&L.rx[lane], rereac, tp, [&](int i) { return gi[i]; }, [&](int s) { return L.c[s]; },
-                  wf1, wr1);
+  auto reaction = [&](auto anyt) {
+    chem_reaction<decltype(anyt)::value>((const ChemRx*)&L.rx[lane], rereac, tp, [&](int i) { return gi[i]; },
+                                         [&](int s) { return L.c[s]; }, wf1, wr1);
+  };
+  if (lane < nr) {
+    if (ST::ANYT && !chem_T_ordinary(T)) reaction(std::bool_constant<ST::ANYT>{});
+    else reaction(std::false_type{});
+  }
   double a[CH_NS];
 #pragma unroll
   for (int i = 0; i < CH_NS; i++) a[i] = ri[i] = 0.0;
