@@ -90,6 +90,8 @@ template <int MODE, class ST>
 __global__ __launch_bounds__(CH_BLOCK, MODE == 1 ? 3 : 2) void k_chem_fixed(long n, double* rho, double* Ecell,
                                                                          const double* dtcell, int nsub) {
   __shared__ LaneLds<CH_BLOCK, MODE == -1> L;
+  // the waves that the launch bounds ask for, four SIMDs a CU, fit its LDS
+  static_assert(4 * (MODE == 1 ? 3 : 2) * sizeof(L) <= 160 * 1024, "LDS of a CU");
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   lane_lds_init(L);
   if (c >= n) return;

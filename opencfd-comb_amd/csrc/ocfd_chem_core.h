@@ -430,12 +430,15 @@ __device__ __forceinline__ void chem_reaction_s(const CH_CONST ChemRx* R, const 
 // workgroup: concentrations (the last row holds 1), Gibbs functions, the
 // Jacobian's 1 / ((c + 1e-20) M) and the cell's partial densities.  A
 // reaction reads them by a uniform index, and the registers that they would
-// take are what lets two waves of the implicit kernels share a SIMD.
+// take are what lets two waves of the implicit kernels share a SIMD.  Without
+// JAC the rows rc are not there, and three waves of the Euler kernel fit the
+// LDS (explicit batches of 300,007 cells, five steps, with the rows / without,
+// us: Euler 151 / 136, RK2 539 / 519, RK3 394 / 394).
 template <int NT, bool JAC>
 struct LaneLds {
   static constexpr int N = NT;
   double c[CH_NS + 1][NT], g[CH_NS][NT];
-  double rc[CH_NS][NT];
+  double rc[JAC ? CH_NS : 1][NT];
   double2 tab[CH_EXPN];
 };
 // fills a workgroup's table and constant row (NT = 64: one wavefront, whose
