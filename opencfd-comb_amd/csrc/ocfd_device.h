@@ -169,8 +169,11 @@ __device__ __forceinline__ double jac_at(const DevState& S, long q, int i, int j
 // hoisted to its entry otherwise, far more than the scalar registers hold, and
 // then moves them through vector lanes at every use (k_stage: 7,000 of its
 // 26,000 instructions).
-template <class T = DevState>
-__device__ __forceinline__ const T& kernarg_again() {
+// (The argument says whose state it is, so that only code with a DevState at hand
+// can ask; that kernels have theirs first is checked where they are launched,
+// state_first.)
+template <class T>
+__device__ __forceinline__ const T& kernarg_again(const T&) {
   typedef const __attribute__((address_space(4))) T* Arg;
   Arg p = (Arg)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(p));

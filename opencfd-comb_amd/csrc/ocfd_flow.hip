@@ -15,6 +15,8 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/ocfd_hip.h"
@@ -928,15 +930,15 @@ __global__ __launch_bounds__(256) void k_stage(DevState S0, StageArgs A) {
   if (A.first && b == 0 && threadIdx.x == 0) negt_reset(S0, 1);
   if (b < p0) {
     if (b < A.nb[0])
-      sweep_tile<0, 0, false>(kernarg_again(), U.x, xcd_block(b, A.nb[0]), A.gx[0], A.mode[0], A.kc[0], A.kct[0], kernarg_again().du);
+      sweep_tile<0, 0, false>(kernarg_again(S0), U.x, xcd_block(b, A.nb[0]), A.gx[0], A.mode[0], A.kc[0], A.kct[0], kernarg_again(S0).du);
   } else if (b < p1) {
     if (b - p0 < A.nb[1])
-      sweep_tile<1, 0, false>(kernarg_again(), U.y, xcd_block(b - p0, A.nb[1]), A.gx[1], A.mode[1], A.kc[1], A.kct[1], kernarg_again().duy);
+      sweep_tile<1, 0, false>(kernarg_again(S0), U.y, xcd_block(b - p0, A.nb[1]), A.gx[1], A.mode[1], A.kc[1], A.kct[1], kernarg_again(S0).duy);
   } else if (b < p2) {
     if (b - p1 < A.nb[2])
-      sweep_tile<2, 0, false>(kernarg_again(), U.z, xcd_block(b - p1, A.nb[2]), A.gx[2], A.mode[2], A.kc[2], A.kct[2], kernarg_again().duz);
+      sweep_tile<2, 0, false>(kernarg_again(S0), U.z, xcd_block(b - p1, A.nb[2]), A.gx[2], A.mode[2], A.kc[2], A.kct[2], kernarg_again(S0).duz);
   } else {
-    visc_prep_at<CD, false, MT>(kernarg_again(), xcd_block(b - p2, (long)gridDim.x - p2) * blockDim.x + threadIdx.x);
+    visc_prep_at<CD, false, MT>(kernarg_again(S0), xcd_block(b - p2, (long)gridDim.x - p2) * blockDim.x + threadIdx.x);
   }
 }
 
@@ -1049,12 +1051,12 @@ __global__ __launch_bounds__(256) void k_visc_prep_col(DevState S, int kc) {
       }
       const YTaps yt{ys[b], lane, wv};
       if (xint && yint)
-        visc_prep_cell<CD, MS, true, true, MT>(kernarg_again(), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr, &xt, &yt);
+        visc_prep_cell<CD, MS, true, true, MT>(kernarg_again(S), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr, &xt, &yt);
       else if (yint)
-        visc_prep_cell<CD, MS, false, true, MT>(kernarg_again(), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr,
+        visc_prep_cell<CD, MS, false, true, MT>(kernarg_again(S), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr,
                                                 (const XTaps*)nullptr, &yt);
       else
-        visc_prep_cell<CD, MS, false, false, MT>(kernarg_again(), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr);
+        visc_prep_cell<CD, MS, false, false, MT>(kernarg_again(S), c, q, P.i, P.j, k, zd[0], zd[1], zd[2], zd[3], ctr);
     }
 #pragma unroll
     for (int o = 0; o < W - 1; o++) {
@@ -1289,7 +1291,7 @@ __global__ __launch_bounds__(256) void k_rk(DevState S, int krk, double dt, int 
         zs[m] = deriv1<CD, true>(S, 2, k, [&](int o) { return Fv[4 * o * pli]; });
       }
     }
-    rk_cell<CD, F, true, true, MT>(kernarg_again(), c, q, i, j, k, krk, dt, flags_rt, zs);
+    rk_cell<CD, F, true, true, MT>(kernarg_again(S), c, q, i, j, k, krk, dt, flags_rt, zs);
   } else {
     if (flags & RK_VISC) {
 #pragma unroll
@@ -1301,7 +1303,7 @@ __global__ __launch_bounds__(256) void k_rk(DevState S, int krk, double dt, int 
         });
       }
     }
-    rk_cell<CD, F, false, false, MT>(kernarg_again(), c, q, i, j, k, krk, dt, flags_rt, zs);
+    rk_cell<CD, F, false, false, MT>(kernarg_again(S), c, q, i, j, k, krk, dt, flags_rt, zs);
   }
 }
 
@@ -1354,17 +1356,17 @@ __global__ __launch_bounds__(256, (CD == 0 && F >= 0 && !(F & RK_MS)) ? 2 : 1) v
 #pragma unroll
         for (int m = 0; m < 4; m++) zs[m] = visc ? deriv1<CD>(S, 2, k, [&](int o) { return z[m][o + R]; }) : 0.0;
       }
-      if (xint && yint) rk_cell<CD, F, true, true, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
-      else if (yint) rk_cell<CD, F, false, true, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
-      else rk_cell<CD, F, false, false, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      if (xint && yint) rk_cell<CD, F, true, true, MT>(kernarg_again(S), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      else if (yint) rk_cell<CD, F, false, true, MT>(kernarg_again(S), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      else rk_cell<CD, F, false, false, MT>(kernarg_again(S), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
     } else if (xint && yint && central_cell(k, S.nz, R)) {
 #pragma unroll
       for (int m = 0; m < 4; m++) zs[m] = visc ? deriv1<CD, true>(S, 2, k, [&](int o) { return z[m][o + R]; }) : 0.0;
-      rk_cell<CD, F, true, true, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      rk_cell<CD, F, true, true, MT>(kernarg_again(S), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
     } else {
 #pragma unroll
       for (int m = 0; m < 4; m++) zs[m] = visc ? deriv1<CD>(S, 2, k, [&](int o) { return z[m][o + R]; }) : 0.0;
-      rk_cell<CD, F, false, false, MT>(kernarg_again(), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
+      rk_cell<CD, F, false, false, MT>(kernarg_again(S), c, q, P.i, P.j, k, krk, dt, flags_rt, zs);
     }
 #pragma unroll
     for (int o = 0; o < W - 1; o++)
@@ -1564,18 +1566,18 @@ __device__ __forceinline__ void face_cell(const DevState& S, int i, int j, int k
 // order.  They read and write cells of their own plane only, so a block does
 // them with barriers in between.
 template <int BC>
-__device__ __forceinline__ void bc_conditions(int k) {
+__device__ __forceinline__ void bc_conditions(const DevState& S0, int k) {
   const int t0 = (int)threadIdx.x;
   if (BC == OCFD_BC_BOUNDARYLAYER) {
     {
-      const DevState& S = kernarg_again();
+      const DevState& S = kernarg_again(S0);
       for (int t = t0; t < S.ny; t += BC_NT) bl_inlet(S, t + 1, k);
     }
     __syncthreads();
     {
       // BcData_upper = -1: no upper data; the face keeps its values.  The wall
       // reads rows 2 and 3, which the upper data (row ny >= 8) do not touch.
-      const DevState& S = kernarg_again();
+      const DevState& S = kernarg_again(S0);
       const int nx = S.nx;
       for (int t = t0; t < 2 * nx; t += BC_NT) {
         if (t >= nx) bl_wall(S, t - nx + 1, k);
@@ -1584,13 +1586,13 @@ __device__ __forceinline__ void bc_conditions(int k) {
     }
     __syncthreads();
     {
-      const DevState& S = kernarg_again();
+      const DevState& S = kernarg_again(S0);
       if (S.bl_outlet == 1 || S.bl_outlet == 2)
         for (int t = t0; t < S.ny; t += BC_NT) bl_outlet(S, t + 1, k);
     }
     __syncthreads();
   } else if (BC == OCFD_BC_JET) {
-    const DevState& S = kernarg_again();
+    const DevState& S = kernarg_again(S0);
     const int ny = S.ny;
     for (int t = t0; t < 2 * ny; t += BC_NT) {
       if (t < ny) jet_inlet(S, t + 1, k);
@@ -1633,14 +1635,14 @@ __global__ __launch_bounds__(BC_NT) void k_bc(DevState S, int krk) {
   __shared__ int idx[16];
   const int nx = S.nx, ny = S.ny, nz = S.nz;
   const int mx = nx - 5, my = ny - 4;  // the middle of a k face
-  if (krk > 0 && S.negt[18 + krk] != 0) negt_repair_first<MS>(kernarg_again(), krk, idx);
+  if (krk > 0 && S.negt[18 + krk] != 0) negt_repair_first<MS>(kernarg_again(S), krk, idx);
   const int b = (int)blockIdx.x;
   const int k = b + 1;  // the plane of a block below nz
   const bool mid = b >= nz, kface = k == 1 || k == nz;
   const long m0 = (long)(b - nz) * BC_NT;
   long n;
   if (!mid) {
-    bc_conditions<BC>(k);
+    bc_conditions<BC>(S, k);
     // a k face: the rows and columns that the conditions write or read (rows
     // 1-3 and ny, columns 1-2 and nx-2..nx); the last blocks do the rest
     n = kface ? 4 * nx + 5 * (ny - 4) : 2 * ny + 2 * (nx - 2);
@@ -1666,7 +1668,7 @@ __global__ __launch_bounds__(BC_NT) void k_bc(DevState S, int krk) {
       j = r < nx - 2 ? 1 : ny;
       i = (r < nx - 2 ? r : r - (nx - 2)) + 2;
     }
-    face_cell<MS>(kernarg_again(), i, j, kk);
+    face_cell<MS>(kernarg_again(S), i, j, kk);
   }
 }
 
@@ -2456,8 +2458,18 @@ int kid(const char* name) {
   return id;
 }
 
+// kernarg_again reads a kernel's first argument: a kernel with a DevState has it
+// there, and only there
+template <class... P>
+constexpr bool state_first(void (*)(P...)) {
+  constexpr int n = (0 + ... + std::is_same<std::decay_t<P>, DevState>::value);
+  if constexpr (n == 0) return true;
+  else return n == 1 && std::is_same<std::tuple_element_t<0, std::tuple<P...>>, DevState>::value;
+}
+
 template <typename K, typename... A>
 void launch_s(hipStream_t st, const char* name, K kern, dim3 g, dim3 b, A... args) {
+  static_assert(state_first(K(nullptr)), "a kernel's DevState is its first argument");
   if (G.timing) {
     hipEvent_t a = get_event(), e = get_event();
     hipEventRecord(a, st);

@@ -562,9 +562,9 @@ __device__ __forceinline__ void species_visc_prep_at(const DevState& S, long c, 
   // central eta and zeta forms
   const bool ix = wave_all(central_cell(i, S.nx, R));
   const bool iyz = wave_all(central_cell(j, S.ny, R) && central_cell(k, S.nz, R));
-  if (ix && iyz) species_visc_prep_cell<CD, true, true, true>(kernarg_again(), c, q, i, j, k, m0, m1, step, out);
-  else if (iyz) species_visc_prep_cell<CD, false, true, true>(kernarg_again(), c, q, i, j, k, m0, m1, step, out);
-  else species_visc_prep_cell<CD, false, false, false>(kernarg_again(), c, q, i, j, k, m0, m1, step, out);
+  if (ix && iyz) species_visc_prep_cell<CD, true, true, true>(kernarg_again(S), c, q, i, j, k, m0, m1, step, out);
+  else if (iyz) species_visc_prep_cell<CD, false, true, true>(kernarg_again(S), c, q, i, j, k, m0, m1, step, out);
+  else species_visc_prep_cell<CD, false, false, false>(kernarg_again(S), c, q, i, j, k, m0, m1, step, out);
 }
 
 // Species m0 .. m1-1, one thread per cell.  Qp starts from zero at the first
@@ -669,9 +669,9 @@ __global__ __launch_bounds__(256) void k_species_rk(DevState S, int krk, double 
   const long q = hq(S, i, j, k);
   const bool ix = wave_all(central_cell(i, S.nx, R));
   const bool iyz = wave_all(central_cell(j, S.ny, R) && central_cell(k, S.nz, R));
-  if (ix && iyz) species_rk_cell<CD, true, true, true>(kernarg_again(), c, q, i, j, k, krk, dt, visc, save, m0, m1);
-  else if (iyz) species_rk_cell<CD, false, true, true>(kernarg_again(), c, q, i, j, k, krk, dt, visc, save, m0, m1);
-  else species_rk_cell<CD, false, false, false>(kernarg_again(), c, q, i, j, k, krk, dt, visc, save, m0, m1);
+  if (ix && iyz) species_rk_cell<CD, true, true, true>(kernarg_again(S), c, q, i, j, k, krk, dt, visc, save, m0, m1);
+  else if (iyz) species_rk_cell<CD, false, true, true>(kernarg_again(S), c, q, i, j, k, krk, dt, visc, save, m0, m1);
+  else species_rk_cell<CD, false, false, false>(kernarg_again(S), c, q, i, j, k, krk, dt, visc, save, m0, m1);
 }
 
 // The two kernels above for large grids, all species: a workgroup takes 32 x
