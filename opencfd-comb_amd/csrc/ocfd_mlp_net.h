@@ -16,7 +16,8 @@
 //              arrays and the flat layout.
 // 12-256x5-9, batch 8192: 464 us a call as GEMMs, 61 so (k_net 41, k_net_dw
 // 16, k_net_sum 6 under the profiler).  A sample's values are
-// those of the GEMM path bit for bit (same K order); sums over samples
+// those of the GEMM path bit for bit (same K order); sums over samples, and the
+// loss over the outputs too,
 // differ in order.
 #pragma once
 
