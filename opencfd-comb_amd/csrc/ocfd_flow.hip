@@ -1099,7 +1099,8 @@ __global__ __launch_bounds__(256) void k_transport(DevState S) {
 // ===========================================================================
 // RK_DU3: the inviscid right-hand side comes as the sweeps' three parts
 // (S.du, S.duy, S.duz), added here in their order.  So no sweep waits for
-// another's result or reads it back; each kernel moves the same bytes.
+// another's result or reads it back (40 B a cell less in each of the second and
+// third), and the update reads 15 values a cell instead of 5 (80 B more).
 // RK_SAVE0 (krk = 1): the stage starts from fn = f, kept here from the f that
 // the update reads, instead of by a copy kernel ahead of the step.
 enum { RK_MASS = 1, RK_VISC = 2, RK_WRITE_DU = 4, RK_UPDATE_F = 8, RK_PRIMS = 16, RK_DI_FROM_D = 32, RK_MS = 64,
@@ -2772,10 +2773,20 @@ void enq_stage(int krk, double dt1) {
 // RK3 step, all kernels with 1 / 2 / 3 shares, jets: 48x36x36 (243 blocks of
 // cells, 324 to 432 of sweep tiles) 670 / 594 / 577, 64x48x40 (480) 745 / 815 /
 // 821, 80x56x48 (840) 1085 / 1178 / 1223, 160x112x64 (4480) 4365 / 5094 / 5150.
-// The sweeps alone keep two shares up to 1344 blocks (48x36x36 jet case, 432
-// blocks in y and z: 11.0 ms, 11.3 with one).
+// The sweeps, whose tiles share less of the work, keep three shares to 512
+// tiles of a direction and two to 1344.  us per step (as launches / as a graph)
+// with 1, 2, 3 shares in all three directions, jets with tiles in x, y, z:
+//   40x32x32    256  320  320   649 559  529 / 615 524  505
+//   48x36x36    324  432  432   707 605  587 / 674 571  563
+//   56x36x32    288  448  504   723 621  605 / 698 585  582
+//   56x40x40    400  560  560   786 700  717 / 756 670  675
+//   64x48x40    960  640  768   844 756  780 / 750 705  728
+//   72x48x48   1152  864  864   968 909  913 / 853 861  870
+//   80x56x48   1344 1440 1120  1086 1075 1092 / 1032 1043 1063
+//   96x64x56   1792 2016 2304  1606 1574 1590 / 1534 1536 1581
+//   112x72x64  2304 2688 3024  2206 2139 2159 / 2105 2109 2165
 int species_groups(long blocks, int nm) { return blocks >= 400 ? 1 : std::min(nm, 3); }
-int sweep_groups(long blocks, int nm) { return blocks >= 1344 ? 1 : std::min(nm, blocks >= 400 ? 2 : 3); }
+int sweep_groups(long blocks, int nm) { return blocks >= 1344 ? 1 : std::min(nm, blocks > 512 ? 2 : 3); }
 
 template <int DIR>
 void launch_species_sweep(hipStream_t st, int m0, int m1) {

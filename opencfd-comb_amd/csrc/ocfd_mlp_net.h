@@ -15,10 +15,9 @@
 //   k_net_sum  adds the splits and shares in a fixed order into the gradient
 //              arrays and the flat layout.
 // 12-256x5-9, batch 8192: 464 us a call as GEMMs, 61 so (k_net 41, k_net_dw
-// 16, k_net_sum 6 under the profiler).  A sample's values are
-// those of the GEMM path bit for bit (same K order); sums over samples, and the
-// loss over the outputs too,
-// differ in order.
+// 16, k_net_sum 6 under the profiler).  A sample's values are those of the GEMM
+// path bit for bit (same K order); sums over samples, and the loss's over the
+// outputs, differ in order.
 #pragma once
 
 constexpr int NET_R = 32, NET_NW = 8, NET_W = 256, NET_LD = NET_W + 8, NET_S = 8;
