@@ -184,17 +184,19 @@ __device__ __forceinline__ void coop_cell(Mech m, CoopLds& L, const double2* tab
 //     longest; without one, consecutive cells (their loads coalesce).
 //   - Refill: a lane whose cell is done takes the next one; the wavefront
 //     asks the queue once for all its idle lanes.
-//   - Tail: once the queue is empty and at most COOP_TAIL lanes of the
-//     wavefront still run, their cells go on one after the other with the
-//     whole wavefront each (coop_attempt: 7 us an attempt against 14 us for
-//     any number of lanes, so two cells break even).
+//   - Tail: once the queue is empty and one lane (COOP_TAIL) of the wavefront
+//     still runs, its cell goes on with the whole wavefront (coop_attempt: 7 us
+//     an attempt against 10 us for any number of lanes, so two cells gain only
+//     where one of them ends early; with a tail of 1 / 2 / 3 cells, ms over three
+//     seeds: 50,021 cells 1.47-1.61 / 1.51-1.83 / 1.62-1.90, 2,097,152 cells
+//     3.49-3.60 / 3.70-3.83 / 3.81-3.96).
 //   - budget > 0: a cell still running after `budget` attempts is handed to
 //     k_chem_coop with its full controller state.  A list of at most
 //     direct_max cells (the surrogate's rejects: few, and mostly stiff) hands
 //     every cell over after its first attempt.
 // A cell ends after at most 2 max_sub attempts, and a lane leaves once the
 // queue is empty and its cell is done, so every wave reaches the exit.
-constexpr int COOP_TAIL = 2;
+constexpr int COOP_TAIL = 1;
 template <class ST>
 __global__ __launch_bounds__(CH_BLOCK, 2) void k_chem_queue(long n, double* rho, double* Ecell, const double* dtcell,
                                                      ChemCtl ctl, int* nsub_out, unsigned long long* queue,

@@ -7,9 +7,10 @@
 // What bounds an attempt is its own instruction stream: a stiff cell's
 // attempts follow one another (up to about 190 on a jet-flame batch), and one
 // wave per SIMD has nothing else to issue.  So the mechanism is laid out for
-// few instructions (on MI355X, 9 species / 19 reactions: about 4,900 issued
-// per attempt, 14 us alone on a SIMD and 16 us for two waves; with the
-// reference's expressions as they stand about 40,000 and 82 us):
+// few instructions (on MI355X, 9 species / 19 reactions: ChemH2 about 4,100
+// issued per attempt, 10 us alone on a SIMD and 15 us for two waves, ChemAny
+// 9,100, 29 and 38 us; with the reference's expressions as they stand about
+// 40,000 and 82 us):
 //   - one exponential per Arrhenius set (chem_arr) instead of pow and exp;
 //   - every constant division, the molar-mass ratios and the NASA/R products
 //     folded into the bank on the host;
