@@ -3338,6 +3338,7 @@ int32_t ocfd_set_species(int32_t n_tct, const double* tct, double tct_max, const
       h.ev[j][0][k] = on ? (h.coef[k][j][0] - 1.0) * h.Ri[k] : 0.0;
       for (int a = 1; a < 5; a++) h.ev[j][a][k] = on ? h.coef[k][j][a] * h.Ri[k] : 0.0;
       h.ev[j][5][k] = on ? h.ect[k][j] * h.Ri[k] : 0.0;
+      h.cpa[j][k] = on ? h.coef[k][j][0] * h.Ri[k] : 0.0;
     }
   for (int k = 0; k < ns; k++) h.rcv[k] = 2.5 * h.Ri[k];
   chem_exp_table(h.exp2t);

@@ -24,8 +24,8 @@ struct FlowGas {
   double Mi[OCFD_NS_MAX], rMi[OCFD_NS_MAX], Ri[OCFD_NS_MAX];  // rMi = 1 / Mi
   double coef[OCFD_NS_MAX][GAS_NT_MAX][7], ect[OCFD_NS_MAX][GAS_NT_MAX];
   // (A-1) R, B R, C R, D R, E R, Ect R of each range, and 2.5 R: the products
-  // that the mixture's sums of energy start with
-  double ev[GAS_NT_MAX][6][OCFD_NS_MAX], rcv[OCFD_NS_MAX];
+  // that the mixture's sums of energy start with; cpa = A R, of Cp
+  double ev[GAS_NT_MAX][6][OCFD_NS_MAX], rcv[OCFD_NS_MAX], cpa[GAS_NT_MAX][OCFD_NS_MAX];
   double exp2t[CH_EXPN][2];  // chem_exp's table
   double mu_an[OCFD_NS_MAX][4], k_an[OCFD_NS_MAX][4], D_an[OCFD_NS_MAX][OCFD_NS_MAX][4];
   // Wilke factors that depend only on the molar masses, evaluated on the
@@ -79,26 +79,28 @@ __device__ __forceinline__ void each_species(F f) {
   }
 }
 
-// sum over the species of the energy polynomial's coefficients 0 .. N-1 in
-// range j (a uniform index)
-template <int N>
+// sum over the species of the energy polynomial's coefficients in range j (a
+// uniform index); CP: of Cp's, whose first is A R and which has no sixth
+template <bool CP>
 __device__ __forceinline__ void gas_sums(Gas g, const double* di, int j, double* s) {
+  constexpr int N = CP ? 5 : 6;
 #pragma unroll
   for (int a = 0; a < N; a++) s[a] = 0.0;
   each_species([&](int k) {
+    s[0] = s[0] + (CP ? g->cpa[j][k] : g->ev[j][0][k]) * di[k];
 #pragma unroll
-    for (int a = 0; a < N; a++) s[a] = s[a] + g->ev[j][a][k] * di[k];
+    for (int a = 1; a < N; a++) s[a] = s[a] + g->ev[j][a][k] * di[k];
   });
 }
 
 // ... in range jc of each lane: the lanes of one range at a time, so that the
 // coefficients stay scalar loads
-template <int N>
+template <bool CP>
 __device__ __forceinline__ void gas_sums_lane(Gas g, const double* di, int jc, double* s) {
 #pragma unroll
-  for (int a = 0; a < N; a++) s[a] = 0.0;
+  for (int a = 0; a < (CP ? 5 : 6); a++) s[a] = 0.0;
   for (int j = 0; j < g->n_tct; j++)
-    if (jc == j) gas_sums<N>(g, di, j, s);
+    if (jc == j) gas_sums<CP>(g, di, j, s);
 }
 
 // comput_E_pgas (CHEM_thermdyn.f90:114-122) / comput_E_rgas (:203-231)
@@ -110,7 +112,7 @@ __device__ __forceinline__ double gas_E(const double* di, double T) {
     return E;
   }
   double s[6];
-  gas_sums_lane<6>(g, di, gas_range(g, T), s);
+  gas_sums_lane<false>(g, di, gas_range(g, T), s);
   const double A1 = s[0], B1 = s[1], C1 = s[2], D1 = s[3], E1 = s[4], Ect = s[5];
   if (T <= g->tct_max) return A1 * T + B1 * (T * T) / 2.0 + quot(C1 * gp3(T), 3.0, 1.0 / 3.0) + D1 * gp4(T) / 4.0 + quot(E1 * gp5(T), 5.0, 0.2) + Ect;
   const double tm = g->tct_max;
@@ -132,7 +134,7 @@ __device__ __forceinline__ double gas_T(const double* di, double E) {
   for (int j = 0; j < GAS_NT_MAX; j++) {
 #pragma unroll
     for (int a = 0; a < 6; a++) s[j][a] = 0.0;
-    if (j < g->n_tct) gas_sums<6>(g, di, j, s[j]);
+    if (j < g->n_tct) gas_sums<false>(g, di, j, s[j]);
   }
   double T1 = E / s[0][0], T2 = T1;
   for (int ks = 0; ks <= 30; ks++) {
@@ -184,7 +186,7 @@ __device__ __forceinline__ double gas_Cp(double d, const double* di, double T) {
     return Cp / d;
   }
   double s[5];
-  gas_sums_lane<5>(g, di, gas_range(g, T), s);
+  gas_sums_lane<true>(g, di, gas_range(g, T), s);
   const double t = T <= g->tct_max ? T : g->tct_max;
   return (s[0] + s[1] * t + s[2] * (t * t) + s[3] * gp3(t) + s[4] * gp4(t)) / d;
 }
