@@ -249,7 +249,7 @@ __device__ __forceinline__ double chem_arr_s(double a, double b, double e, const
     const double u = s - ph;
     lo = ((ph - (s - u)) - (eh + u)) + (pl - el);
   }
-  const double k = a * chem_exp(t.tab, s);
+  const double k = chem_exp_times(t.tab, a, s);
   return fm(k, lo, k);
 }
 // Whether ln T, 1/T and the exponent are ordinary numbers.  They are not for a
@@ -335,7 +335,7 @@ __device__ __forceinline__ void chem_reaction(RX R, int rereac, const ChemTp& t,
     double dg = 0.0;
 #pragma unroll
     for (int i = 0; i < CH_NS; i++) dg = fm(g(i), R->nu[i], dg);
-    wr = wf * chem_exp(t.tab, dg);
+    wr = chem_exp_times(t.tab, wf, dg);  // dg passes 709 for a dissociation at 73 K, wf is as small
     const int sgm = R->sgm;
     if (sgm > 0) wr = wr * ipow(t.rs, sgm);
     else if (sgm < 0) wr = wr * ipow(t.irs, -sgm);
@@ -410,7 +410,7 @@ __device__ __forceinline__ void chem_reaction_s(const CH_CONST ChemRx* R, const 
     constexpr int i = decltype(I)::value, nu = ST::vr[K][i] - ST::vf[K][i];
     if constexpr (nu != 0) dg = fm(g(i), (double)nu, dg);
   });
-  double wr = wf * chem_exp(t.tab, dg);
+  double wr = chem_exp_times(t.tab, wf, dg);
   constexpr int sgm = ST::sgm(K);
   if constexpr (sgm > 0) wr = wr * ipow(t.rs, sgm);
   else if constexpr (sgm < 0) wr = wr * ipow(t.irs, -sgm);

@@ -14,7 +14,9 @@
 // range of a double the result is 0 or infinite up to |x| = 2e7, where k still
 // is a 32-bit number; an infinite x gives NaN, so callers keep x finite.
 constexpr int CH_EXPN = 64;
-__device__ __forceinline__ double chem_exp(const double2* tab, double x) {
+// w exp(x), scaled last: finite where the product is, though exp(x) by itself
+// may overflow or w be subnormal; otherwise the same bits as w * exp(x)
+__device__ __forceinline__ double chem_exp_times(const double2* tab, double w, double x) {
   const double n = __builtin_rint(x * 92.332482616893656877);  // 64 / ln 2
   // ln2 / 64 as a 32-bit head (its products with n are exact) and a tail
   double f = __builtin_fma(-n, 0x1.62e42fefp-7, x);
@@ -25,8 +27,9 @@ __device__ __forceinline__ double chem_exp(const double2* tab, double x) {
   p = __builtin_fma(f, p, 1.0 / 6.0);
   p = __builtin_fma(f, p, 0.5);
   p = __builtin_fma(f * f, p, f);
-  return __builtin_amdgcn_ldexp(t.x + __builtin_fma(t.x, p, t.y), k >> 6);
+  return __builtin_amdgcn_ldexp(w * (t.x + __builtin_fma(t.x, p, t.y)), k >> 6);
 }
+__device__ __forceinline__ double chem_exp(const double2* tab, double x) { return chem_exp_times(tab, 1.0, x); }
 
 // 2^(j/64) and its rounding
 inline void chem_exp_table(double (*t)[2]) {
