@@ -173,7 +173,7 @@ __global__ __launch_bounds__(64 * NET_NW) void k_net(NetArgs P) {
       }
     }
   }
-  float e2 = 0.f;
+  double e2 = 0.0;  // a lane adds up to 16 squares of one column: as floats they may overflow together
   {
     const NetLayer& y = P.l[P.L - 1];
     const int nj = net_product(H[cur], y.Wf, y.dinp, y.doutp, w, lane, acc);
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(64 * NET_NW) void k_net(NetArgs P) {
           g[i][r] = 0.f;
           if (row < P.B && c < y.dout) {
             const float e = ((j ? acc[1][i][r] : acc[0][i][r]) + bias) - P.y[row * y.dout + c];
-            e2 += e * e;
+            e2 += (double)e * (double)e;
             g[i][r] = 2.0f * e / cnt;
           }
         }
@@ -200,9 +200,8 @@ __global__ __launch_bounds__(64 * NET_NW) void k_net(NetArgs P) {
     }
     cur ^= 1;
   }
-  double d2 = e2;
-  for (int o = 32; o > 0; o >>= 1) d2 += __shfl_xor(d2, o, 64);
-  if (lane == 0) sl[w] = d2;
+  for (int o = 32; o > 0; o >>= 1) e2 += __shfl_xor(e2, o, 64);
+  if (lane == 0) sl[w] = e2;
   __syncthreads();
   if (t == 0) {
     double s = 0.0;
